@@ -464,7 +464,7 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
 // ---------------------------------------------------------------------------
 __global__ void k_adj_points(Geo g, ShotPtrs sh, StatePtrs a, const float *resid, double *gm6,
                              int n, int n_m) {
-    const int s = blockIdx.x;
+    const int s = g.s0 + blockIdx.x;
     const int nts = sh.nt[s];
     if (threadIdx.x == 0 && n_m >= 0 && n_m < nts) {
         const int *sp = sh.src + 3 * s;

@@ -195,15 +195,7 @@ extern "C" int efm_forward(const EfmDims *d, const EfmMedium *m, const EfmShots 
         return fail(EFM_E_ARG, "efm_forward: CPML too wide for the border save");
     const Geo g = make_geo(*d);
     const ShotPtrs shp = make_shots(*sh);
-    const StatePtrs s = make_state(*st);
-    hipStream_t hs = (hipStream_t)stream;
-    for (int it = it0; it < it0 + nsteps; ++it) {
-        if ((rc = launch_stress_src(g, *m, shp, s, s, it, 1, hs))) return rc;
-        if ((rc = launch_velocity(g, *m, shp, s, s, it, hs, gathers))) return rc;
-        if (gathers && !shp.recmask && (rc = launch_record(g, shp, s, gathers, it, hs))) return rc;
-        if (borders && (rc = launch_border(g, shp, s, borders, W, it, 1, it, hs))) return rc;
-    }
-    return EFM_OK;
+    return run_forward(g, *m, shp, &st, true, gathers, borders, W, it0, nsteps, (hipStream_t)stream);
 }
 
 namespace efm {
@@ -226,7 +218,6 @@ extern "C" int efm_forward_graph(const EfmDims *d, const EfmMedium *m, const Efm
     hipStream_t hs = (hipStream_t)stream;
     if (!hs) return fail(EFM_E_ARG, "efm_forward_graph: graph capture needs a non-default stream");
     const ShotPtrs shp = make_shots(*sh);
-    const StatePtrs s = make_state(*st);
     const int nchunks = nsteps / chunk;
     if (nchunks > 0) {
         hipLaunchKernelGGL(k_counter_set, dim3(1), dim3(64), 0, hs, counter, it0);
@@ -235,12 +226,7 @@ extern "C" int efm_forward_graph(const EfmDims *d, const EfmMedium *m, const Efm
         g.itp = counter;
         if (hipStreamBeginCapture(hs, hipStreamCaptureModeThreadLocal) != hipSuccess)
             return fail(EFM_E_HIP, "efm_forward_graph: hipStreamBeginCapture failed");
-        int crc = EFM_OK;
-        for (int k = 0; k < chunk && crc == EFM_OK; ++k) {
-            if ((crc = launch_stress_src(g, *m, shp, s, s, k, 1, hs))) break;
-            if ((crc = launch_velocity(g, *m, shp, s, s, k, hs, gathers))) break;
-            if (gathers && !shp.recmask) crc = launch_record(g, shp, s, gathers, k, hs);
-        }
+        int crc = run_forward(g, *m, shp, &st, true, gathers, nullptr, 0, 0, chunk, hs);
         if (crc == EFM_OK) {
             hipLaunchKernelGGL(k_counter_add, dim3(1), dim3(64), 0, hs, counter, chunk);
             crc = check_launch("counter add");
@@ -261,13 +247,8 @@ extern "C" int efm_forward_graph(const EfmDims *d, const EfmMedium *m, const Efm
         (void)hipGraphDestroy(graph);
         if (el != hipSuccess || es != hipSuccess) return fail(EFM_E_HIP, "efm_forward_graph: graph launch failed");
     }
-    const Geo g = make_geo(*d);
-    for (int it = it0 + nchunks * chunk; it < it0 + nsteps; ++it) {
-        if ((rc = launch_stress_src(g, *m, shp, s, s, it, 1, hs))) return rc;
-        if ((rc = launch_velocity(g, *m, shp, s, s, it, hs, gathers))) return rc;
-        if (gathers && !shp.recmask && (rc = launch_record(g, shp, s, gathers, it, hs))) return rc;
-    }
-    return EFM_OK;
+    return run_forward(make_geo(*d), *m, shp, &st, true, gathers, nullptr, 0, it0 + nchunks * chunk,
+                       nsteps - nchunks * chunk, hs);
 }
 
 extern "C" int efm_forward_states(const EfmDims *d, const EfmMedium *m, const EfmShots *sh,
@@ -280,15 +261,6 @@ extern "C" int efm_forward_states(const EfmDims *d, const EfmMedium *m, const Ef
         return fail(EFM_E_ARG, "efm_forward_states: step range outside [0, ntmax)");
     for (int k = 0; k <= nsteps; ++k)
         if ((rc = validate_state(d, states[k]))) return rc;
-    const Geo g = make_geo(*d);
-    const ShotPtrs shp = make_shots(*sh);
-    hipStream_t hs = (hipStream_t)stream;
-    for (int k = 0; k < nsteps; ++k) {
-        const StatePtrs in = make_state(*states[k]), out = make_state(*states[k + 1]);
-        if ((rc = launch_stress_src(g, *m, shp, in, out, it0 + k, 1, hs))) return rc;
-        if ((rc = launch_velocity(g, *m, shp, in, out, it0 + k, hs, gathers))) return rc;
-        if (gathers && !shp.recmask && (rc = launch_record(g, shp, out, gathers, it0 + k, hs)))
-            return rc;
-    }
-    return EFM_OK;
+    return run_forward(make_geo(*d), *m, make_shots(*sh), states, false, gathers, nullptr, 0, it0, nsteps,
+                       (hipStream_t)stream);
 }

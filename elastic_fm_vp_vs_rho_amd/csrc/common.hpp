@@ -15,6 +15,7 @@ constexpr int H = 2;  // interior guard: 2 <= x,y,z < n-2 (reference M:54, 77, 1
 // Everything a sweep kernel needs, passed by value (kernel-argument memory).
 struct Geo {
     int nx, ny, nz, S;
+    int s0;                            // first shot of this launch (it covers shots s0 .. s0+S-1)
     int wxl, wxh, wyl, wyh, wzl, wzh;  // CPML widths per face
     int Lx, Ly, Lz;                    // slab extents wxl+wxh, ...
     int ntmax, nrec;
@@ -46,7 +47,7 @@ struct ShotPtrs {
 
 inline Geo make_geo(const EfmDims &d) {
     Geo g;
-    g.nx = d.nx; g.ny = d.ny; g.nz = d.nz; g.S = d.nshot;
+    g.nx = d.nx; g.ny = d.ny; g.nz = d.nz; g.S = d.nshot; g.s0 = 0;
     g.wxl = d.wx_lo; g.wxh = d.wx_hi; g.wyl = d.wy_lo; g.wyh = d.wy_hi;
     g.wzl = d.wz_lo; g.wzh = d.wz_hi;
     g.Lx = d.wx_lo + d.wx_hi; g.Ly = d.wy_lo + d.wy_hi; g.Lz = d.wz_lo + d.wz_hi;
@@ -219,9 +220,10 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
         const int run = (per_shot + 7) / 8;
         const int w = blockIdx.x;
         const int j = w / 8;
-        s = j / run;
-        const int gi = (w % 8) * run + (j - s * run);
-        if (s >= g.S || gi >= per_shot) return false;
+        const int sl = j / run;
+        const int gi = (w % 8) * run + (j - sl * run);
+        if (sl >= g.S || gi >= per_shot) return false;
+        s = g.s0 + sl;
         const int qb = gi % nqb;
         yb = gi / nqb;
         const int q = qb * (BX * BZ) + threadIdx.y * BX + threadIdx.x;
@@ -237,8 +239,9 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
     if (MAP == 0) {
         x = blockIdx.x * BX + threadIdx.x;
         z = blockIdx.y * BZ + threadIdx.y;
-        s = blockIdx.z / nyc;
-        yb = blockIdx.z - s * nyc;
+        const int sl = blockIdx.z / nyc;
+        s = g.s0 + sl;
+        yb = blockIdx.z - sl * nyc;
         return true;
     }
     const int nbx = (g.nx + BX - 1) / BX, nbz = (g.nz + BZ - 1) / BZ;
@@ -247,9 +250,10 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
     const int run = (per_shot + K - 1) / K;
     const int w = blockIdx.x;
     const int j = w / K;
-    s = j / run;
-    const int gi = (w % K) * run + (j - s * run);
-    if (s >= g.S || gi >= per_shot) return false;
+    const int sl = j / run;
+    const int gi = (w % K) * run + (j - sl * run);
+    if (sl >= g.S || gi >= per_shot) return false;
+    s = g.s0 + sl;
     const int xb = gi % nbx;
     const int r = gi / nbx;
     const int zb = r % nbz;
@@ -271,6 +275,44 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
 Tile get_tile(int kernel);  // 0 stress, 1 velocity, 2 adjoint-velocity, 3 adjoint-stress
 int set_tile(int kernel, Tile t);
 
+// ---- shot groups ---------------------------------------------------------------
+// The forward loop takes the shots of a batch through all its steps a group at a
+// time, each group as many shots as fit the 256 MB Infinity Cache with the medium,
+// so that a group's fields come from HBM once per loop and not once per step.
+// Measured on the two sweeps, ns per thousand interior cell-steps by shots per
+// launch: 96^3 25.6 at 4 shots (190 MB), 25.8 at 5 (237 MB), 32.1 at 6 (281 MB), 35.0
+// at 32; 64^3 29.0 at 16 (248 MB), 42.0 at 24 (371 MB); 128^3 22.7 at 2 (223 MB),
+// 34.2 at 3.  32 shots of 96^3 went from 872 to 682 us per step.  Where even one shot
+// exceeds the cache all shots stay in one launch (fewer, longer launches).  The
+// adjoint sweeps gain nothing from groups (96^3: 71 ns with 8 shots in a launch,
+// 74-83 in groups of 2 or 1), so they take the whole batch.
+constexpr long long kCacheBytes = 240LL * 1000 * 1000;
+
+// Bytes of one shot's nine fields and of its ψ slabs.
+inline long long field_bytes(const Geo &g) { return 36 * g.N; }
+inline long long psi_bytes(const Geo &g) { return 24LL * ((long long)g.pxc + g.pyc + g.pzc); }
+
+// Shots per group for a loop that touches `per_shot` bytes of each shot and
+// `shared` bytes of the medium in every step; groups are as equal as possible.
+inline int group_shots(const Geo &g, long long per_shot, long long shared) {
+    const long long fit = (kCacheBytes - shared) / (per_shot > 0 ? per_shot : 1);
+    if (fit < 1 || fit >= g.S) return g.S;
+    const int groups = (int)((g.S + fit - 1) / fit);
+    return (g.S + groups - 1) / groups;
+}
+
+// Calls f(geo) for each group (geo.s0, geo.S name its shots); f returns an error code.
+template <typename F>
+int for_shot_groups(const Geo &g, int group, F f) {
+    for (int s = 0; s < g.S; s += group) {
+        Geo gg = g;
+        gg.s0 = g.s0 + s;
+        gg.S = g.S - s < group ? g.S - s : group;
+        if (int rc = f(gg)) return rc;
+    }
+    return EFM_OK;
+}
+
 // ---- launchers (defined in the .hip files) ------------------------------------
 int launch_stress_src(const Geo &g, const EfmMedium &m, const ShotPtrs &sh, const StatePtrs &in,
                       const StatePtrs &out, int it, int src_mode, hipStream_t st);
@@ -283,5 +325,12 @@ int launch_record(const Geo &g, const ShotPtrs &sh, const StatePtrs &s, float *g
 int launch_border(const Geo &g, const ShotPtrs &sh, const StatePtrs &s, float *borders, int W,
                   int slot, int save, int it_gate, hipStream_t st);
 long long border_floats(const Geo &g, int W);
+// Steps it0 .. it0+nsteps-1 of the forward loop.  `states`: nsteps + 1 states, step
+// it0 + k reading state k and writing state k + 1, or (in_place) one state advanced
+// in place.  Receivers are sampled when `gathers` is set, the reference's border
+// layers saved when `borders` is set.
+int run_forward(const Geo &g, const EfmMedium &m, const ShotPtrs &sh, const EfmState *const *states,
+                bool in_place, float *gathers, float *borders, int W, int it0, int nsteps,
+                hipStream_t st);
 
 }  // namespace efm

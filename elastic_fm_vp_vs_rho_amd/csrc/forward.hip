@@ -250,7 +250,7 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_velocity(Geo g, Med m, ShotPtrs 
 __global__ void k_record(Geo g, ShotPtrs sh, StatePtrs st, float *gathers, int it) {
     if (g.itp) it += *g.itp;
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
+    const int s = g.s0 + blockIdx.y;
     if (r >= g.nrec || it >= sh.nt[s]) return;
     const int cell = sh.rec[(long long)s * g.nrec + r];
     if (cell < 0) return;
@@ -287,7 +287,7 @@ __global__ void k_border(Geo g, ShotPtrs sh, StatePtrs st, float *borders, int W
                          int nslot, int save, int it_gate) {
     const BorderLayout L = border_layout(g.nx, g.ny, g.nz);
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
+    const int s = g.s0 + blockIdx.y;
     if (i >= 3 * L.comp) return;
     if (it_gate >= 0 && it_gate >= sh.nt[s]) return;
     const int comp = (int)(i / L.comp);
@@ -368,6 +368,26 @@ int launch_border(const Geo &g, const ShotPtrs &sh, const StatePtrs &s, float *b
     hipLaunchKernelGGL(k_border, grid, dim3(256), 0, st, g, sh, s, borders, W, slot, g.ntmax,
                        save, it_gate);
     return check_launch("border");
+}
+
+int run_forward(const Geo &g0, const EfmMedium &m, const ShotPtrs &sh, const EfmState *const *states,
+                bool in_place, float *gathers, float *borders, int W, int it0, int nsteps,
+                hipStream_t st) {
+    const int group = group_shots(g0, field_bytes(g0) + psi_bytes(g0), 12 * g0.N);
+    return for_shot_groups(g0, group, [&](const Geo &g) {
+        for (int k = 0; k < nsteps; ++k) {
+            const int it = it0 + k;
+            const StatePtrs in = make_state(*states[in_place ? 0 : k]);
+            const StatePtrs out = make_state(*states[in_place ? 0 : k + 1]);
+            if (int rc = launch_stress_src(g, m, sh, in, out, it, 1, st)) return rc;
+            if (int rc = launch_velocity(g, m, sh, in, out, it, st, gathers)) return rc;
+            if (gathers && !sh.recmask)
+                if (int rc = launch_record(g, sh, out, gathers, it, st)) return rc;
+            if (borders)
+                if (int rc = launch_border(g, sh, out, borders, W, it, 1, it, st)) return rc;
+        }
+        return (int)EFM_OK;
+    });
 }
 
 }  // namespace efm

@@ -157,7 +157,6 @@ extern "C" int efm_plan_forward(EfmPlan *p, const EfmState *state, float *gather
     std::lock_guard<std::mutex> lk(p->mu);
     hipStream_t st = (hipStream_t)stream;
     const ShotPtrs shp = make_shots(p->sh);
-    const StatePtrs s = make_state(*state);
     const int K = p->chunk, nchunks = nsteps / K;
     if (nchunks > 0) {
         hipLaunchKernelGGL(k_plan_counter, dim3(1), dim3(64), 0, st, p->counter, it0);
@@ -170,26 +169,15 @@ extern "C" int efm_plan_forward(EfmPlan *p, const EfmState *state, float *gather
             const int rc = replay(p, key, st, [&](hipStream_t cs) {
                 Geo g = make_geo(p->d);
                 g.itp = p->counter;
-                for (int k = 0; k < K; ++k) {
-                    if (int r = launch_stress_src(g, p->m, shp, s, s, k, 1, cs)) return r;
-                    if (int r = launch_velocity(g, p->m, shp, s, s, k, cs, gathers)) return r;
-                    if (gathers && !shp.recmask)
-                        if (int r = launch_record(g, shp, s, gathers, k, cs)) return r;
-                }
+                if (int r = run_forward(g, p->m, shp, &state, true, gathers, nullptr, 0, 0, K, cs)) return r;
                 hipLaunchKernelGGL(k_plan_counter_add, dim3(1), dim3(64), 0, cs, p->counter, K);
                 return check_launch("plan counter add");
             });
             if (rc) return rc;
         }
     }
-    const Geo g = make_geo(p->d);
-    for (int it = it0 + nchunks * K; it < it0 + nsteps; ++it) {
-        if (int rc = launch_stress_src(g, p->m, shp, s, s, it, 1, st)) return rc;
-        if (int rc = launch_velocity(g, p->m, shp, s, s, it, st, gathers)) return rc;
-        if (gathers && !shp.recmask)
-            if (int rc = launch_record(g, shp, s, gathers, it, st)) return rc;
-    }
-    return EFM_OK;
+    return run_forward(make_geo(p->d), p->m, shp, &state, true, gathers, nullptr, 0, it0 + nchunks * K,
+                       nsteps - nchunks * K, st);
 }
 
 extern "C" int efm_plan_forward_states(EfmPlan *p, const EfmState *const *states, float *gathers,
@@ -208,16 +196,8 @@ extern "C" int efm_plan_forward_states(EfmPlan *p, const EfmState *const *states
     key_add(key, nsteps);
     for (int k = 0; k <= nsteps; ++k) key_add(key, *states[k]);
     return replay(p, key, (hipStream_t)stream, [&](hipStream_t cs) {
-        const Geo g = make_geo(p->d);
-        const ShotPtrs shp = make_shots(p->sh);
-        for (int k = 0; k < nsteps; ++k) {
-            const StatePtrs in = make_state(*states[k]), out = make_state(*states[k + 1]);
-            if (int r = launch_stress_src(g, p->m, shp, in, out, it0 + k, 1, cs)) return r;
-            if (int r = launch_velocity(g, p->m, shp, in, out, it0 + k, cs, gathers)) return r;
-            if (gathers && !shp.recmask)
-                if (int r = launch_record(g, shp, out, gathers, it0 + k, cs)) return r;
-        }
-        return EFM_OK;
+        return run_forward(make_geo(p->d), p->m, make_shots(p->sh), states, false, gathers, nullptr, 0, it0,
+                           nsteps, cs);
     });
 }
 

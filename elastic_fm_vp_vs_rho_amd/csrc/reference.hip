@@ -22,7 +22,7 @@ int launch_stress_src(const Geo &g, const EfmMedium &m, const ShotPtrs &sh, cons
                       const StatePtrs &out, int it, int src_mode, hipStream_t st);
 
 __global__ void k_inject_ref(Geo g, ShotPtrs sh, StatePtrs a, const float *res, int it) {
-    const int s = blockIdx.x;
+    const int s = g.s0 + blockIdx.x;
     const int nts = sh.nt[s];
     const int n = nts - it - 1;
     if (n < 0 || n >= nts) return;
@@ -42,8 +42,8 @@ __global__ void k_inject_ref(Geo g, ShotPtrs sh, StatePtrs a, const float *res, 
 // the reference evaluates this with double literals, so it is done in double.
 __global__ void k_image_mt_ref(Geo g, const float *lam, const float *mu, ShotPtrs sh, StatePtrs a,
                                double *gm6, int it) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= g.S) return;
+    const int s = g.s0 + blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= g.s0 + g.S) return;
     const int nts = sh.nt[s];
     if (it >= nts) return;
     const int *sp = sh.src + 3 * s;
@@ -79,7 +79,7 @@ __global__ void k_image_ref(Geo g, const float *lam, const float *mu, StatePtrs 
                             StatePtrs fp, float dt, float dx, float dy, float dz, float *glam,
                             float *gmu, float *grho) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
+    const int s = g.s0 + blockIdx.y;
     if (i >= g.N) return;
     const int row = i / g.nx;
     const int x = i - row * g.nx;
@@ -129,7 +129,7 @@ __global__ void k_image_ref(Geo g, const float *lam, const float *mu, StatePtrs 
 
 __global__ void k_zero_cpml(Geo g, StatePtrs f, int W) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = blockIdx.y;
+    const int s = g.s0 + blockIdx.y;
     if (i >= g.N) return;
     const int row = i / g.nx;
     const int x = i - row * g.nx;
