@@ -141,7 +141,7 @@ int validate_state(const EfmDims *d, const EfmState *s);
 struct Tile {
     int bx, bz, ny;  // threads in x, threads in z, cells per thread along y
     int map;         // block mapping: 0 = linear 3-D grid; 8 = XCD-aware over 8 XCDs;
-                     // 16 = XCD-aware over the compact interior plane (see tile_coords)
+                     // 16 = XCD-aware over the plane's cells in memory order (see tile_coords)
 };
 
 // Compiled tile variants (bx, bz, ny, map).  Whole 64-lane waves along x.
@@ -168,12 +168,19 @@ struct Tile {
 // XCDs the blocks of an XCD-aware mapping are dealt over.
 __host__ __device__ constexpr int map_xcds(int map) { return map == 16 ? 8 : map; }
 
+// Floats of a 128-byte cache line, and the cells a compact sweep walks in a plane:
+// from the line of the first interior cell to the last interior cell.
+constexpr int kLine = 32;
+__host__ __device__ inline int plane_span(const Geo &g) {
+    return (g.nz - 2 * H) * g.nx - 2 * H + kLine - 1;
+}
+
 // Number of tiles (blocks × y-chunks × shots) of a sweep: x-blocks × z-blocks,
-// or, for the compact mapping, blocks of bx·bz consecutive interior (x, z) cells.
+// or, for the compact mapping, blocks of bx·bz consecutive cells of the plane.
 inline long long sweep_tiles(const Geo &g, int bx, int bz, int ny, int map) {
     const long long nyc = (g.ny - 2 * H + ny - 1) / ny;
     if (map == 16) {
-        const long long q = (long long)(g.nx - 2 * H) * (g.nz - 2 * H);
+        const long long q = plane_span(g);
         return (q + bx * bz - 1) / (bx * bz) * nyc * g.S;
     }
     const long long nbx = (g.nx + bx - 1) / bx, nbz = (g.nz + bz - 1) / bz;
@@ -202,20 +209,22 @@ inline dim3 sweep_grid(const Geo &g, const Tile &t) {
 // runs are per shot (XCD k takes the k-th run of shot 0, then of shot 1, ...), so
 // all XCDs work on the same shot at a time and a batch's sweep keeps one shot's
 // working set in the Infinity Cache, as a one-shot sweep does.
-// MAP = 16: the same XCD order over blocks of BX·BZ consecutive cells of the
-// interior (x, z) plane numbered x fastest with rows wrapped, so that every
-// 64-lane wave is full whatever nx is (with nx - 4 not a multiple of 64 the
-// other mappings leave part-empty waves, which cost the HBM-bound sweeps their
-// share of bytes in flight); a wave then reads at most two row segments.
-// Lanes past the last interior cell get x = -1 (the kernels return on it).
+// MAP = 16: the same XCD order over blocks of BX·BZ consecutive cells of the plane's
+// memory, rows wrapped, from the 128-byte line of its first interior cell: waves are
+// full but for the four guard cells of each row whatever nx is (the other mappings
+// leave part-empty waves where nx is not a multiple of 64), and each wave's row of
+// 64 floats is two whole cache lines in every array whose base is line-aligned.
+// Walking the interior cells only (124 of 128 lanes more useful at 128^3, but waves
+// that straddle three lines) was slower: adjoint step 107 against 97 us at 128^3, 226
+// against 204 at 200x200x100; forward step 979 against 906 us for four shots of
+// 256x256x128, 728 against 704 for 32 of 96^3, the same at 128^3.
+// The kernels return on lanes outside the interior.
 // Returns false for the padding blocks past the last tile.
 template <int BX, int BZ, int NYC, int MAP>
 __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s, int &yb) {
     const int nyc = (g.ny - 2 * H + NYC - 1) / NYC;
     if (MAP == 16) {
-        const int nxi = g.nx - 2 * H;
-        const int Q = nxi * (g.nz - 2 * H);
-        const int nqb = (Q + BX * BZ - 1) / (BX * BZ);
+        const int nqb = (plane_span(g) + BX * BZ - 1) / (BX * BZ);
         const int per_shot = nqb * nyc;
         const int run = (per_shot + 7) / 8;
         const int w = blockIdx.x;
@@ -226,14 +235,11 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
         s = g.s0 + sl;
         const int qb = gi % nqb;
         yb = gi / nqb;
-        const int q = qb * (BX * BZ) + threadIdx.y * BX + threadIdx.x;
-        if (q >= Q) {
-            x = z = -1;
-            return true;
-        }
-        const int zi = q / nxi;
-        z = H + zi;
-        x = H + (q - zi * nxi);
+        // position in the plane of the line-aligned cell the plane's walk starts at
+        const int row0 = (H + yb * NYC) * g.sxz32;
+        const int p = ((row0 + H * g.nx + H) & ~(kLine - 1)) - row0 + qb * (BX * BZ) + threadIdx.y * BX + threadIdx.x;
+        z = p / g.nx;
+        x = p - z * g.nx;
         return true;
     }
     if (MAP == 0) {
