@@ -9,10 +9,10 @@
 //
 //   reverse step n     R1 v̄[rec] += r[n]
 //                      R2 u = c·b̄·v̄;  h̄ = u + a(C+u);  C ← b(C+u);  τ̄ += D_τᵀ h̄
-//                         ρ-accumulators  += v̄·(v^{n+1} - v^n)   (= v̄·c·b̄·F)
 //                      R3 M̄ += w[n]·τ̄(src)
 //                      R4 ē = c·Sᵀτ̄;  ḡ = ē + a(C+ē);  C ← b(C+ē);  v̄ += D_vᵀ ḡ
-//                         λ/μ accumulators += τ̄·(∂S/∂λ,μ)e
+//   images             λ/μ sums += τ̄·(∂S/∂λ,μ)e (by R2, with the τ̄ it writes);
+//                      ρ sums += v̄·(v^{n+1} - v^n) (= v̄·c·b̄·F; by R4, with the v̄ it reads)
 //
 // D_ᵀ are applied in gather form (each thread writes only its own cell), which
 // needs h̄/ḡ at the ±1 neighbours; C is read at neighbours while its owner
@@ -27,42 +27,128 @@
 
 namespace efm {
 
-// Loads of the stored forward state carry the streaming (nontemporal) hint:
-// each value is read by one step of the reverse sweep only, and the hint keeps
-// the reused adjoint state, medium and accumulators cached.
+// Streaming (nontemporal) load of a stored forward value: the hint keeps the
+// reused adjoint state, medium and accumulators cached.
 #define LDF(p) __builtin_nontemporal_load(p)
-
-// CPML coefficient of cell i (0 outside the slab, slab coordinate < 0).  The
-// load is unconditional (every interior cell's ±1 neighbour indexes the
-// profile), so it issues with the others instead of behind a branch.
-static __device__ __forceinline__ float coef(const float *p, int i, int slab) {
-    const float v = p[i];
-    return slab >= 0 ? v : 0.f;
-}
 
 struct AdjArgs {
     const float *lam, *mu;
     const float *mbar, *bbar;      // (3, N) each
     StatePtrs fn, fn1;             // forward S^n, S^{n+1}
+    const float *vm1[3];           // forward velocities before step n - 1 (R4's two-step ρ sums)
     StatePtrs a, a2;               // adjoint: a = live (v̄, τ̄, C in), a2 = C out
     float *acc;                    // per shot 8 padded components: λ, μ, μ_xy, μ_xz sums
-                                   // interleaved (one float4 per cell) in components 0-3,
-                                   // the ρ sum in 4, μ_yz in 7 (5 and 6 unused: 8 components
+                                   // interleaved (one float4 per cell) in components 0-3, the
+                                   // ρ sums of the x, y, z faces in 4-6, μ_yz in 7 (8 components
                                    // keep every shot's float4 base 16-byte aligned for any N)
     ShotPtrs sh;
     const float *resid;            // ∂J/∂gathers, used by R4 when the shots carry a receiver mask
     double *gm6;                   // ∂J/∂M, likewise
+    int n0, n1;                    // step range of the call: n0 <= n < n1
 };
 
+// The reverse sweep images two steps at a time, so that the accumulators cross
+// memory every other step: of each pair (n odd, n - 1) R2 of step n - 1 holds τ̄
+// before and after its update and adds the λ/μ products of both steps, and R4 of
+// step n holds v̄ before and after its update and adds the ρ products of both.  A
+// step whose partner is outside the call's range or past the shot's record is
+// imaged alone, by R2 with the new τ̄ and by R4 with the old v̄.
+//   older: the products of step n + 1 (R2) / of step n (R4) from the value read
+//   newer: the products of step n (R2) / of step n - 1 (R4) from the value written
+struct Pairing {
+    bool older, newer;
+};
+__device__ __forceinline__ Pairing image_r2(const AdjArgs &A, int nts, int n) {
+    const int end = min(A.n1, nts);
+    return n & 1 ? Pairing{false, n == A.n0} : Pairing{n + 1 < end, true};
+}
+__device__ __forceinline__ Pairing image_r4(const AdjArgs &A, int nts, int n) {
+    const int end = min(A.n1, nts);
+    // without a receiver mask the residual of step n - 1 joins v̄ in a kernel of its
+    // own after this sweep: every step is imaged alone
+    if (!A.sh.recmask) return Pairing{true, false};
+    return n & 1 ? Pairing{true, n > A.n0} : Pairing{n + 1 >= end, false};
+}
+
+// The five λ/μ sums of a cell, fed by the adjoint stress τ̄ and the forward strain
+// e = Δ + ψ' of a step (from the velocities and the ψ_v before the step).
+struct ImageSums {
+    float lam, mu, xy, xz, yz;
+};
+template <bool STREAM>
+static __device__ __forceinline__ float ldf(const float *p) {
+    return STREAM ? LDF(p) : *p;
+}
+struct StrainLoads {
+    float v0, v1, v2, v0mx, v1my, v2mz, v0pz, v0py, v1px, v1pz, v2px, v2py;
+    float fx0, fx1, fx2, fy0, fy1, fy2, fz0, fz1, fz2;
+};
+struct Slabs {
+    int ix, iy, iz;                // own offsets of component 0 in the three slabs (-1 outside)
+    float ax, bx, ay, by, az, bz;  // own coefficients (0 outside)
+};
+template <bool STREAM>
+static __device__ __forceinline__ StrainLoads strain_loads(const Geo &g, const StatePtrs &f, int s, int t,
+                                                           const Slabs &q) {
+    const long long so = (long long)s * g.N;
+    const float *__restrict__ V0 = f.v[0] + so, *__restrict__ V1 = f.v[1] + so, *__restrict__ V2 = f.v[2] + so;
+    const int nx = g.nx, sxz = g.sxz32;
+    StrainLoads l;
+    l.v0 = ldf<STREAM>(&V0[t]); l.v1 = ldf<STREAM>(&V1[t]); l.v2 = ldf<STREAM>(&V2[t]);
+    l.v0mx = ldf<STREAM>(&V0[t - 1]); l.v1my = ldf<STREAM>(&V1[t - sxz]); l.v2mz = ldf<STREAM>(&V2[t - nx]);
+    l.v0pz = ldf<STREAM>(&V0[t + nx]); l.v0py = ldf<STREAM>(&V0[t + sxz]); l.v1px = ldf<STREAM>(&V1[t + 1]);
+    l.v1pz = ldf<STREAM>(&V1[t + nx]); l.v2px = ldf<STREAM>(&V2[t + 1]); l.v2py = ldf<STREAM>(&V2[t + sxz]);
+    l.fx0 = l.fx1 = l.fx2 = l.fy0 = l.fy1 = l.fy2 = l.fz0 = l.fz1 = l.fz2 = 0.f;
+    if (q.ix >= 0) {
+        const float *F = f.px + px_shot(g, s);
+        l.fx0 = ldf<STREAM>(&F[q.ix]); l.fx1 = ldf<STREAM>(&F[q.ix + g.pxc]); l.fx2 = ldf<STREAM>(&F[q.ix + 2 * g.pxc]);
+    }
+    if (q.iy >= 0) {
+        const float *F = f.py + py_shot(g, s);
+        l.fy0 = ldf<STREAM>(&F[q.iy]); l.fy1 = ldf<STREAM>(&F[q.iy + g.pyc]); l.fy2 = ldf<STREAM>(&F[q.iy + 2 * g.pyc]);
+    }
+    if (q.iz >= 0) {
+        const float *F = f.pz + pz_shot(g, s);
+        l.fz0 = ldf<STREAM>(&F[q.iz]); l.fz1 = ldf<STREAM>(&F[q.iz + g.pzc]); l.fz2 = ldf<STREAM>(&F[q.iz + 2 * g.pzc]);
+    }
+    return l;
+}
+// a += the products of one step.  Every rounding is spelled out: a pair's two steps
+// then give the same bits added in one sweep or in two.
+static __device__ __forceinline__ void image_add(ImageSums &a, const StrainLoads &l, const Slabs &q, float txx,
+                                                 float tyy, float tzz, float txy, float txz, float tyz) {
+#pragma clang fp contract(off)
+    const float d_xx = l.v0 - l.v0mx, d_yy = l.v1 - l.v1my, d_zz = l.v2 - l.v2mz;
+    const float d_xz = l.v0pz - l.v0, d_xy = l.v0py - l.v0, d_yx = l.v1px - l.v1, d_yz = l.v1pz - l.v1;
+    const float d_zx = l.v2px - l.v2, d_zy = l.v2py - l.v2;
+    // e = Δ + (bψ + aΔ); a = b = 0 outside the slabs
+    const float fxx = d_xx + fmaf(q.bx, l.fx0, q.ax * d_xx);
+    const float fyx = d_yx + fmaf(q.bx, l.fx1, q.ax * d_yx);
+    const float fzx = d_zx + fmaf(q.bx, l.fx2, q.ax * d_zx);
+    const float fxy = d_xy + fmaf(q.by, l.fy0, q.ay * d_xy);
+    const float fyy = d_yy + fmaf(q.by, l.fy1, q.ay * d_yy);
+    const float fzy = d_zy + fmaf(q.by, l.fy2, q.ay * d_zy);
+    const float fxz = d_xz + fmaf(q.bz, l.fz0, q.az * d_xz);
+    const float fyz = d_yz + fmaf(q.bz, l.fz1, q.az * d_yz);
+    const float fzz = d_zz + fmaf(q.bz, l.fz2, q.az * d_zz);
+    a.lam = fmaf(txx + tyy + tzz, fxx + fyy + fzz, a.lam);
+    a.mu = fmaf(2.f, fmaf(txx, fxx, fmaf(tyy, fyy, tzz * fzz)), a.mu);
+    a.xy = fmaf(txy, fxy + fyx, a.xy);
+    a.xz = fmaf(txz, fxz + fzx, a.xz);
+    a.yz = fmaf(tyz, fyz + fzy, a.yz);
+}
+
 // ---------------------------------------------------------------------------
-// R2: transpose of the velocity sweep
+// R2: transpose of the velocity sweep, λ/μ imaging
 // ---------------------------------------------------------------------------
-template <int BX, int BZ, int NYC, int MAP>
-__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity(Geo g, AdjArgs A, int n) {
+template <int BX, int BZ, int NYC, int MAP, bool IMAGE, bool STREAM>
+static __device__ __forceinline__ void adj_velocity_cells(const Geo &g, const AdjArgs &A, int n) {
     int x, z, s, yb;
     if (!tile_coords<BX, BZ, NYC, MAP>(g, x, z, s, yb)) return;
     if (x < H || x >= g.nx - H || z < H || z >= g.nz - H) return;
-    if (n >= A.sh.nt[s]) return;
+    const int nts = A.sh.nt[s];
+    if (n >= nts) return;
+    const Pairing im = image_r2(A, nts, n);
     const int y0 = H + yb * NYC;
     const int y1 = min(y0 + NYC, g.ny - H);
     const int nx = g.nx, sxz = g.sxz32;
@@ -70,7 +156,7 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity(Geo g, AdjArgs A, i
     const float c = g.c;
     const ShotPtrs &sh = A.sh;
 
-    // slab coordinates and coefficients of this column and its x/z neighbours
+    // slab coordinates of this column and its x/z neighbours
     const int sx0 = slab_coord(x, g.nx, g.wxl, g.wxh);
     const int sxm = slab_coord(x - 1, g.nx, g.wxl, g.wxh);
     const int sxp = slab_coord(x + 1, g.nx, g.wxl, g.wxh);
@@ -80,10 +166,6 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity(Geo g, AdjArgs A, i
     const float *axs = sh.ax + (long long)s * g.nx, *bxs = sh.bx + (long long)s * g.nx;
     const float *ays = sh.ay + (long long)s * g.ny, *bys = sh.by + (long long)s * g.ny;
     const float *azs = sh.az + (long long)s * g.nz, *bzs = sh.bz + (long long)s * g.nz;
-    const float ax0 = coef(axs, x, sx0), bx0 = coef(bxs, x, sx0);
-    const float axm = coef(axs, x - 1, sxm), axp = coef(axs, x + 1, sxp);
-    const float az0 = coef(azs, z, sz0), bz0 = coef(bzs, z, sz0);
-    const float azm = coef(azs, z - 1, szm), azp = coef(azs, z + 1, szp);
     const int csx = g.pxc, csy = g.pyc, csz = g.pzc;
 
     const float *__restrict__ bbx = A.bbar;
@@ -98,137 +180,151 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity(Geo g, AdjArgs A, i
     float *__restrict__ tb3 = A.a.t[3] + so;
     float *__restrict__ tb4 = A.a.t[4] + so;
     float *__restrict__ tb5 = A.a.t[5] + so;
-    // forward velocities after and before step n: their difference is c·b̄·F, the
-    // velocity update the ρ products need (read at the cell and at p-x, p-y, p-z, so
-    // without the streaming hint)
-    const float *__restrict__ Wx1 = A.fn1.v[0] + so;
-    const float *__restrict__ Wy1 = A.fn1.v[1] + so;
-    const float *__restrict__ Wz1 = A.fn1.v[2] + so;
-    const float *__restrict__ Wx0 = A.fn.v[0] + so;
-    const float *__restrict__ Wy0 = A.fn.v[1] + so;
-    const float *__restrict__ Wz0 = A.fn.v[2] + so;
     const float *__restrict__ Cx = A.a.px + px_shot(g, s);
     const float *__restrict__ Cy = A.a.py + py_shot(g, s);
     const float *__restrict__ Cz = A.a.pz + pz_shot(g, s);
     float *__restrict__ Cxo = A.a2.px + px_shot(g, s);
     float *__restrict__ Cyo = A.a2.py + py_shot(g, s);
     float *__restrict__ Czo = A.a2.pz + pz_shot(g, s);
-    // ρ sums: component 4 of the shot
-    float *__restrict__ accr = A.acc + ((long long)s * 8 + 4) * g.ps;
+    float4 *__restrict__ acc4v = reinterpret_cast<float4 *>(A.acc + (long long)s * 8 * g.ps);
+    float *__restrict__ accyz = A.acc + ((long long)s * 8 + 7) * g.ps;
 
     for (int y = y0; y < y1; ++y) {
         const int t = x + z * nx + y * sxz;
         const int sy0 = slab_coord(y, g.ny, g.wyl, g.wyh);
         const int sym = slab_coord(y - 1, g.ny, g.wyl, g.wyh);
         const int syp = slab_coord(y + 1, g.ny, g.wyl, g.wyh);
-        const float ay0 = coef(ays, y, sy0), by0 = coef(bys, y, sy0);
-        const float aym = coef(ays, y - 1, sym), ayp = coef(ays, y + 1, syp);
 
-        // Every load of the cell that does not depend on the CPML slabs is issued
-        // here, before the first store: the compiler cannot prove that the stores
-        // below miss these arrays, so a load placed after a store would wait for it.
+        // Every load of the cell is issued before the first use or store.  The slab
+        // loads above all: a slab cell used to wait for each neighbour's ψ in turn.
         const float tbo0 = tb0[t], tbo1 = tb1[t], tbo2 = tb2[t];
         const float tbo3 = tb3[t], tbo4 = tb4[t], tbo5 = tb5[t];
-        const float acco = accr[t];
-        const float dwx = Wx1[t] - Wx0[t], dwy = Wy1[t] - Wy0[t], dwz = Wz1[t] - Wz0[t];
-        const float dwx_m = Wx1[t - 1] - Wx0[t - 1];
-        const float dwy_m = Wy1[t - sxz] - Wy0[t - sxz];
-        const float dwz_m = Wz1[t - nx] - Wz0[t - nx];
-        // u = c·b̄·v̄ at p and at the neighbours the transposes need
-        const float vx0 = vbx[t], vy0 = vby[t], vz0 = vbz[t];
-        const float ux = c * bbx[t] * vx0;
-        const float uy = c * bby[t] * vy0;
-        const float uz = c * bbz[t] * vz0;
-        const float ux_mx = c * bbx[t - 1] * vbx[t - 1];        // txx_x at p-x
-        const float uy_my = c * bby[t - sxz] * vby[t - sxz];    // tyy_y at p-y
-        const float uz_mz = c * bbz[t - nx] * vbz[t - nx];      // tzz_z at p-z
-        const float ux_py = c * bbx[t + sxz] * vbx[t + sxz];    // txy_y at p+y
-        const float uy_px = c * bby[t + 1] * vby[t + 1];        // txy_x at p+x
-        const float ux_pz = c * bbx[t + nx] * vbx[t + nx];      // txz_z at p+z
-        const float uz_px = c * bbz[t + 1] * vbz[t + 1];        // txz_x at p+x
-        const float uy_pz = c * bby[t + nx] * vby[t + nx];      // tyz_z at p+z
-        const float uz_py = c * bbz[t + sxz] * vbz[t + sxz];    // tyz_y at p+y
-        // ρ: this cell enters the averaged buoyancy of its own three faces and of the
-        // faces at p-x, p-y, p-z; each face contributes u·Δv (= c·b̄·v̄ times this step's
-        // forward velocity change).  u vanishes off the interior (b̄ = 0 there).
-        const float px = ux * dwx, py = uy * dwy, pz = uz * dwz;
-        const float accn = acco + ((px + ux_mx * dwx_m) + (py + uy_my * dwy_m) + (pz + uz_mz * dwz_m));
-
-        // h̄ = u + a(C + u) with C read from the "in" buffer
-        float hb_xx_m = ux_mx, hb_xx_0 = ux;           // txx_x
-        float hb_yy_m = uy_my, hb_yy_0 = uy;           // tyy_y
-        float hb_zz_m = uz_mz, hb_zz_0 = uz;           // tzz_z
-        float hb_xyy_0 = ux, hb_xyy_p = ux_py;         // txy_y
-        float hb_xyx_0 = uy, hb_xyx_p = uy_px;         // txy_x
-        float hb_xzz_0 = ux, hb_xzz_p = ux_pz;         // txz_z
-        float hb_xzx_0 = uz, hb_xzx_p = uz_px;         // txz_x
-        float hb_yzz_0 = uy, hb_yzz_p = uy_pz;         // tyz_z
-        float hb_yzy_0 = uz, hb_yzy_p = uz_py;         // tyz_y
-        // x-slab components 3 txx_x, 4 txy_x, 5 txz_x
-        if (sxm >= 0) hb_xx_m += axm * (Cx[px_off(g, y, z, sxm) + 3 * csx] + ux_mx);
+        const float wx0 = vbx[t], wy0 = vby[t], wz0 = vbz[t];
+        const float wx_mx = vbx[t - 1], wy_my = vby[t - sxz], wz_mz = vbz[t - nx];
+        const float wx_py = vbx[t + sxz], wy_px = vby[t + 1], wx_pz = vbx[t + nx];
+        const float wz_px = vbz[t + 1], wy_pz = vby[t + nx], wz_py = vbz[t + sxz];
+        const float gx0 = bbx[t], gy0 = bby[t], gz0 = bbz[t];
+        const float gx_mx = bbx[t - 1], gy_my = bby[t - sxz], gz_mz = bbz[t - nx];
+        const float gx_py = bbx[t + sxz], gy_px = bby[t + 1], gx_pz = bbx[t + nx];
+        const float gz_px = bbz[t + 1], gy_pz = bby[t + nx], gz_py = bbz[t + sxz];
+        // x-slab components 3 txx_x, 4 txy_x, 5 txz_x; y: 3 txy_y, 4 tyy_y, 5 tyz_y;
+        // z: 3 txz_z, 4 tyz_z, 5 tzz_z.  a = 0 outside the slab.
+        Slabs q{-1, -1, -1, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float axm = 0.f, axp = 0.f, aym = 0.f, ayp = 0.f, azm = 0.f, azp = 0.f;
+        float cxm = 0.f, cxp1 = 0.f, cxp2 = 0.f, cx0 = 0.f, cx1 = 0.f, cx2 = 0.f;
+        float cym = 0.f, cyp0 = 0.f, cyp2 = 0.f, cy0 = 0.f, cy1 = 0.f, cy2 = 0.f;
+        float czm = 0.f, czp0 = 0.f, czp1 = 0.f, cz0 = 0.f, cz1 = 0.f, cz2 = 0.f;
+        if (sxm >= 0) { axm = axs[x - 1]; cxm = Cx[px_off(g, y, z, sxm) + 3 * csx]; }
         if (sxp >= 0) {
             const int pi = px_off(g, y, z, sxp) + 4 * csx;
-            hb_xyx_p += axp * (Cx[pi] + uy_px);
-            hb_xzx_p += axp * (Cx[pi + csx] + uz_px);
+            axp = axs[x + 1]; cxp1 = Cx[pi]; cxp2 = Cx[pi + csx];
         }
         if (sx0 >= 0) {
-            const int pi = px_off(g, y, z, sx0) + 3 * csx;
-            const float c0 = Cx[pi] + ux, c1 = Cx[pi + csx] + uy, c2 = Cx[pi + 2 * csx] + uz;
-            hb_xx_0 += ax0 * c0; hb_xyx_0 += ax0 * c1; hb_xzx_0 += ax0 * c2;
-            Cxo[pi] = bx0 * c0; Cxo[pi + csx] = bx0 * c1; Cxo[pi + 2 * csx] = bx0 * c2;
+            q.ix = px_off(g, y, z, sx0);
+            q.ax = axs[x]; q.bx = bxs[x];
+            cx0 = Cx[q.ix + 3 * csx]; cx1 = Cx[q.ix + 4 * csx]; cx2 = Cx[q.ix + 5 * csx];
         }
-        // y-slab components 3 txy_y, 4 tyy_y, 5 tyz_y
-        if (sym >= 0) hb_yy_m += aym * (Cy[py_off(g, sym, z, x) + 4 * csy] + uy_my);
+        if (sym >= 0) { aym = ays[y - 1]; cym = Cy[py_off(g, sym, z, x) + 4 * csy]; }
         if (syp >= 0) {
             const int pi = py_off(g, syp, z, x) + 3 * csy;
-            hb_xyy_p += ayp * (Cy[pi] + ux_py);
-            hb_yzy_p += ayp * (Cy[pi + 2 * csy] + uz_py);
+            ayp = ays[y + 1]; cyp0 = Cy[pi]; cyp2 = Cy[pi + 2 * csy];
         }
         if (sy0 >= 0) {
-            const int pi = py_off(g, sy0, z, x) + 3 * csy;
-            const float c0 = Cy[pi] + ux, c1 = Cy[pi + csy] + uy, c2 = Cy[pi + 2 * csy] + uz;
-            hb_xyy_0 += ay0 * c0; hb_yy_0 += ay0 * c1; hb_yzy_0 += ay0 * c2;
-            Cyo[pi] = by0 * c0; Cyo[pi + csy] = by0 * c1; Cyo[pi + 2 * csy] = by0 * c2;
+            q.iy = py_off(g, sy0, z, x);
+            q.ay = ays[y]; q.by = bys[y];
+            cy0 = Cy[q.iy + 3 * csy]; cy1 = Cy[q.iy + 4 * csy]; cy2 = Cy[q.iy + 5 * csy];
         }
-        // z-slab components 3 txz_z, 4 tyz_z, 5 tzz_z
-        if (szm >= 0) hb_zz_m += azm * (Cz[pz_off(g, y, szm, x) + 5 * csz] + uz_mz);
+        if (szm >= 0) { azm = azs[z - 1]; czm = Cz[pz_off(g, y, szm, x) + 5 * csz]; }
         if (szp >= 0) {
             const int pi = pz_off(g, y, szp, x) + 3 * csz;
-            hb_xzz_p += azp * (Cz[pi] + ux_pz);
-            hb_yzz_p += azp * (Cz[pi + csz] + uy_pz);
+            azp = azs[z + 1]; czp0 = Cz[pi]; czp1 = Cz[pi + csz];
         }
         if (sz0 >= 0) {
-            const int pi = pz_off(g, y, sz0, x) + 3 * csz;
-            const float c0 = Cz[pi] + ux, c1 = Cz[pi + csz] + uy, c2 = Cz[pi + 2 * csz] + uz;
-            hb_xzz_0 += az0 * c0; hb_yzz_0 += az0 * c1; hb_zz_0 += az0 * c2;
-            Czo[pi] = bz0 * c0; Czo[pi + csz] = bz0 * c1; Czo[pi + 2 * csz] = bz0 * c2;
+            q.iz = pz_off(g, y, sz0, x);
+            q.az = azs[z]; q.bz = bzs[z];
+            cz0 = Cz[q.iz + 3 * csz]; cz1 = Cz[q.iz + 4 * csz]; cz2 = Cz[q.iz + 5 * csz];
         }
-        // τ̄ += D_τᵀ h̄
-        tb0[t] = tbo0 + (hb_xx_m - hb_xx_0);
-        tb1[t] = tbo1 + (hb_yy_m - hb_yy_0);
-        tb2[t] = tbo2 + (hb_zz_m - hb_zz_0);
-        tb3[t] = tbo3 + ((hb_xyy_0 - hb_xyy_p) + (hb_xyx_0 - hb_xyx_p));
-        tb4[t] = tbo4 + ((hb_xzz_0 - hb_xzz_p) + (hb_xzx_0 - hb_xzx_p));
-        tb5[t] = tbo5 + ((hb_yzz_0 - hb_yzz_p) + (hb_yzy_0 - hb_yzy_p));
 
-        // A face on the last interior plane also feeds the cell beyond it, which no
-        // thread of this sweep owns; that cell has no other face in the interior, so
-        // the face's thread adds it there (one writer per cell).
-        accr[t] = accn;
-        if (x == g.nx - H - 1) accr[t + 1] += px;
-        if (y == g.ny - H - 1) accr[t + sxz] += py;
-        if (z == g.nz - H - 1) accr[t + nx] += pz;
+        // u = c·b̄·v̄ at p and at the neighbours the transposes need (b̄ = 0 off the interior)
+        const float ux = c * gx0 * wx0, uy = c * gy0 * wy0, uz = c * gz0 * wz0;
+        const float ux_mx = c * gx_mx * wx_mx;        // txx_x at p-x
+        const float uy_my = c * gy_my * wy_my;        // tyy_y at p-y
+        const float uz_mz = c * gz_mz * wz_mz;        // tzz_z at p-z
+        const float ux_py = c * gx_py * wx_py;        // txy_y at p+y
+        const float uy_px = c * gy_px * wy_px;        // txy_x at p+x
+        const float ux_pz = c * gx_pz * wx_pz;        // txz_z at p+z
+        const float uz_px = c * gz_px * wz_px;        // txz_x at p+x
+        const float uy_pz = c * gy_pz * wy_pz;        // tyz_z at p+z
+        const float uz_py = c * gz_py * wz_py;        // tyz_y at p+y
+        // h̄ = u + a(C + u) with C read from the "in" buffer
+        cx0 += ux; cx1 += uy; cx2 += uz;
+        cy0 += ux; cy1 += uy; cy2 += uz;
+        cz0 += ux; cz1 += uy; cz2 += uz;
+        const float hb_xx = (ux_mx + axm * (cxm + ux_mx)) - (ux + q.ax * cx0);
+        const float hb_yy = (uy_my + aym * (cym + uy_my)) - (uy + q.ay * cy1);
+        const float hb_zz = (uz_mz + azm * (czm + uz_mz)) - (uz + q.az * cz2);
+        const float hb_xyy = (ux + q.ay * cy0) - (ux_py + ayp * (cyp0 + ux_py));
+        const float hb_xyx = (uy + q.ax * cx1) - (uy_px + axp * (cxp1 + uy_px));
+        const float hb_xzz = (ux + q.az * cz0) - (ux_pz + azp * (czp0 + ux_pz));
+        const float hb_xzx = (uz + q.ax * cx2) - (uz_px + axp * (cxp2 + uz_px));
+        const float hb_yzz = (uy + q.az * cz1) - (uy_pz + azp * (czp1 + uy_pz));
+        const float hb_yzy = (uz + q.ay * cy2) - (uz_py + ayp * (cyp2 + uz_py));
+        // τ̄ += D_τᵀ h̄
+        const float n0 = tbo0 + hb_xx, n1 = tbo1 + hb_yy, n2 = tbo2 + hb_zz;
+        const float n3 = tbo3 + (hb_xyy + hb_xyx);
+        const float n4 = tbo4 + (hb_xzz + hb_xzx);
+        const float n5 = tbo5 + (hb_yzz + hb_yzy);
+        if (IMAGE && im.newer) {
+            const float4 a = acc4v[t];
+            ImageSums sum{a.x, a.y, a.z, a.w, accyz[t]};
+            const StrainLoads l = strain_loads<STREAM>(g, A.fn, s, t, q);
+            if (im.older) {
+                const StrainLoads l1 = strain_loads<STREAM>(g, A.fn1, s, t, q);
+                image_add(sum, l1, q, tbo0, tbo1, tbo2, tbo3, tbo4, tbo5);
+            }
+            image_add(sum, l, q, n0, n1, n2, n3, n4, n5);
+            acc4v[t] = make_float4(sum.lam, sum.mu, sum.xy, sum.xz);
+            accyz[t] = sum.yz;
+        }
+        tb0[t] = n0; tb1[t] = n1; tb2[t] = n2;
+        tb3[t] = n3; tb4[t] = n4; tb5[t] = n5;
+        if (sx0 >= 0) {
+            const int pi = q.ix + 3 * csx;
+            Cxo[pi] = q.bx * cx0; Cxo[pi + csx] = q.bx * cx1; Cxo[pi + 2 * csx] = q.bx * cx2;
+        }
+        if (sy0 >= 0) {
+            const int pi = q.iy + 3 * csy;
+            Cyo[pi] = q.by * cy0; Cyo[pi + csy] = q.by * cy1; Cyo[pi + 2 * csy] = q.by * cy2;
+        }
+        if (sz0 >= 0) {
+            const int pi = q.iz + 3 * csz;
+            Czo[pi] = q.bz * cz0; Czo[pi + csz] = q.bz * cz1; Czo[pi + 2 * csz] = q.bz * cz2;
+        }
     }
 }
 
-// ---------------------------------------------------------------------------
-// R4: transpose of the stress sweep
-// ---------------------------------------------------------------------------
-// At least 7 waves per SIMD: the compiler then fits the sweep in 71 VGPRs (73 by
-// itself, which allows only 6) by moving some SGPRs to VGPR lanes; the C2 adjoint
-// step gets 2-3 % faster.
+// Three instances.  The steps that no shot images (one of every pair) run without
+// the imaging's registers (78 VGPRs against 98): 28 against 65 us at 128^3, where one
+// instance for both took 53 on average of either.  The imaging instances differ in
+// the streaming hint on the forward state (see launch_adj_velocity).
 template <int BX, int BZ, int NYC, int MAP>
-__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_adj_stress(Geo g, AdjArgs A, int n) {
+__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity(Geo g, AdjArgs A, int n) {
+    adj_velocity_cells<BX, BZ, NYC, MAP, false, false>(g, A, n);
+}
+template <int BX, int BZ, int NYC, int MAP>
+__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity_image(Geo g, AdjArgs A, int n) {
+    adj_velocity_cells<BX, BZ, NYC, MAP, true, false>(g, A, n);
+}
+template <int BX, int BZ, int NYC, int MAP>
+__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_velocity_image_stream(Geo g, AdjArgs A, int n) {
+    adj_velocity_cells<BX, BZ, NYC, MAP, true, true>(g, A, n);
+}
+
+// ---------------------------------------------------------------------------
+// R4: transpose of the stress sweep, ρ imaging
+// ---------------------------------------------------------------------------
+template <int BX, int BZ, int NYC, int MAP>
+__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_stress(Geo g, AdjArgs A, int n) {
     int x, z, s, yb;
     if (!tile_coords<BX, BZ, NYC, MAP>(g, x, z, s, yb)) return;
     if (x < H || x >= g.nx - H || z < H || z >= g.nz - H) return;
@@ -260,6 +356,7 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
             }
         return;
     }
+    const Pairing im = image_r4(A, nts, n);
     const int *sp = sh.src + 3 * s;
     const int tsrc = sp[0] + sp[2] * nx + sp[1] * sxz;
     const bool inject = fused && n >= 1 && g.nrec > 0;
@@ -273,10 +370,6 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
     const float *axs = sh.ax + (long long)s * g.nx, *bxs = sh.bx + (long long)s * g.nx;
     const float *ays = sh.ay + (long long)s * g.ny, *bys = sh.by + (long long)s * g.ny;
     const float *azs = sh.az + (long long)s * g.nz, *bzs = sh.bz + (long long)s * g.nz;
-    const float ax0 = sx0 >= 0 ? axs[x] : 0.f, bx0 = sx0 >= 0 ? bxs[x] : 0.f;
-    const float axm = sxm >= 0 ? axs[x - 1] : 0.f, axp = sxp >= 0 ? axs[x + 1] : 0.f;
-    const float az0 = sz0 >= 0 ? azs[z] : 0.f, bz0 = sz0 >= 0 ? bzs[z] : 0.f;
-    const float azm = szm >= 0 ? azs[z - 1] : 0.f, azp = szp >= 0 ? azs[z + 1] : 0.f;
     const int csx = g.pxc, csy = g.pyc, csz = g.pzc;
 
     const float *__restrict__ mxy = A.mbar;
@@ -293,42 +386,62 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
     float *__restrict__ vb0 = A.a.v[0] + so;
     float *__restrict__ vb1 = A.a.v[1] + so;
     float *__restrict__ vb2 = A.a.v[2] + so;
-    const float *__restrict__ V0 = A.fn.v[0] + so;
-    const float *__restrict__ V1 = A.fn.v[1] + so;
-    const float *__restrict__ V2 = A.fn.v[2] + so;
     const float *__restrict__ Cx = A.a.px + px_shot(g, s);
     const float *__restrict__ Cy = A.a.py + py_shot(g, s);
     const float *__restrict__ Cz = A.a.pz + pz_shot(g, s);
     float *__restrict__ Cxo = A.a2.px + px_shot(g, s);
     float *__restrict__ Cyo = A.a2.py + py_shot(g, s);
     float *__restrict__ Czo = A.a2.pz + pz_shot(g, s);
-    const float *__restrict__ Fx = A.fn.px + px_shot(g, s);
-    const float *__restrict__ Fy = A.fn.py + py_shot(g, s);
-    const float *__restrict__ Fz = A.fn.pz + pz_shot(g, s);
-    // λ, μ-normal, μ_xy, μ_xz sums: one float4 per cell at the shot's base;
-    // μ_yz sum: a scalar array at component offset 7
-    float4 *__restrict__ acc4v = reinterpret_cast<float4 *>(A.acc + (long long)s * 8 * g.ps);
-    float *__restrict__ accyz = A.acc + ((long long)s * 8 + 7) * g.ps;
+    float *__restrict__ accr = A.acc + ((long long)s * 8 + 4) * g.ps;
 
     for (int y = y0; y < y1; ++y) {
         const int t = x + z * nx + y * sxz;
         const int sy0 = slab_coord(y, g.ny, g.wyl, g.wyh);
         const int sym = slab_coord(y - 1, g.ny, g.wyl, g.wyh);
         const int syp = slab_coord(y + 1, g.ny, g.wyl, g.wyh);
-        const float ay0 = sy0 >= 0 ? ays[y] : 0.f, by0 = sy0 >= 0 ? bys[y] : 0.f;
-        const float aym = sym >= 0 ? ays[y - 1] : 0.f, ayp = syp >= 0 ? ays[y + 1] : 0.f;
 
         const float txx = Txx[t], tyy = Tyy[t], tzz = Tzz[t];
         const float txy = Txy[t], txz = Txz[t], tyz = Tyz[t];
-
-        // ē at p
         const float L0 = lam[t], M0 = mu[t];
-        const float e_xx = c * ((L0 + 2.f * M0) * txx + L0 * (tyy + tzz));
-        const float e_yy = c * ((L0 + 2.f * M0) * tyy + L0 * (txx + tzz));
-        const float e_zz = c * ((L0 + 2.f * M0) * tzz + L0 * (txx + tyy));
-        const float e_xy = c * mxy[t] * txy;
-        const float e_xz = c * mxz[t] * txz;
-        const float e_yz = c * myz[t] * tyz;
+        const float kxy = mxy[t], kxz = mxz[t], kyz = myz[t];
+        const float vo0 = vb0[t], vo1 = vb1[t], vo2 = vb2[t];
+        // x-slab components 0 vx_x, 1 vy_x, 2 vz_x; y: 0 vx_y, 1 vy_y, 2 vz_y;
+        // z: 0 vx_z, 1 vy_z, 2 vz_z.  a = 0 outside the slab; all loads before the first use.
+        float ax0 = 0.f, bx0 = 0.f, ay0 = 0.f, by0 = 0.f, az0 = 0.f, bz0 = 0.f;
+        float axm = 0.f, axp = 0.f, aym = 0.f, ayp = 0.f, azm = 0.f, azp = 0.f;
+        float cxp = 0.f, cxm1 = 0.f, cxm2 = 0.f, cx0 = 0.f, cx1 = 0.f, cx2 = 0.f;
+        float cyp = 0.f, cym0 = 0.f, cym2 = 0.f, cy0 = 0.f, cy1 = 0.f, cy2 = 0.f;
+        float czp = 0.f, czm0 = 0.f, czm1 = 0.f, cz0 = 0.f, cz1 = 0.f, cz2 = 0.f;
+        if (sxp >= 0) { axp = axs[x + 1]; cxp = Cx[px_off(g, y, z, sxp)]; }
+        if (sxm >= 0) {
+            const int pi = px_off(g, y, z, sxm) + csx;
+            axm = axs[x - 1]; cxm1 = Cx[pi]; cxm2 = Cx[pi + csx];
+        }
+        if (sx0 >= 0) {
+            const int pi = px_off(g, y, z, sx0);
+            ax0 = axs[x]; bx0 = bxs[x];
+            cx0 = Cx[pi]; cx1 = Cx[pi + csx]; cx2 = Cx[pi + 2 * csx];
+        }
+        if (syp >= 0) { ayp = ays[y + 1]; cyp = Cy[py_off(g, syp, z, x) + csy]; }
+        if (sym >= 0) {
+            const int pi = py_off(g, sym, z, x);
+            aym = ays[y - 1]; cym0 = Cy[pi]; cym2 = Cy[pi + 2 * csy];
+        }
+        if (sy0 >= 0) {
+            const int pi = py_off(g, sy0, z, x);
+            ay0 = ays[y]; by0 = bys[y];
+            cy0 = Cy[pi]; cy1 = Cy[pi + csy]; cy2 = Cy[pi + 2 * csy];
+        }
+        if (szp >= 0) { azp = azs[z + 1]; czp = Cz[pz_off(g, y, szp, x) + 2 * csz]; }
+        if (szm >= 0) {
+            const int pi = pz_off(g, y, szm, x);
+            azm = azs[z - 1]; czm0 = Cz[pi]; czm1 = Cz[pi + csz];
+        }
+        if (sz0 >= 0) {
+            const int pi = pz_off(g, y, sz0, x);
+            az0 = azs[z]; bz0 = bzs[z];
+            cz0 = Cz[pi]; cz1 = Cz[pi + csz]; cz2 = Cz[pi + 2 * csz];
+        }
         // ē at the neighbours
         float exx_px, eyy_py, ezz_pz;
         {
@@ -352,59 +465,30 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
         const float eyz_mz = c * myz[t - nx] * Tyz[t - nx];     // vy_z at p-z
         const float exz_mx = c * mxz[t - 1] * Txz[t - 1];       // vz_x at p-x
         const float eyz_my = c * myz[t - sxz] * Tyz[t - sxz];   // vz_y at p-y
-
-        float g_vxx_0 = e_xx, g_vxx_p = exx_px;     // vx_x
-        float g_vyy_0 = e_yy, g_vyy_p = eyy_py;     // vy_y
-        float g_vzz_0 = e_zz, g_vzz_p = ezz_pz;     // vz_z
-        float g_vxz_m = exz_mz, g_vxz_0 = e_xz;     // vx_z
-        float g_vxy_m = exy_my, g_vxy_0 = e_xy;     // vx_y
-        float g_vyx_m = exy_mx, g_vyx_0 = e_xy;     // vy_x
-        float g_vyz_m = eyz_mz, g_vyz_0 = e_yz;     // vy_z
-        float g_vzx_m = exz_mx, g_vzx_0 = e_xz;     // vz_x
-        float g_vzy_m = eyz_my, g_vzy_0 = e_yz;     // vz_y
-        // x-slab components 0 vx_x, 1 vy_x, 2 vz_x
-        if (sxp >= 0) g_vxx_p += axp * (Cx[px_off(g, y, z, sxp)] + exx_px);
-        if (sxm >= 0) {
-            const int pi = px_off(g, y, z, sxm) + csx;
-            g_vyx_m += axm * (Cx[pi] + exy_mx);
-            g_vzx_m += axm * (Cx[pi + csx] + exz_mx);
-        }
-        if (sx0 >= 0) {
-            const int pi = px_off(g, y, z, sx0);
-            const float c0 = Cx[pi] + e_xx, c1 = Cx[pi + csx] + e_xy, c2 = Cx[pi + 2 * csx] + e_xz;
-            g_vxx_0 += ax0 * c0; g_vyx_0 += ax0 * c1; g_vzx_0 += ax0 * c2;
-            Cxo[pi] = bx0 * c0; Cxo[pi + csx] = bx0 * c1; Cxo[pi + 2 * csx] = bx0 * c2;
-        }
-        // y-slab components 0 vx_y, 1 vy_y, 2 vz_y
-        if (syp >= 0) g_vyy_p += ayp * (Cy[py_off(g, syp, z, x) + csy] + eyy_py);
-        if (sym >= 0) {
-            const int pi = py_off(g, sym, z, x);
-            g_vxy_m += aym * (Cy[pi] + exy_my);
-            g_vzy_m += aym * (Cy[pi + 2 * csy] + eyz_my);
-        }
-        if (sy0 >= 0) {
-            const int pi = py_off(g, sy0, z, x);
-            const float c0 = Cy[pi] + e_xy, c1 = Cy[pi + csy] + e_yy, c2 = Cy[pi + 2 * csy] + e_yz;
-            g_vxy_0 += ay0 * c0; g_vyy_0 += ay0 * c1; g_vzy_0 += ay0 * c2;
-            Cyo[pi] = by0 * c0; Cyo[pi + csy] = by0 * c1; Cyo[pi + 2 * csy] = by0 * c2;
-        }
-        // z-slab components 0 vx_z, 1 vy_z, 2 vz_z
-        if (szp >= 0) g_vzz_p += azp * (Cz[pz_off(g, y, szp, x) + 2 * csz] + ezz_pz);
-        if (szm >= 0) {
-            const int pi = pz_off(g, y, szm, x);
-            g_vxz_m += azm * (Cz[pi] + exz_mz);
-            g_vyz_m += azm * (Cz[pi + csz] + eyz_mz);
-        }
-        if (sz0 >= 0) {
-            const int pi = pz_off(g, y, sz0, x);
-            const float c0 = Cz[pi] + e_xz, c1 = Cz[pi + csz] + e_yz, c2 = Cz[pi + 2 * csz] + e_zz;
-            g_vxz_0 += az0 * c0; g_vyz_0 += az0 * c1; g_vzz_0 += az0 * c2;
-            Czo[pi] = bz0 * c0; Czo[pi + csz] = bz0 * c1; Czo[pi + 2 * csz] = bz0 * c2;
-        }
+        // ē at p
+        const float e_xx = c * ((L0 + 2.f * M0) * txx + L0 * (tyy + tzz));
+        const float e_yy = c * ((L0 + 2.f * M0) * tyy + L0 * (txx + tzz));
+        const float e_zz = c * ((L0 + 2.f * M0) * tzz + L0 * (txx + tyy));
+        const float e_xy = c * kxy * txy;
+        const float e_xz = c * kxz * txz;
+        const float e_yz = c * kyz * tyz;
+        // ḡ = ē + a(C + ē)
+        cx0 += e_xx; cx1 += e_xy; cx2 += e_xz;
+        cy0 += e_xy; cy1 += e_yy; cy2 += e_yz;
+        cz0 += e_xz; cz1 += e_yz; cz2 += e_zz;
+        const float g_vxx = (e_xx + ax0 * cx0) - (exx_px + axp * (cxp + exx_px));
+        const float g_vyy = (e_yy + ay0 * cy1) - (eyy_py + ayp * (cyp + eyy_py));
+        const float g_vzz = (e_zz + az0 * cz2) - (ezz_pz + azp * (czp + ezz_pz));
+        const float g_vxz = (exz_mz + azm * (czm0 + exz_mz)) - (e_xz + az0 * cz0);
+        const float g_vxy = (exy_my + aym * (cym0 + exy_my)) - (e_xy + ay0 * cy0);
+        const float g_vyx = (exy_mx + axm * (cxm1 + exy_mx)) - (e_xy + ax0 * cx1);
+        const float g_vyz = (eyz_mz + azm * (czm1 + eyz_mz)) - (e_yz + az0 * cz1);
+        const float g_vzx = (exz_mx + axm * (cxm2 + exz_mx)) - (e_xz + ax0 * cx2);
+        const float g_vzy = (eyz_my + aym * (cym2 + eyz_my)) - (e_yz + ay0 * cy2);
         // v̄ += D_vᵀ ḡ
-        float nv0 = vb0[t] + ((g_vxx_0 - g_vxx_p) + (g_vxz_m - g_vxz_0) + (g_vxy_m - g_vxy_0));
-        float nv1 = vb1[t] + ((g_vyy_0 - g_vyy_p) + (g_vyx_m - g_vyx_0) + (g_vyz_m - g_vyz_0));
-        float nv2 = vb2[t] + ((g_vzz_0 - g_vzz_p) + (g_vzx_m - g_vzx_0) + (g_vzy_m - g_vzy_0));
+        float nv0 = vo0 + (g_vxx + g_vxz + g_vxy);
+        float nv1 = vo1 + (g_vyy + g_vyx + g_vyz);
+        float nv2 = vo2 + (g_vzz + g_vzx + g_vzy);
         if (inject && is_receiver(g, sh, s, t)) {      // R1 of step n-1 at this cell's receivers
             for (int r = 0; r < g.nrec; ++r)
                 if (rs[r] == t) {
@@ -413,49 +497,44 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(7, 8
                     nv2 += A.resid[rbase + 2 * rcs + r];
                 }
         }
+        if (im.older) {
+            // ρ: each of the cell's own faces sums v̄·Δv over the steps (k_combine puts in
+            // c·b̄ and gathers the six faces of a cell)
+            float a0 = accr[t], a1 = accr[t + g.ps], a2 = accr[t + 2 * g.ps];
+            const float q0 = LDF(&A.fn.v[0][so + t]), q1 = LDF(&A.fn.v[1][so + t]), q2 = LDF(&A.fn.v[2][so + t]);
+            a0 = fmaf(vo0, LDF(&A.fn1.v[0][so + t]) - q0, a0);
+            a1 = fmaf(vo1, LDF(&A.fn1.v[1][so + t]) - q1, a1);
+            a2 = fmaf(vo2, LDF(&A.fn1.v[2][so + t]) - q2, a2);
+            if (im.newer) {
+                a0 = fmaf(nv0, q0 - LDF(&A.vm1[0][so + t]), a0);
+                a1 = fmaf(nv1, q1 - LDF(&A.vm1[1][so + t]), a1);
+                a2 = fmaf(nv2, q2 - LDF(&A.vm1[2][so + t]), a2);
+            }
+            accr[t] = a0;
+            accr[t + g.ps] = a1;
+            accr[t + 2 * g.ps] = a2;
+        }
         vb0[t] = nv0;
         vb1[t] = nv1;
         vb2[t] = nv2;
+        if (sx0 >= 0) {
+            const int pi = px_off(g, y, z, sx0);
+            Cxo[pi] = bx0 * cx0; Cxo[pi + csx] = bx0 * cx1; Cxo[pi + 2 * csx] = bx0 * cx2;
+        }
+        if (sy0 >= 0) {
+            const int pi = py_off(g, sy0, z, x);
+            Cyo[pi] = by0 * cy0; Cyo[pi + csy] = by0 * cy1; Cyo[pi + 2 * csy] = by0 * cy2;
+        }
+        if (sz0 >= 0) {
+            const int pi = pz_off(g, y, sz0, x);
+            Czo[pi] = bz0 * cz0; Czo[pi + csz] = bz0 * cz1; Czo[pi + 2 * csz] = bz0 * cz2;
+        }
         if (fused && t == tsrc) {                       // R3 of step n: ∂J/∂M += w[n]·τ̄(src)
             const double w = sh.wav[(long long)s * g.ntmax + n];
             double *gm = A.gm6 + 6 * s;
             gm[0] += w * (double)txx; gm[1] += w * (double)tyy; gm[2] += w * (double)tzz;
             gm[3] += w * (double)txy; gm[4] += w * (double)txz; gm[5] += w * (double)tyz;
         }
-
-        // λ, μ accumulators: forward e at p from v^n and ψv^n
-        const float v0 = LDF(&V0[t]), v1 = LDF(&V1[t]), v2 = LDF(&V2[t]);
-        const float d_xx = v0 - LDF(&V0[t - 1]), d_yy = v1 - LDF(&V1[t - sxz]), d_zz = v2 - LDF(&V2[t - nx]);
-        const float d_xz = LDF(&V0[t + nx]) - v0, d_xy = LDF(&V0[t + sxz]) - v0;
-        const float d_yx = LDF(&V1[t + 1]) - v1, d_yz = LDF(&V1[t + nx]) - v1;
-        const float d_zx = LDF(&V2[t + 1]) - v2, d_zy = LDF(&V2[t + sxz]) - v2;
-        float fxx = d_xx, fyy = d_yy, fzz = d_zz, fxz = d_xz, fxy = d_xy;
-        float fyx = d_yx, fyz = d_yz, fzx = d_zx, fzy = d_zy;
-        if (sx0 >= 0) {
-            const int pi = px_off(g, y, z, sx0);
-            fxx += bx0 * LDF(&Fx[pi]) + ax0 * d_xx;
-            fyx += bx0 * LDF(&Fx[pi + csx]) + ax0 * d_yx;
-            fzx += bx0 * LDF(&Fx[pi + 2 * csx]) + ax0 * d_zx;
-        }
-        if (sy0 >= 0) {
-            const int pi = py_off(g, sy0, z, x);
-            fxy += by0 * LDF(&Fy[pi]) + ay0 * d_xy;
-            fyy += by0 * LDF(&Fy[pi + csy]) + ay0 * d_yy;
-            fzy += by0 * LDF(&Fy[pi + 2 * csy]) + ay0 * d_zy;
-        }
-        if (sz0 >= 0) {
-            const int pi = pz_off(g, y, sz0, x);
-            fxz += bz0 * LDF(&Fz[pi]) + az0 * d_xz;
-            fyz += bz0 * LDF(&Fz[pi + csz]) + az0 * d_yz;
-            fzz += bz0 * LDF(&Fz[pi + 2 * csz]) + az0 * d_zz;
-        }
-        float4 a = acc4v[t];
-        a.x += (txx + tyy + tzz) * (fxx + fyy + fzz);
-        a.y += 2.f * (txx * fxx + tyy * fyy + tzz * fzz);
-        a.z += txy * (fxy + fyx);
-        a.w += txz * (fxz + fzx);
-        acc4v[t] = a;
-        accyz[t] += tyz * (fyz + fzy);
     }
 }
 
@@ -524,11 +603,12 @@ __global__ void k_combine(Geo g, const float *mu, const float *mbar, const float
     const long long N = g.ps, nx = g.nx, sxz = g.sxz;   // N: padded component stride
     const float c = g.c;
     const float *mxy = mbar, *mxz = mbar + N, *myz = mbar + 2 * N;
-    (void)bbar;                   // the ρ sums already carry b̄
+    const float *bx = bbar, *by = bbar + N, *bz = bbar + 2 * N;
     float sl = 0.f, sm = 0.f, shear = 0.f, sr = 0.f;
     for (int s = 0; s < g.S; ++s) {
         const float *A = acc + (long long)s * 8 * N;
-        // component k of cell j: 0-3 interleaved at the base, 4 (μ_yz) at 7·N
+        // component k of cell j: 0-3 interleaved at the base, 4 (μ_yz) at 7·N; the ρ sums
+        // of the x, y, z faces at 4·N, 5·N, 6·N
         auto AC = [&](int k, long long j) -> float { return k < 4 ? A[4 * j + k] : A[7 * N + j]; };
         sl += AC(0, i);
         sm += AC(1, i);
@@ -542,14 +622,18 @@ __global__ void k_combine(Geo g, const float *mu, const float *mbar, const float
         shear += sh4(2, mxy, 1, x > 0, sxz, y > 0);
         shear += sh4(3, mxz, 1, x > 0, nx, z > 0);
         shear += sh4(4, myz, sxz, y > 0, nx, z > 0);
-        // the ρ sum holds Σ c·b̄·v̄·Δv over the cell's six faces; per face
-        // ∂J/∂ρ = -(c/2)·b̄²·v̄·F = -(1/(2c))·(c·b̄·v̄·Δv)
-        sr += A[4 * N + i];
+        // a face's sum is Σ v̄·Δv (Δv = c·b̄·F); per face of the cell
+        // ∂J/∂ρ = -(c/2)·b̄²·v̄·F = -½·b̄·(v̄·Δv)
+        const float *R = A + 4 * N;
+        sr += bx[i] * R[i] + by[i] * R[N + i] + bz[i] * R[2 * N + i];
+        if (x > 0) sr += bx[i - 1] * R[i - 1];
+        if (y > 0) sr += by[i - sxz] * R[N + i - sxz];
+        if (z > 0) sr += bz[i - nx] * R[2 * N + i - nx];
     }
     const float m = mu[i];
     glam[i] = c * sl;
     gmu[i] = c * (sm + (m != 0.f ? 0.25f * shear / (m * m) : 0.f));
-    grho[i] = -0.5f / c * sr;
+    grho[i] = -0.5f * sr;
 }
 
 // r = mod - obs and J += ½Σr² (block partial sums in double, one atomic per block)
@@ -598,9 +682,25 @@ __global__ void k_lame_adjoint(const float *vp, const float *vs, const float *rh
 int launch_adj_velocity(const Geo &g, const AdjArgs &A, int n, hipStream_t st) {
     const Tile t = get_tile(2);
     bool launched = false;
-#define X(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity, g, A, n)
-    EFM_TILE_LIST(X)
-#undef X
+#define X_PLAIN(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity, g, A, n)
+#define X_IMAGE(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity_image, g, A, n)
+#define X_STREAM(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity_image_stream, g, A, n)
+    // Streaming reads of the forward state pay where they keep the adjoint's own
+    // working set (15 volumes a shot, 8 of the medium, two sets of ψ slabs) in the
+    // 256 MB Infinity Cache: adjoint step at 128^3 (240 MB) 95 us with the hint, 106
+    // without; above it the hint only drops lines that the neighbouring cells still
+    // read: 256x256x128 463 with, 447 without, 200x200x100 204 and 200.
+    const bool stream = 60 * g.S * g.N + 32 * g.N + 2 * g.S * psi_bytes(g) <= 250LL * 1000 * 1000;
+    if (n % 2 && n != A.n0) {          // image_r2 images nothing in this step
+        EFM_TILE_LIST(X_PLAIN)
+    } else if (stream) {
+        EFM_TILE_LIST(X_STREAM)
+    } else {
+        EFM_TILE_LIST(X_IMAGE)
+    }
+#undef X_PLAIN
+#undef X_IMAGE
+#undef X_STREAM
     if (!launched) return fail(EFM_E_UNSUPPORTED, "unsupported adjoint-velocity tile");
     return check_launch("adjoint velocity sweep");
 }
@@ -660,6 +760,8 @@ static int run_adjoint(const EfmDims *d, const Geo &g, AdjArgs A, const EfmState
         }
         A.fn = make_state(*fwd[n - n0]);
         A.fn1 = make_state(*fwd[n - n0 + 1]);
+        const StatePtrs fm1 = make_state(*fwd[n > n0 ? n - n0 - 1 : 0]);
+        for (int k = 0; k < 3; ++k) A.vm1[k] = fm1.v[k];
         A.a = live;
         A.a2 = other;
         A.a2.v[0] = live.v[0]; A.a2.v[1] = live.v[1]; A.a2.v[2] = live.v[2];
@@ -714,6 +816,8 @@ extern "C" int efm_adjoint(const EfmDims *d, const EfmMedium *m, const float *mb
     A.sh = make_shots(*sh);
     A.resid = resid;
     A.gm6 = gm6;
+    A.n0 = n0;
+    A.n1 = n1;
     return run_adjoint(d, g, A, fwd, adj, adj2, n0, n1, last, true, (hipStream_t)stream);
 }
 
@@ -854,6 +958,8 @@ extern "C" int efm_gradient_static(const EfmDims *d, const EfmMedium *m, const E
     A.sh = make_shots(*sh);
     A.resid = resid;
     A.gm6 = gm6;
+    A.n0 = 0;
+    A.n1 = d->ntmax;
     if ((rc = run_adjoint(d, g, A, fwd, adj, &second, 0, d->ntmax, 1, false, st))) return rc;
     hipLaunchKernelGGL(k_combine, dim3(blocks_for(g.N, 256)), dim3(256), 0, st, g, m->mu, mbar, bbar,
                        acc, glam, gmu, grho);

@@ -95,8 +95,8 @@ int efm_last_error(char *buf, int len);
  * velocity, 3 adjoint stress.  A tile is bx × bz threads, ny cells per thread
  * along y; map 0 launches a linear 3-D grid, map 8 deals contiguous runs of
  * tiles to each of the 8 XCDs (workgroups are dispatched to XCDs round-robin),
- * map 16 does the same over blocks of bx·bz consecutive interior (x, z) cells
- * with rows wrapped (full 64-lane waves whatever nx is).  efm_tile_variants
+ * map 16 does the same over blocks of bx·bz consecutive cells of the (x, z)
+ * plane's memory (full, line-aligned 64-lane waves whatever nx is).  efm_tile_variants
  * writes the compiled tiles as quadruples and returns their count.  The
  * autotuner (autotune.py) drives these. */
 int efm_set_tile(int kernel, int bx, int bz, int ny, int map);
@@ -172,9 +172,8 @@ int efm_derived_medium(const EfmDims *d, const EfmMedium *m, float *mbar, float 
  * the live ψ adjoint is in adj).  resid is ∂J/∂gathers (S, 3, ntmax, nrec).
  * acc (S·8 components of stride N + EFM_PAD, zeroed by the caller) accumulates
  * the λ, μ_n, μ_xy, μ_xz sums (interleaved per cell in components 0-3), the ρ
- * sum (component 4; it also covers the cells one past the interior on the high
- * x, y, z faces) and the μ_yz sum (component 7) of each shot; components 5
- * and 6 are not used.  Only efm_gradient_combine reads it.  gm6 (S, 6) double
+ * sums of each cell's x, y and z face (components 4-6) and the μ_yz sum
+ * (component 7) of each shot.  Only efm_gradient_combine reads it.  gm6 (S, 6) double
  * accumulates ∂J/∂M.  The run is
  * covered by calls over consecutive descending ranges, the first with
  * n1 = ntmax.  Without a receiver mask `last` = 1 marks the call with n0 = 0
