@@ -123,6 +123,10 @@ __device__ __forceinline__ bool interior(int x, int y, int z, const Geo &g) {
     return x >= H && x < g.nx - H && y >= H && y < g.ny - H && z >= H && z < g.nz - H;
 }
 
+// Four consecutive floats read or written with one instruction; 4-byte alignment is
+// enough for global memory.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // ---- error plumbing ---------------------------------------------------------
 void set_error(const std::string &msg);
 int fail(int code, const std::string &msg);

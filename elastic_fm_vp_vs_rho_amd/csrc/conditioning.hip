@@ -18,6 +18,7 @@
 // writes.  All passes are HBM-bound streaming kernels (8 B per cell and pass;
 // the neighbours come from the caches).
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 #include "common.hpp"
@@ -47,33 +48,117 @@ __device__ __forceinline__ bool masked(const Margins &mg, int x, int y, int z, i
     return x < mg.xl || x >= nx - mg.xh || y < mg.yl || y >= ny - mg.yh || z < mg.zl || z >= nz - mg.zh;
 }
 
-// One separable pass along `axis` (0 = y, 1 = z, 2 = x); mask applied when
-// `mask` is set (the last pass).
-__global__ void k_gauss_pass(const float *__restrict__ in, float *__restrict__ out, int nx, int ny,
-                             int nz, int axis, GaussTaps taps, int mask, Margins mg) {
+// The same for -n <= j < 2n (one reflection), without the modulo.
+__device__ __forceinline__ int reflect_once(int j, int n) {
+    return j < 0 ? -1 - j : (j >= n ? 2 * n - 1 - j : j);
+}
+
+// The sum of one output cell from its 2R+1 values, in scipy's order.
+template <int R>
+__device__ __forceinline__ float gauss_sum(const float *v, const GaussTaps &taps) {
 #pragma clang fp contract(off)
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long N = (long long)nx * ny * nz;
-    if (i >= N) return;
-    const int x = (int)(i % nx);
-    const int z = (int)((i / nx) % nz);
-    const int y = (int)(i / ((long long)nx * nz));
-    if (mask && masked(mg, x, y, z, nx, ny, nz)) {
-        out[i] = 0.f;
-        return;
-    }
-    int n, c;
-    long long stride, base;
-    if (axis == 0) { n = ny; c = y; stride = (long long)nx * nz; base = i - (long long)y * stride; }
-    else if (axis == 1) { n = nz; c = z; stride = nx; base = i - (long long)z * nx; }
-    else { n = nx; c = x; stride = 1; base = i - x; }
-    double acc = (double)in[base + (long long)c * stride] * taps.w[0];
-    for (int j = taps.r; j >= 1; --j) {
-        const double a = (double)in[base + (long long)reflect_index(c - j, n) * stride];
-        const double b = (double)in[base + (long long)reflect_index(c + j, n) * stride];
-        acc += (a + b) * taps.w[j];
-    }
-    out[i] = (float)acc;
+    double acc = (double)v[R] * taps.w[0];
+#pragma unroll
+    for (int j = R; j >= 1; --j) acc += ((double)v[R - j] + (double)v[R + j]) * taps.w[j];
+    return (float)acc;
+}
+
+// One separable pass along AXIS (0 = y, 1 = z, 2 = x); mask applied when
+// `mask` is set (the last pass).  Threads are (x, z), the blocks' third index is y, so
+// coordinates cost no division.  Any radius, any line.
+template <int AXIS>
+__global__ __launch_bounds__(256) void k_gauss_pass(const float *__restrict__ in, float *__restrict__ out,
+                                                    int nx, int ny, int nz, GaussTaps taps, int mask,
+                                                    Margins mg) {
+#pragma clang fp contract(off)
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, r = taps.r;
+    if (x >= nx) return;
+    const long long stride = AXIS == 0 ? (long long)nx * nz : AXIS == 1 ? nx : 1;
+    const int n = AXIS == 0 ? ny : AXIS == 1 ? nz : nx;
+    for (int y = blockIdx.z; y < ny; y += gridDim.z)
+        for (int z = blockIdx.y * blockDim.y + threadIdx.y; z < nz; z += gridDim.y * blockDim.y) {
+            const int c = AXIS == 0 ? y : AXIS == 1 ? z : x;
+            const long long i = ((long long)y * nz + z) * nx + x;
+            if (mask && masked(mg, x, y, z, nx, ny, nz)) {
+                out[i] = 0.f;
+                continue;
+            }
+            const float *line = in + (i - c * stride);
+            double acc = (double)line[c * stride] * taps.w[0];
+            if (n >= r) {
+#pragma unroll 4
+                for (int j = r; j >= 1; --j)
+                    acc += ((double)line[reflect_once(c - j, n) * stride] +
+                            (double)line[reflect_once(c + j, n) * stride]) * taps.w[j];
+            } else {
+                for (int j = r; j >= 1; --j)
+                    acc += ((double)line[reflect_index(c - j, n) * stride] +
+                            (double)line[reflect_index(c + j, n) * stride]) * taps.w[j];
+            }
+            out[i] = (float)acc;
+        }
+}
+
+// The pass for radius 4 on lines of at least 4 cells and planes below 2^31 cells (σ = 1
+// with scipy's truncate, the driver's rule): a thread makes NC consecutive cells of
+// its line from NC + 8 values, loaded together.  A pass has 8 bytes a cell to move
+// (6.5 us at 200x200x100 at the copy rate).  One cell a thread with the modulo of the
+// reflected index twice a tap took 38 us, with two selects in its place 20-26: a wave
+// then lived for one round of loads and paid nine conversions to double a cell.  Eight
+// cells of a column a thread: y 14.0, z 10.5 us (four: 16.9, 11.5); four cells of a row
+// as 16-byte loads: x 12.9.  A 33x40x37 volume is launch-bound either way.
+template <int AXIS, int NC>
+__global__ __launch_bounds__(256) void k_gauss_pass4(const float *__restrict__ in, float *__restrict__ out,
+                                                     int nx, int ny, int nz, GaussTaps taps, int mask,
+                                                     Margins mg) {
+    constexpr int R = 4, M = NC + 2 * R;
+    const int x = (blockIdx.x * blockDim.x + threadIdx.x) * (AXIS == 2 ? NC : 1);
+    if (x >= nx) return;
+    const int n = AXIS == 0 ? ny : AXIS == 1 ? nz : nx;
+    constexpr int dy = AXIS == 0 ? NC : 1, dz = AXIS == 1 ? NC : 1;
+    for (int y = blockIdx.z * dy; y < ny; y += gridDim.z * dy)
+        for (int z = (blockIdx.y * blockDim.y + threadIdx.y) * dz; z < nz; z += gridDim.y * blockDim.y * dz) {
+            const int c = AXIS == 0 ? y : AXIS == 1 ? z : x;
+            const long long plane = (long long)nx * nz;
+            float v[M];
+            if (AXIS == 0) {
+                const float *p = in + (z * nx + x);
+#pragma unroll
+                for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n) * plane];
+            } else if (AXIS == 1) {
+                const float *p = in + y * plane;
+#pragma unroll
+                for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n) * nx + x];
+            } else {
+                const float *p = in + y * plane + z * nx;
+                if (c >= R && c + NC + R <= n) {
+#pragma unroll
+                    for (int k = 0; k < M; k += 4) {
+                        const f32x4u a = *reinterpret_cast<const f32x4u *>(p + (c - R + k));
+                        v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n)];
+                }
+            }
+            float o[NC];
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                const bool off = mask && masked(mg, AXIS == 2 ? x + k : x, AXIS == 0 ? y + k : y,
+                                                AXIS == 1 ? z + k : z, nx, ny, nz);
+                o[k] = off ? 0.f : gauss_sum<R>(v + k, taps);
+            }
+            float *q = out + (y * plane + (z * nx + x));
+            if (AXIS == 2 && NC == 4 && c + NC <= n) {
+                f32x4u a = {o[0], o[1 % NC], o[2 % NC], o[3 % NC]};
+                *reinterpret_cast<f32x4u *>(q) = a;
+            } else {
+#pragma unroll
+                for (int k = 0; k < NC; ++k)
+                    if (c + k < n) q[k * (AXIS == 0 ? plane : AXIS == 1 ? (long long)nx : 1LL)] = o[k];
+            }
+        }
 }
 
 __global__ void k_mask_copy(const float *__restrict__ in, float *__restrict__ out, int nx, int ny,
@@ -253,12 +338,31 @@ extern "C" int efm_condition_gradient(const EfmSmooth *p, int nx, int ny, int nz
     for (int j = -r; j <= r; ++j) sum += (phi[j + r] = std::exp(-0.5 / s2 * (double)j * (double)j));
     for (int j = 0; j <= r; ++j) taps.w[j] = phi[j + r] / sum;
     const Margins none{0, 0, 0, 0, 0, 0};
-    hipLaunchKernelGGL(k_gauss_pass, dim3(nblocks(N)), dim3(256), 0, st, in, out, nx, ny, nz, 0, taps, 0, none);
-    if (int rc = check_launch("gaussian pass y")) return rc;
-    hipLaunchKernelGGL(k_gauss_pass, dim3(nblocks(N)), dim3(256), 0, st, out, work, nx, ny, nz, 1, taps, 0, none);
-    if (int rc = check_launch("gaussian pass z")) return rc;
-    hipLaunchKernelGGL(k_gauss_pass, dim3(nblocks(N)), dim3(256), 0, st, work, out, nx, ny, nz, 2, taps, 1, mg);
-    return check_launch("gaussian pass x");
+    auto launch = [&](auto kernel, int dx, int dy, int dz, const float *src, float *dst, int mask, const Margins &m) {
+        const int cells = (nx + dx - 1) / dx, rows = (nz + dz - 1) / dz, planes = (ny + dy - 1) / dy;
+        // rows of 32 lanes where that leaves fewer of them idle than 64
+        const int bx = (cells + 31) / 32 % 2 ? 32 : 64, bz = 256 / bx;
+        hipLaunchKernelGGL(kernel, dim3((cells + bx - 1) / bx, std::min((rows + bz - 1) / bz, 65535),
+                                        std::min(planes, 65535)), dim3(bx, bz), 0, st, src, dst, nx, ny, nz, taps, mask, m);
+    };
+    const bool r4 = r == 4 && (long long)nx * nz <= INT_MAX;
+    auto pass = [&](const float *src, float *dst, int axis, int mask, const Margins &m, const char *what) {
+        const bool fixed = r4 && (axis == 0 ? ny : axis == 1 ? nz : nx) >= r;
+        if (axis == 0) {
+            if (fixed) launch(k_gauss_pass4<0, 8>, 1, 8, 1, src, dst, mask, m);
+            else launch(k_gauss_pass<0>, 1, 1, 1, src, dst, mask, m);
+        } else if (axis == 1) {
+            if (fixed) launch(k_gauss_pass4<1, 8>, 1, 1, 8, src, dst, mask, m);
+            else launch(k_gauss_pass<1>, 1, 1, 1, src, dst, mask, m);
+        } else {
+            if (fixed) launch(k_gauss_pass4<2, 4>, 4, 1, 1, src, dst, mask, m);
+            else launch(k_gauss_pass<2>, 1, 1, 1, src, dst, mask, m);
+        }
+        return check_launch(what);
+    };
+    if (int rc = pass(in, out, 0, 0, none, "gaussian pass y")) return rc;
+    if (int rc = pass(out, work, 1, 0, none, "gaussian pass z")) return rc;
+    return pass(work, out, 2, 1, mg, "gaussian pass x");
 }
 
 extern "C" int efm_model_update(const float *lam0, const float *dlam, double alpha_lam,
