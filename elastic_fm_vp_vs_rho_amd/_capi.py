@@ -111,6 +111,11 @@ _SIGS = {
                       c_void_p, c_void_p, c_int, c_void_p], c_int),
     "efm_net_im2col": ([c_void_p, c_void_p] + [c_int] * 6 + [c_void_p], c_int),
     "efm_net_col2im": ([c_void_p, c_void_p] + [c_int] * 6 + [c_void_p], c_int),
+    "efm_net_conv1d": ([c_void_p] * 5 + [c_int] * 8 + [c_void_p], c_int),
+    "efm_net_conv1d_work": ([c_int] * 7, c_ll),
+    "efm_net_conv1d_dw": ([c_void_p] * 3 + [c_int] * 7 + [c_void_p] * 2, c_int),
+    "efm_net_relu_bias_backward": ([c_void_p] * 4 + [c_int] * 4 + [c_void_p] * 2, c_int),
+    "efm_net_col2im_relu_bias": ([c_void_p] * 4 + [c_int] * 6 + [c_void_p] * 2, c_int),
     "efm_net_relu_backward": ([c_void_p] * 4 + [c_ll, c_void_p], c_int),
     "efm_net_bias_grad": ([c_void_p, c_void_p, c_int, c_ll, c_void_p], c_int),
     "efm_net_mse": ([c_void_p] * 5 + [c_ll, c_float, c_void_p], c_int),

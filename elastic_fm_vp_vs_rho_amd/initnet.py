@@ -148,15 +148,20 @@ class InitNet:
             return b
         s, dev = self.spec, self.dev
         b = {"x": _bf((s.cin, B, s.length), dev)}
-        for i, (ci, co, L, lo) in enumerate(s.convs()):
-            b[f"col{i}"] = _bf((ci * s.ks, B * lo), dev)
+        convs, work = s.convs(), 0
+        for i, (ci, co, L, lo) in enumerate(convs):
             b[f"y{i}"] = _f((co, B * lo), dev)
-            b[f"yb{i}"] = _bf((co, B * lo), dev)
-            b[f"dy{i}"] = _f((co, B * lo), dev)
-            b[f"dp{i}"] = _f((co, B * lo), dev)
+            if i < len(convs) - 1:               # the last block writes its output flattened (X)
+                b[f"yb{i}"] = _bf((co, B * lo), dev)
             b[f"dpb{i}"] = _bf((co, B * lo), dev)
             if i > 0:
                 b[f"dcol{i}"] = _f((ci * s.ks, B * lo), dev)
+            n = self.L.efm_net_conv1d_work(ci, B, L, co, s.ks, s.stride, s.pad)
+            work = max(work, n)
+            if n < 0:            # more than 9 taps or short rows: im2col matrix and GEMM
+                b[f"col{i}"] = _bf((ci * s.ks, B * lo), dev)
+                b["yb_last"] = _bf((co, B * lo), dev)
+        b["work"] = _f((max(work, 2048),), dev)
         b["X"] = _bf((s.flat, B), dev)
         b["z"] = _f((s.hidden, B), dev)
         b["zb"] = _bf((s.hidden, B), dev)
@@ -165,7 +170,6 @@ class InitNet:
         b["dout"] = _f((s.nout, B), dev)
         b["doutb"] = _bf((s.nout, B), dev)
         b["dz"] = _f((s.hidden, B), dev)
-        b["dzp"] = _f((s.hidden, B), dev)
         b["dzpb"] = _bf((s.hidden, B), dev)
         b["dX"] = _f((s.flat, B), dev)
         b["loss"] = torch.zeros(1, dtype=torch.float64, device=dev)
@@ -182,16 +186,23 @@ class InitNet:
     def forward_buffers(self, B):
         """Forward pass on the input already in the B-sized buffer ``x``."""
         s, b, L = self.spec, self._buffers(B), self.L
-        h = b["x"]
+        h, last = b["x"], s.nblocks - 1
         for i, (ci, co, Lin, lo) in enumerate(s.convs()):
-            self._c(L.efm_net_im2col(_ptr(h), _ptr(b[f"col{i}"]), ci, B, Lin, s.ks, s.stride, s.pad,
-                                     _stream()), "efm_net_im2col")
-            K, N = ci * s.ks, B * lo
-            self._gemm(co, N, K, self.wb[f"W{i}"], K, 1, b[f"col{i}"], N, 1, b[f"y{i}"], N,
-                       bias=self.w[f"b{i}"], Cb=b[f"yb{i}"], epi=1)
-            h = b[f"yb{i}"]
-        co, lo = s.channels, s.convs()[-1][3]
-        self._c(L.efm_net_flatten(_ptr(h), _ptr(b["X"]), co, B, lo, _stream()), "efm_net_flatten")
+            out = b["X"] if i == last else b[f"yb{i}"]
+            if f"col{i}" not in b:
+                self._c(L.efm_net_conv1d(_ptr(h), _ptr(self.wb[f"W{i}"]), _ptr(self.w[f"b{i}"]), _ptr(b[f"y{i}"]),
+                                         _ptr(out), ci, B, Lin, co, s.ks, s.stride, s.pad, int(i == last),
+                                         _stream()), "efm_net_conv1d")
+            else:
+                K, N = ci * s.ks, B * lo
+                self._c(L.efm_net_im2col(_ptr(h), _ptr(b[f"col{i}"]), ci, B, Lin, s.ks, s.stride, s.pad, _stream()),
+                        "efm_net_im2col")
+                yb = b["yb_last"] if i == last else out
+                self._gemm(co, N, K, self.wb[f"W{i}"], K, 1, b[f"col{i}"], N, 1, b[f"y{i}"], N,
+                           bias=self.w[f"b{i}"], Cb=yb, epi=1)
+                if i == last:
+                    self._c(L.efm_net_flatten(_ptr(yb), _ptr(out), co, B, lo, _stream()), "efm_net_flatten")
+            h = out
         self._gemm(s.hidden, B, s.flat, self.wb["F1"], s.flat, 1, b["X"], B, 1, b["z"], B,
                    bias=self.w["c1"], Cb=b["zb"], epi=1)
         self._gemm(s.nout, B, s.hidden, self.wb["F2"], s.hidden, 1, b["zb"], B, 1, b["out"], B,
@@ -211,32 +222,33 @@ class InitNet:
         self._c(L.efm_net_bias_grad(_ptr(b["dout"]), _ptr(self.g["c2"]), s.nout, B, _stream()),
                 "efm_net_bias_grad")
         self._gemm(s.hidden, B, s.nout, self.wb["F2"], 1, s.hidden, b["doutb"], B, 1, b["dz"], B)
-        self._c(L.efm_net_relu_backward(_ptr(b["dz"]), _ptr(b["z"]), _ptr(b["dzp"]), _ptr(b["dzpb"]),
-                                        s.hidden * B, _stream()), "efm_net_relu_backward")
+        self._c(L.efm_net_relu_bias_backward(_ptr(b["dz"]), _ptr(b["z"]), _ptr(b["dzpb"]), _ptr(self.g["c1"]),
+                                             s.hidden, B, 0, 0, _ptr(b["work"]), _stream()), "efm_net_relu_bias_backward")
         self._gemm(s.hidden, s.flat, B, b["dzpb"], B, 1, b["X"], 1, B, self.g["F1"], s.flat)
-        self._c(L.efm_net_bias_grad(_ptr(b["dzp"]), _ptr(self.g["c1"]), s.hidden, B, _stream()),
-                "efm_net_bias_grad")
         self._gemm(s.flat, B, s.hidden, self.wb["F1"], 1, s.flat, b["dzpb"], B, 1, b["dX"], B)
-        convs = s.convs()
-        co, lo = convs[-1][1], convs[-1][3]
+        convs, conv = s.convs(), (s.ks, s.stride, s.pad)
         last = len(convs) - 1
-        self._c(L.efm_net_unflatten(_ptr(b["dX"]), _ptr(b[f"dy{last}"]), co, B, lo, _stream()),
-                "efm_net_unflatten")
+        co, lo = convs[last][1], convs[last][3]
+        self._c(L.efm_net_relu_bias_backward(_ptr(b["dX"]), _ptr(b[f"y{last}"]), _ptr(b[f"dpb{last}"]),
+                                             _ptr(self.g[f"b{last}"]), co, B * lo, B, lo, _ptr(b["work"]),
+                                             _stream()),
+                "efm_net_relu_bias_backward")
         for i in range(last, -1, -1):
             ci, co, Lin, lo = convs[i]
             N, K = B * lo, ci * s.ks
-            self._c(L.efm_net_relu_backward(_ptr(b[f"dy{i}"]), _ptr(b[f"y{i}"]), _ptr(b[f"dp{i}"]),
-                                            _ptr(b[f"dpb{i}"]), co * N, _stream()),
-                    "efm_net_relu_backward")
-            # dW = dpre_b · colᵀ, db = Σ dpre
-            self._gemm(co, K, N, b[f"dpb{i}"], N, 1, b[f"col{i}"], 1, N, self.g[f"W{i}"], K)
-            self._c(L.efm_net_bias_grad(_ptr(b[f"dp{i}"]), _ptr(self.g[f"b{i}"]), co, N, _stream()),
-                    "efm_net_bias_grad")
+            h = b["x"] if i == 0 else b[f"yb{i - 1}"]
+            if f"col{i}" in b:
+                self._gemm(co, K, N, b[f"dpb{i}"], N, 1, b[f"col{i}"], 1, N, self.g[f"W{i}"], K)
+            else:
+                self._c(L.efm_net_conv1d_dw(_ptr(b[f"dpb{i}"]), _ptr(h), _ptr(self.g[f"W{i}"]), ci, B, Lin, co,
+                                            *conv, _ptr(b["work"]), _stream()), "efm_net_conv1d_dw")
             if i > 0:
-                # dcol = Wᵀ · dpre_b, then the transposed im2col into the previous layer
+                # dcol = Wᵀ · dpre_b, its transposed im2col is the previous layer's dy
                 self._gemm(K, N, co, self.wb[f"W{i}"], 1, K, b[f"dpb{i}"], N, 1, b[f"dcol{i}"], N)
-                self._c(L.efm_net_col2im(_ptr(b[f"dcol{i}"]), _ptr(b[f"dy{i - 1}"]), ci, B, Lin, s.ks,
-                                         s.stride, s.pad, _stream()), "efm_net_col2im")
+                self._c(L.efm_net_col2im_relu_bias(_ptr(b[f"dcol{i}"]), _ptr(b[f"y{i - 1}"]), _ptr(b[f"dpb{i - 1}"]),
+                                                   _ptr(self.g[f"b{i - 1}"]), ci, B, Lin, *conv,
+                                                   _ptr(b["work"]), _stream()),
+                        "efm_net_col2im_relu_bias")
         return b["loss"]
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):

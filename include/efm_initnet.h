@@ -51,6 +51,31 @@ int efm_net_relu_backward(const float *dy, const float *y, float *dpre, uint16_t
 /* db[m] = sum_n dpre[m*N + n]. */
 int efm_net_bias_grad(const float *dpre, float *db, int M, long long N, void *stream);
 
+/* A convolution with bias and ReLU, its weight gradient, and the ReLU and bias
+ * backward of a layer, without the im2col matrix in memory.  Kernel sizes 1 to 9 over
+ * rows of at least 8 samples (else EFM_E_ARG).
+ * x (C, B, L) BF16, W (M, C·ks) BF16; y[m, b*Lout + l] = max(sum_(c,k) W[m, c*ks + k] *
+ * x[c, b, l*stride + k - pad] + bias[m], 0) (the sums of efm_net_im2col and
+ * efm_net_gemm, bit for bit), yb = bf16(y) at the same offsets or, with flat,
+ * flattened as efm_net_flatten. */
+int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float *bias, float *y, uint16_t *yb,
+                   int C, int B, int L, int M, int ks, int stride, int pad, int flat, void *stream);
+/* Floats of the workspace that suffices for the three calls below on this
+ * convolution's arrays (-1: not a convolution efm_net_conv1d takes). */
+long long efm_net_conv1d_work(int C, int B, int L, int M, int ks, int stride, int pad);
+/* dW (M, C·ks) of dp (M, B·Lout) BF16 against x; a long sum over (b, l) is cut over
+ * blocks and its parts added in a fixed order. */
+int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M,
+                      int ks, int stride, int pad, float *work, void *stream);
+/* dpb = bf16(dy * (y > 0)) and db[m] = sum_n dy * (y > 0) for rows m < M of N values;
+ * dy row-major, or with L > 0 flattened as efm_net_flatten (N = B·L).  work: 2048
+ * floats. */
+int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, int M,
+                               int N, int B, int L, float *work, void *stream);
+/* The same for dy = efm_net_col2im(dcol), y (C, B, L). */
+int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C,
+                             int B, int L, int ks, int stride, int pad, float *work, void *stream);
+
 /* Mean-squared error over n values: *loss += sum (out - t)^2 * inv_n (a device
  * double the caller zeroes); dout = 2 (out - t) inv_n; dout_b (nullable) = bf16(dout). */
 int efm_net_mse(const float *out, const float *target, float *dout, uint16_t *dout_b,
