@@ -274,12 +274,13 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
 }
 
 // Launch KER<bx,bz,ny,map> for the selected tile; sets `launched`.
-#define EFM_LAUNCH_IF(BX_, BZ_, NY_, MAP_, KER, ...)                                           \
-    if (!launched && t.bx == BX_ && t.bz == BZ_ && t.ny == NY_ && t.map == MAP_) {              \
-        hipLaunchKernelGGL((KER<BX_, BZ_, NY_, MAP_>), sweep_grid(g, t), dim3(BX_, BZ_), 0, st, \
-                           __VA_ARGS__);                                                        \
-        launched = true;                                                                       \
+#define EFM_LAUNCH_GRID_IF(BX_, BZ_, NY_, MAP_, GRID, KER, ...)                                       \
+    if (!launched && t.bx == BX_ && t.bz == BZ_ && t.ny == NY_ && t.map == MAP_) {                    \
+        hipLaunchKernelGGL((KER<BX_, BZ_, NY_, MAP_>), GRID, dim3(BX_, BZ_), 0, st, __VA_ARGS__);     \
+        launched = true;                                                                             \
     }
+#define EFM_LAUNCH_IF(BX_, BZ_, NY_, MAP_, KER, ...) \
+    EFM_LAUNCH_GRID_IF(BX_, BZ_, NY_, MAP_, sweep_grid(g, t), KER, __VA_ARGS__)
 #define EFM_KERNEL_ATTRS(BX, BZ, MAP) __launch_bounds__(BX *BZ)
 
 Tile get_tile(int kernel);  // 0 stress, 1 velocity, 2 adjoint-velocity, 3 adjoint-stress
