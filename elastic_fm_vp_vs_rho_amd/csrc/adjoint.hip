@@ -338,21 +338,17 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_stress(Geo g, AdjArgs A, int
     // with a receiver mask this sweep also injects the residual of step n-1 (R1
     // of the next reverse step) and sums ∂J/∂M of step n (R3)
     const bool fused = sh.recmask != nullptr;
-    const int *rs = sh.rec + (long long)s * g.nrec;
-    const long long rcs = (long long)g.ntmax * g.nrec;
-    const long long rbase = ((long long)s * 3 * g.ntmax + (n - 1)) * g.nrec;
     if (n >= nts) {
         // the shot's record ends at step nts - 1: its first residual is injected here
         if (fused && n == nts && n >= 1 && g.nrec > 0)
             for (int y = y0; y < y1; ++y) {
                 const int t = x + z * nx + y * sxz;
+                float v0 = A.a.v[0][so + t], v1 = A.a.v[1][so + t], v2 = A.a.v[2][so + t];
+                inject_wave(g, sh, s, t, A.resid, n - 1, v0, v1, v2);
                 if (!is_receiver(g, sh, s, t)) continue;
-                for (int r = 0; r < g.nrec; ++r)
-                    if (rs[r] == t) {
-                        A.a.v[0][so + t] += A.resid[rbase + r];
-                        A.a.v[1][so + t] += A.resid[rbase + rcs + r];
-                        A.a.v[2][so + t] += A.resid[rbase + 2 * rcs + r];
-                    }
+                A.a.v[0][so + t] = v0;
+                A.a.v[1][so + t] = v1;
+                A.a.v[2][so + t] = v2;
             }
         return;
     }
@@ -489,14 +485,8 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_adj_stress(Geo g, AdjArgs A, int
         float nv0 = vo0 + (g_vxx + g_vxz + g_vxy);
         float nv1 = vo1 + (g_vyy + g_vyx + g_vyz);
         float nv2 = vo2 + (g_vzz + g_vzx + g_vzy);
-        if (inject && is_receiver(g, sh, s, t)) {      // R1 of step n-1 at this cell's receivers
-            for (int r = 0; r < g.nrec; ++r)
-                if (rs[r] == t) {
-                    nv0 += A.resid[rbase + r];
-                    nv1 += A.resid[rbase + rcs + r];
-                    nv2 += A.resid[rbase + 2 * rcs + r];
-                }
-        }
+        // R1 of step n-1 at this cell's receivers
+        if (inject) inject_wave(g, sh, s, t, A.resid, n - 1, nv0, nv1, nv2);
         if (im.older) {
             // ρ: each of the cell's own faces sums v̄·Δv over the steps (k_combine puts in
             // c·b̄ and gathers the six faces of a cell)

@@ -119,6 +119,43 @@ __device__ __forceinline__ bool is_receiver(const Geo &g, const ShotPtrs &sh, in
     return (sh.recmask[(long long)s * g.recw + (t >> 5)] >> (t & 31)) & 1u;
 }
 
+// The receivers among a wave's cells, which follow one another in memory: t is the lane's
+// cell.  The active lanes take the list one receiver each; f(r, lane, hit) is called by all
+// of them for each share of the list, with the lane that owns the cell of this lane's
+// receiver r where there is one (hit).  A lane with a receiver that walked the list by
+// itself kept its wave, and with it the sweep, for 6.5 us per 100 receivers: velocity sweep
+// of 100^3 with 200 receivers 25.7 -> 13.0 us, 64^3 with 16 receivers 6.2 -> 5.7.
+template <typename F>
+__device__ __forceinline__ void wave_receivers(const Geo &g, const ShotPtrs &sh, int s, int t, F f) {
+    const unsigned long long on = __ballot(1);
+    const int lane = __lane_id(), n = __popcll(on), rank = __popcll(on & ((1ull << lane) - 1));
+    const int *rs = sh.rec + (long long)s * g.nrec;
+    for (int r0 = 0; r0 < g.nrec; r0 += n) {
+        const int r = r0 + rank;
+        const int j = (r < g.nrec ? rs[r] : -1) - (t - lane);
+        f(r, j & 63, (unsigned)j < 64u && (on >> (j & 63) & 1));
+    }
+}
+
+// Adds the residual of sample n, res (S, 3, ntmax, nrec), to v at the receivers among the
+// wave's cells, in the order of the list where several share a cell.
+__device__ __forceinline__ void inject_wave(const Geo &g, const ShotPtrs &sh, int s, int t, const float *res, int n,
+                                            float &v0, float &v1, float &v2) {
+    if (!__any(is_receiver(g, sh, s, t))) return;
+    const long long cs = (long long)g.ntmax * g.nrec, base = ((long long)s * 3 * g.ntmax + n) * g.nrec;
+    wave_receivers(g, sh, s, t, [&](int r, int owner, bool hit) __attribute__((always_inline)) {
+        unsigned long long todo = __ballot(hit);
+        if (!todo) return;
+        float q0 = 0.f, q1 = 0.f, q2 = 0.f;
+        if (hit) { q0 = res[base + r]; q1 = res[base + cs + r]; q2 = res[base + 2 * cs + r]; }
+        for (; todo; todo &= todo - 1) {
+            const int i = __ffsll(todo) - 1;
+            const float a0 = __shfl(q0, i), a1 = __shfl(q1, i), a2 = __shfl(q2, i);
+            if ((int)__lane_id() == __shfl(owner, i)) { v0 += a0; v1 += a1; v2 += a2; }
+        }
+    });
+}
+
 __device__ __forceinline__ bool interior(int x, int y, int z, const Geo &g) {
     return x >= H && x < g.nx - H && y >= H && y < g.ny - H && z >= H && z < g.nz - H;
 }

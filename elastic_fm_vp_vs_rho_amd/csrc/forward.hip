@@ -45,17 +45,17 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_velocity(Geo g, Med m, ShotPtrs 
     if (it >= sh.nt[s]) return;
     auto keep = [](int, int, float, float, float) {};
     velocity_cells<NYC>(g, m, sh, in, out, x, z, s, yb, keep, [&](int t, float n0, float n1, float n2) EFM_INLINE {
-        // receiver sampling by the cell's own thread (kernel_get_Station, M:324-335)
-        if (!gathers || !is_receiver(g, sh, s, t)) return;
-        const int *rs = sh.rec + (long long)s * g.nrec;
+        // receiver sampling from the cells' own lanes (kernel_get_Station, M:324-335)
+        if (!gathers || !__any(is_receiver(g, sh, s, t))) return;
         const long long cs = (long long)g.ntmax * g.nrec;
         const long long base = ((long long)s * 3 * g.ntmax + it) * g.nrec;
-        for (int r = 0; r < g.nrec; ++r)
-            if (rs[r] == t) {
-                gathers[base + r] = n0;
-                gathers[base + cs + r] = n1;
-                gathers[base + 2 * cs + r] = n2;
-            }
+        wave_receivers(g, sh, s, t, [&](int r, int owner, bool hit) EFM_INLINE {
+            const float v0 = __shfl(n0, owner), v1 = __shfl(n1, owner), v2 = __shfl(n2, owner);
+            if (!hit) return;
+            gathers[base + r] = v0;
+            gathers[base + cs + r] = v1;
+            gathers[base + 2 * cs + r] = v2;
+        });
     });
 }
 
@@ -106,7 +106,7 @@ __global__ void k_border(Geo g, ShotPtrs sh, StatePtrs st, float *borders, int W
 }
 
 // The stress sweep of step `it` with the border save of step it - 1 in the blocks behind
-// it: both only read v.  A launch of its own took the save 4.7 us of a step's 45 at 100^3,
+// it: both only read v.  A launch of its own took the save 4.7 us of a step's 32 at 100^3,
 // nearly all of it the launch; here it adds 0.5.
 template <int BX, int BZ, int NYC, int MAP>
 __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_stress_save(Geo g, Med m, ShotPtrs sh, StatePtrs in, StatePtrs out,

@@ -225,7 +225,7 @@ __device__ __forceinline__ void restore_guard(const Geo &g, const BorderLayout &
 // (res null: not here), and the reconstruction's velocity sweep of the iteration, from
 // cur to nxt, whose border cells take the saved values of step `slot` and whose x, y and
 // bottom CPML zones stay zero.  Blocks behind the sweeps serve receivers and border
-// elements in the guard rows.  100^3: 28 us, against 12 + 12 + 8 + 5 + 7 us of two sweeps,
+// elements in the guard rows.  100^3: 22.5 us, against 12 + 12 + 8 + 5 + 7 us of two sweeps,
 // injection, border and zeroing.
 template <int BX, int BZ, int NYC, int MAP>
 __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_ref_velocity(Geo g, Med m, ShotPtrs sh, StatePtrs a, StatePtrs cur,
@@ -266,15 +266,7 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_ref_velocity(Geo g, Med m, ShotP
         const int n = sh.nt[s] - it - 1;
         if (n < 0) return;
         velocity_cells<NYC>(g, m, sh, a, a, x, z, s, yb, [&](int, int t, float &v0, float &v1, float &v2) EFM_INLINE {
-            if (!res || !is_receiver(g, sh, s, t)) return;
-            const int *rs = sh.rec + (long long)s * g.nrec;
-            const long long base = ((long long)s * 3 * g.ntmax + n) * g.nrec;
-            for (int r = 0; r < g.nrec; ++r)
-                if (rs[r] == t) {
-                    v0 += res[base + r];
-                    v1 += res[base + cs + r];
-                    v2 += res[base + 2 * cs + r];
-                }
+            if (res) inject_wave(g, sh, s, t, res, n, v0, v1, v2);
         }, [](int, float, float, float) {});
     } else {
         const int y0 = H + yb * NYC, y1 = min(y0 + NYC, g.ny - H);
