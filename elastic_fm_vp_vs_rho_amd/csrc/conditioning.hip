@@ -15,10 +15,10 @@
 // from the outermost inwards) and rounded to float32 per pass, as
 // scipy.ndimage.correlate1d does for float32 arrays; 'reflect' extends a line
 // as (d c b a | a b c d | d c b a).  The masks are applied while the last pass
-// writes.  All passes are HBM-bound streaming kernels (8 B per cell and pass;
-// the neighbours come from the caches).
+// writes.  For the driver's radius the three passes are one kernel (k_gauss4); any other
+// takes a streaming pass per axis (8 B per cell and pass; the neighbours come from the
+// caches).
 #include <algorithm>
-#include <climits>
 #include <cmath>
 
 #include "common.hpp"
@@ -53,13 +53,13 @@ __device__ __forceinline__ int reflect_once(int j, int n) {
     return j < 0 ? -1 - j : (j >= n ? 2 * n - 1 - j : j);
 }
 
-// The sum of one output cell from its 2R+1 values, in scipy's order.
+// The sum of one output cell from its 2R+1 values, in scipy's order (products not rounded).
 template <int R>
 __device__ __forceinline__ float gauss_sum(const float *v, const GaussTaps &taps) {
 #pragma clang fp contract(off)
     double acc = (double)v[R] * taps.w[0];
 #pragma unroll
-    for (int j = R; j >= 1; --j) acc += ((double)v[R - j] + (double)v[R + j]) * taps.w[j];
+    for (int j = R; j >= 1; --j) acc = fma((double)v[R - j] + (double)v[R + j], taps.w[j], acc);
     return (float)acc;
 }
 
@@ -99,66 +99,66 @@ __global__ __launch_bounds__(256) void k_gauss_pass(const float *__restrict__ in
         }
 }
 
-// The pass for radius 4 on lines of at least 4 cells and planes below 2^31 cells (σ = 1
-// with scipy's truncate, the driver's rule): a thread makes NC consecutive cells of
-// its line from NC + 8 values, loaded together.  A pass has 8 bytes a cell to move
-// (6.5 us at 200x200x100 at the copy rate).  One cell a thread with the modulo of the
-// reflected index twice a tap took 38 us, with two selects in its place 20-26: a wave
-// then lived for one round of loads and paid nine conversions to double a cell.  Eight
-// cells of a column a thread: y 14.0, z 10.5 us (four: 16.9, 11.5); four cells of a row
-// as 16-byte loads: x 12.9.  A 33x40x37 volume is launch-bound either way.
-template <int AXIS, int NC>
-__global__ __launch_bounds__(256) void k_gauss_pass4(const float *__restrict__ in, float *__restrict__ out,
-                                                     int nx, int ny, int nz, GaussTaps taps, int mask,
-                                                     Margins mg) {
-    constexpr int R = 4, M = NC + 2 * R;
-    const int x = (blockIdx.x * blockDim.x + threadIdx.x) * (AXIS == 2 ? NC : 1);
-    if (x >= nx) return;
-    const int n = AXIS == 0 ? ny : AXIS == 1 ? nz : nx;
-    constexpr int dy = AXIS == 0 ? NC : 1, dz = AXIS == 1 ? NC : 1;
-    for (int y = blockIdx.z * dy; y < ny; y += gridDim.z * dy)
-        for (int z = (blockIdx.y * blockDim.y + threadIdx.y) * dz; z < nz; z += gridDim.y * blockDim.y * dz) {
-            const int c = AXIS == 0 ? y : AXIS == 1 ? z : x;
-            const long long plane = (long long)nx * nz;
-            float v[M];
-            if (AXIS == 0) {
-                const float *p = in + (z * nx + x);
+// All three passes for radius 4 on lines of at least 4 cells (σ = 1 with scipy's truncate,
+// the driver's rule).  A block makes 64 x TZ x 8 cells (x, z, y): its columns of 16 values
+// along y from memory, 8 sums of each into LDS with the 4 cells on either side in x and z,
+// then the z sums in place (a column of a plane belongs to one thread) and the x sums,
+// four a thread, to memory.  An image is read 2·(TZ + 8)/TZ·72/64 times, mostly from the
+// caches, and written once; three passes moved 8 bytes a cell each and paid three launches
+// of about 4 us.  200x200x100 under the driver's margins: 37.4 us in
+// three passes (13.9 + 10.5 + 13), 24 here, bound by the double sums (about 17 operations
+// for each of 2.6 sums a cell; 16 rows a tile halve the surplus but leave fewer waves: 28).
+constexpr int kTX = 64, kTY = 8, kTZ = 8, kR4 = 4, kGaussThreads = 576;
+__global__ __launch_bounds__(kGaussThreads) void k_gauss4(const float *__restrict__ in, float *__restrict__ out,
+                                                          int nx, int ny, int nz, int ntx, int ntz, GaussTaps taps,
+                                                          Margins mg) {
+    constexpr int W = kTX + 2 * kR4, D = kTZ + 2 * kR4, M = kTY + 2 * kR4;
+    __shared__ __attribute__((aligned(16))) float A[kTY][D][W];
+    const int tile = blockIdx.x, tx = tile % ntx, tz = tile / ntx % ntz, ty = tile / (ntx * ntz);
+    const int x0 = tx * kTX, z0 = tz * kTZ, y0 = ty * kTY;
+    const long long plane = (long long)nx * nz;
+    // a tile the mask covers is only cleared
+    const bool clear = x0 + kTX <= mg.xl || x0 >= nx - mg.xh || y0 + kTY <= mg.yl || y0 >= ny - mg.yh ||
+                       z0 + kTZ <= mg.zl || z0 >= nz - mg.zh;
+    for (int k = threadIdx.x; !clear && k < D * W; k += kGaussThreads) {
+        const int zr = k / W, xr = k - zr * W;
+        const int x = reflect_once(min(x0 + xr - kR4, nx - 1 + kR4), nx);
+        const int z = reflect_once(min(z0 + zr - kR4, nz - 1 + kR4), nz);
+        const float *p = in + ((long long)z * nx + x);
+        float v[M];
 #pragma unroll
-                for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n) * plane];
-            } else if (AXIS == 1) {
-                const float *p = in + y * plane;
+        for (int j = 0; j < M; ++j) v[j] = p[reflect_once(min(y0 + j - kR4, ny - 1 + kR4), ny) * plane];
 #pragma unroll
-                for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n) * nx + x];
-            } else {
-                const float *p = in + y * plane + z * nx;
-                if (c >= R && c + NC + R <= n) {
+        for (int j = 0; j < kTY; ++j) A[j][zr][xr] = gauss_sum<kR4>(v + j, taps);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; !clear && k < kTY * W; k += kGaussThreads) {
+        const int y = k / W, xr = k - y * W;
+        float v[D];
 #pragma unroll
-                    for (int k = 0; k < M; k += 4) {
-                        const f32x4u a = *reinterpret_cast<const f32x4u *>(p + (c - R + k));
-                        v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w;
-                    }
-                } else {
+        for (int j = 0; j < D; ++j) v[j] = A[y][j][xr];
 #pragma unroll
-                    for (int k = 0; k < M; ++k) v[k] = p[reflect_once(min(c + k - R, n - 1 + R), n)];
-                }
-            }
-            float o[NC];
+        for (int j = 0; j < kTZ; ++j) A[y][j][xr] = gauss_sum<kR4>(v + j, taps);
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < kTY * kTZ * (kTX / 4); k += kGaussThreads) {
+        const int q = k % (kTX / 4), zr = k / (kTX / 4) % kTZ, yr = k / (kTX / 4 * kTZ);
+        const int x = x0 + 4 * q, y = y0 + yr, z = z0 + zr;
+        if (x >= nx || y >= ny || z >= nz) continue;
+        float v[4 + 2 * kR4], o[4];
 #pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                const bool off = mask && masked(mg, AXIS == 2 ? x + k : x, AXIS == 0 ? y + k : y,
-                                                AXIS == 1 ? z + k : z, nx, ny, nz);
-                o[k] = off ? 0.f : gauss_sum<R>(v + k, taps);
-            }
-            float *q = out + (y * plane + (z * nx + x));
-            if (AXIS == 2 && NC == 4 && c + NC <= n) {
-                f32x4u a = {o[0], o[1 % NC], o[2 % NC], o[3 % NC]};
-                *reinterpret_cast<f32x4u *>(q) = a;
-            } else {
+        for (int j = 0; j < 4 + 2 * kR4; j += 4)
+            *reinterpret_cast<float4 *>(v + j) = *reinterpret_cast<const float4 *>(&A[yr][zr][4 * q + j]);
 #pragma unroll
-                for (int k = 0; k < NC; ++k)
-                    if (c + k < n) q[k * (AXIS == 0 ? plane : AXIS == 1 ? (long long)nx : 1LL)] = o[k];
-            }
+        for (int j = 0; j < 4; ++j)
+            o[j] = masked(mg, x + j, y, z, nx, ny, nz) ? 0.f : gauss_sum<kR4>(v + j, taps);
+        float *d = out + (y * plane + (long long)z * nx + x);
+        if (x + 4 <= nx) {
+            *reinterpret_cast<f32x4u *>(d) = f32x4u{o[0], o[1], o[2], o[3]};
+        } else {
+            for (int j = 0; j < nx - x; ++j) d[j] = o[j];
         }
+    }
 }
 
 __global__ void k_mask_copy(const float *__restrict__ in, float *__restrict__ out, int nx, int ny,
@@ -345,24 +345,24 @@ extern "C" int efm_condition_gradient(const EfmSmooth *p, int nx, int ny, int nz
         hipLaunchKernelGGL(kernel, dim3((cells + bx - 1) / bx, std::min((rows + bz - 1) / bz, 65535),
                                         std::min(planes, 65535)), dim3(bx, bz), 0, st, src, dst, nx, ny, nz, taps, mask, m);
     };
-    const bool r4 = r == 4 && (long long)nx * nz <= INT_MAX;
-    auto pass = [&](const float *src, float *dst, int axis, int mask, const Margins &m, const char *what) {
-        const bool fixed = r4 && (axis == 0 ? ny : axis == 1 ? nz : nx) >= r;
-        if (axis == 0) {
-            if (fixed) launch(k_gauss_pass4<0, 8>, 1, 8, 1, src, dst, mask, m);
-            else launch(k_gauss_pass<0>, 1, 1, 1, src, dst, mask, m);
-        } else if (axis == 1) {
-            if (fixed) launch(k_gauss_pass4<1, 8>, 1, 1, 8, src, dst, mask, m);
-            else launch(k_gauss_pass<1>, 1, 1, 1, src, dst, mask, m);
-        } else {
-            if (fixed) launch(k_gauss_pass4<2, 4>, 4, 1, 1, src, dst, mask, m);
-            else launch(k_gauss_pass<2>, 1, 1, 1, src, dst, mask, m);
+    if (r == kR4 && nx >= r && ny >= r && nz >= r) {
+        const long long ntx = (nx + kTX - 1) / kTX, ntz = (nz + kTZ - 1) / kTZ, nty = (ny + kTY - 1) / kTY;
+        if (ntx * ntz * nty <= (long long)UINT32_MAX / kGaussThreads) {
+            hipLaunchKernelGGL(k_gauss4, dim3((unsigned)(ntx * ntz * nty)), dim3(kGaussThreads), 0, st, in, out, nx, ny,
+                               nz, (int)ntx, (int)ntz, taps, mg);
+            return check_launch("gaussian smoothing");
         }
+    }
+    auto pass = [&](auto kernel, const float *src, float *dst, int mask, const Margins &m, const char *what) {
+        // rows of 32 lanes where that leaves fewer of them idle than 64
+        const int bx = (nx + 31) / 32 % 2 ? 32 : 64, bz = 256 / bx;
+        hipLaunchKernelGGL(kernel, dim3((nx + bx - 1) / bx, std::min((nz + bz - 1) / bz, 65535), std::min(ny, 65535)),
+                           dim3(bx, bz), 0, st, src, dst, nx, ny, nz, taps, mask, m);
         return check_launch(what);
     };
-    if (int rc = pass(in, out, 0, 0, none, "gaussian pass y")) return rc;
-    if (int rc = pass(out, work, 1, 0, none, "gaussian pass z")) return rc;
-    return pass(work, out, 2, 1, mg, "gaussian pass x");
+    if (int rc = pass(k_gauss_pass<0>, in, out, 0, none, "gaussian pass y")) return rc;
+    if (int rc = pass(k_gauss_pass<1>, out, work, 0, none, "gaussian pass z")) return rc;
+    return pass(k_gauss_pass<2>, work, out, 1, mg, "gaussian pass x");
 }
 
 extern "C" int efm_model_update(const float *lam0, const float *dlam, double alpha_lam,

@@ -43,3 +43,21 @@ def test_xcorr_residual_for_any_trace_count_and_length(gpu_lib, nrec, nt):
         want = ref[s][0]
         assert (np.abs(r[s].double().cpu().numpy() - want) <= 6e-8 * np.abs(want) + 1e-14 * term[0]).all()
     assert abs(float(J) - sum(x[1] for x in ref)) <= 1e-9 * max(1.0, sum(x[1] for x in ref))
+
+
+@pytest.mark.parametrize("shape,margins", [((4, 4, 4), (0,) * 6), ((5, 8, 64), (1, 1, 1, 1, 1, 1)),
+                                           ((8, 9, 65), (3, 0, 0, 2, 8, 0)), ((17, 25, 131), (64, 3, 8, 8, 9, 9)),
+                                           ((9, 7, 67), (0, 67, 0, 0, 0, 0)), ((24, 16, 128), (0, 0, 8, 8, 8, 0))])
+def test_gaussian_tiles_and_masks(gpu_lib, shape, margins):
+    """Tiles of 64 x 8 x 8 cells: volumes around one tile, ragged last tiles, tiles the mask
+    covers in part, whole, and altogether."""
+    g = np.random.default_rng(7).standard_normal(shape).astype(np.float32)
+    ref = gaussian_filter(g, sigma=1.0, mode="reflect", truncate=4.0)
+    ny, nz, nx = shape
+    keep = np.zeros(shape, bool)
+    xl, xh, yl, yh, zl, zh = margins
+    keep[yl:ny - yh, zl:nz - zh, xl:max(xl, nx - xh)] = True
+    ref[~keep] = 0
+    got = C.condition_gradient(torch.as_tensor(g, device="cuda"), 1.0, 4.0, margins).cpu().numpy()
+    assert (got[~keep] == 0).all()
+    assert np.abs(got - ref).max() <= 2e-7 * np.abs(g).max()
