@@ -118,6 +118,9 @@ _SIGS = {
     "efm_net_col2im_relu_bias": ([c_void_p] * 4 + [c_int] * 6 + [c_void_p] * 2, c_int),
     "efm_net_relu_backward": ([c_void_p] * 4 + [c_ll, c_void_p], c_int),
     "efm_net_bias_grad": ([c_void_p, c_void_p, c_int, c_ll, c_void_p], c_int),
+    "efm_net_head_fits": ([c_int] * 4, c_int),
+    "efm_net_head_forward": ([c_void_p] * 8 + [c_int] * 4 + [c_void_p], c_int),
+    "efm_net_head_backward": ([c_void_p] * 10 + [c_int] * 3 + [c_float, c_void_p], c_int),
     "efm_net_mse": ([c_void_p] * 5 + [c_ll, c_float, c_void_p], c_int),
     "efm_net_adam": ([c_void_p] * 5 + [c_ll] + [c_float] * 6 + [c_void_p], c_int),
     "efm_net_flatten": ([c_void_p, c_void_p, c_int, c_int, c_int, c_void_p], c_int),

@@ -557,6 +557,155 @@ __global__ __launch_bounds__(256) void k_col2im_relu_bias(const float *__restric
     });
 }
 
+// ---- the dense head --------------------------------------------------------------------
+// Two small products forward and four backward, each a launch of 4 us or more whatever it
+// holds: the two forward ones walked their sums slab by slab on one or two blocks (11.4 and
+// 6.5 us for 128 x 256 by 64).  Here a block takes 16 examples through both layers,
+// its waves 16 rows each, eight slabs of a row's sum in flight at once: 8.5 us; and one
+// block takes the loss and the last layer back to the hidden layer: 10.3 us in place of six
+// launches (25 us).  MFMA steps of 32 k in rising order, as the general product's.
+__device__ __forceinline__ f32x4 mfma_1(const uint4 &a, const uint4 &b, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(&a),
+                                                   *reinterpret_cast<const bf16x8 *>(&b), acc, 0, 0, 0);
+}
+__host__ __device__ constexpr int up32(int n) { return (n + 31) & ~31; }
+
+__global__ __launch_bounds__(512) void k_head_fwd(int B, int flat, int hidden, int nout,
+                                                  const uint16_t *__restrict__ X, const uint16_t *__restrict__ F1,
+                                                  const float *__restrict__ c1, const uint16_t *__restrict__ F2,
+                                                  const float *__restrict__ c2, float *__restrict__ z,
+                                                  uint16_t *__restrict__ zb, float *__restrict__ out, int xvec,
+                                                  int avec1, int avec2) {
+    extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
+    const int LX = up32(flat) + 8, LZ = up32(hidden) + 8;
+    uint16_t *Xs = sm, *Zs = sm + 16 * LX;                  // [example][k]
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, i = lane & 15, ko = 8 * (lane >> 4);
+    const int n0 = blockIdx.x * 16, col = n0 + i;
+    for (int k = t; k < 2 * up32(flat); k += 512) {
+        const int kk = k >> 1, n = n0 + 8 * (k & 1);
+        const uint4 v = kk < flat ? conv_a8(X, B, flat, kk, n, B, xvec) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) Xs[(8 * (k & 1) + u) * LX + kk] = tap_of(v, 0, u);
+    }
+    for (int k = t; k < 16 * LZ; k += 512) Zs[k] = 0;
+    __syncthreads();
+    for (int r0 = 16 * w; r0 < hidden; r0 += 128) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        int k0 = 0;
+        for (; k0 + 256 <= up32(flat); k0 += 256) {
+            uint4 a[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[u] = conv_a8(F1, flat, hidden, r0 + i, k0 + 32 * u + ko, flat, avec1);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                acc = mfma_1(a[u], *reinterpret_cast<const uint4 *>(&Xs[i * LX + k0 + 32 * u + ko]), acc);
+        }
+        for (; k0 < up32(flat); k0 += 32)
+            acc = mfma_1(conv_a8(F1, flat, hidden, r0 + i, k0 + ko, flat, avec1),
+                         *reinterpret_cast<const uint4 *>(&Xs[i * LX + k0 + ko]), acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = r0 + 4 * (lane >> 4) + r;
+            if (row >= hidden || col >= B) continue;
+            const float v = fmaxf(acc[r] + c1[row], 0.f);
+            z[(long long)row * B + col] = v;
+            zb[(long long)row * B + col] = Zs[i * LZ + row] = f2bf(v);
+        }
+    }
+    __syncthreads();
+    for (int r0 = 16 * w; r0 < nout; r0 += 128) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int k0 = 0; k0 < up32(hidden); k0 += 32)
+            acc = mfma_1(conv_a8(F2, hidden, nout, r0 + i, k0 + ko, hidden, avec2),
+                         *reinterpret_cast<const uint4 *>(&Zs[i * LZ + k0 + ko]), acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = r0 + 4 * (lane >> 4) + r;
+            if (row < nout && col < B) out[(long long)row * B + col] = acc[r] + c2[row];
+        }
+    }
+}
+
+// loss = Σ (out - t)²/n and its way back: dF2, dc2, dc1 and bf16(dz·(z > 0)).  One block;
+// at most kHeadB examples and 16 outputs.
+constexpr int kHeadB = 128;
+__global__ __launch_bounds__(512) void k_head_bwd(int B, int hidden, int nout, float inv_n,
+                                                  const float *__restrict__ out, const float *__restrict__ tg,
+                                                  const float *__restrict__ z, const uint16_t *__restrict__ zb,
+                                                  const uint16_t *__restrict__ F2, float *__restrict__ dF2,
+                                                  float *__restrict__ dc2, float *__restrict__ dc1,
+                                                  uint16_t *__restrict__ dzpb, double *loss, int bvec) {
+    constexpr int LM = kHeadB + 8, LN = 40;
+    __shared__ __attribute__((aligned(16))) uint16_t Dm[16 * LM], Dn[kHeadB * LN];     // bf16(dout): [o][n], [n][o]
+    __shared__ float Df[16][kHeadB];
+    __shared__ double red[512];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, i = lane & 15, ko = 8 * (lane >> 4);
+    for (int k = t; k < 16 * LM; k += 512) Dm[k] = 0;
+    for (int k = t; k < kHeadB * LN; k += 512) Dn[k] = 0;
+    __syncthreads();
+    double s = 0.0;
+    for (int k = t; k < nout * B; k += 512) {
+        const int o = k / B, n = k - o * B;
+        const float r = out[k] - tg[k];
+        s += (double)r * (double)r;
+        const float g = 2.f * r * inv_n;
+        Df[o][n] = g;
+        Dm[o * LM + n] = Dn[n * LN + o] = f2bf(g);
+    }
+    red[t] = s;
+    __syncthreads();
+    for (int o = 256; o > 0; o >>= 1) {
+        if (t < o) red[t] += red[t + o];
+        __syncthreads();
+    }
+    if (t == 0) *loss = red[0] * (double)inv_n;
+    for (int o = w; o < nout; o += 8) {
+        float v = (lane < B ? Df[o][lane] : 0.f) + (lane + 64 < B ? Df[o][lane + 64] : 0.f);
+        for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+        if (lane == 0) dc2[o] = v;
+    }
+    for (int r0 = 16 * w; r0 < hidden; r0 += 128) {
+        // dF2[:, r0 .. r0+15] = dout · zbᵀ
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int k0 = 0; k0 < up32(B); k0 += 32)
+            acc = mfma_1(*reinterpret_cast<const uint4 *>(&Dm[i * LM + k0 + ko]),
+                         conv_a8(zb, B, hidden, r0 + i, k0 + ko, B, bvec), acc);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 4 * (lane >> 4) + r;
+            if (o < nout && r0 + i < hidden) dF2[o * hidden + r0 + i] = acc[r];
+        }
+        // rows r0 .. r0+15 of dz = F2ᵀ · dout
+        uint16_t e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            e[u] = ko + u < nout && r0 + i < hidden ? F2[(ko + u) * hidden + r0 + i] : (uint16_t)0;
+        const uint4 a = pack8(e);
+        float sum[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int n0 = 0; n0 < B; n0 += 16) {
+            const f32x4 dz = mfma_1(a, *reinterpret_cast<const uint4 *>(&Dn[(n0 + i) * LN + ko]),
+                                    f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = r0 + 4 * (lane >> 4) + r;
+                if (row >= hidden || n0 + i >= B) continue;
+                const int p = row * B + n0 + i;
+                const float v = z[p] > 0.f ? dz[r] : 0.f;
+                dzpb[p] = f2bf(v);
+                sum[r] += v;
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            for (int d = 8; d > 0; d >>= 1) sum[r] += __shfl_xor(sum[r], d);
+            const int row = r0 + 4 * (lane >> 4) + r;
+            if (i == 0 && row < hidden) dc1[row] = sum[r];
+        }
+    }
+}
+
 // ---- elementwise / layout kernels -----------------------------------------------
 __global__ void k_cast(const float *__restrict__ x, uint16_t *__restrict__ y, long long n) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
@@ -930,6 +1079,39 @@ extern "C" int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint1
     k_col2im_relu_bias<<<dim3(C, nb), 256, 0, st>>>(dcol, y, dpb, nb > 1 ? work : db, q);
     if (nb > 1) k_sum_rows<<<(C + 63) / 64, 64, 0, st>>>(work, db, C, nb);
     return check_launch("efm_net_col2im_relu_bias");
+}
+
+// 16 examples' inputs and hidden values in 64 KB of LDS.
+static bool head_fits(int B, int flat, int hidden, int nout) {
+    return B > 0 && flat > 0 && hidden > 0 && nout > 0 && (long long)flat + hidden <= 1968 && nout <= 4096 &&
+           (long long)B * (hidden > flat ? hidden : flat) < (1LL << 31);
+}
+
+extern "C" int efm_net_head_fits(int B, int flat, int hidden, int nout) {
+    if (!head_fits(B, flat, hidden, nout)) return 0;
+    return B <= kHeadB && nout <= 16 ? 3 : 1;
+}
+
+extern "C" int efm_net_head_forward(const uint16_t *X, const uint16_t *F1, const float *c1, const uint16_t *F2,
+                                    const float *c2, float *z, uint16_t *zb, float *out, int B, int flat, int hidden,
+                                    int nout, void *stream) {
+    NET_CHECK(X && F1 && c1 && F2 && c2 && z && zb && out && head_fits(B, flat, hidden, nout),
+              "efm_net_head_forward: bad arguments");
+    const auto vec = [](const void *p, int ld) { return (int)(ld % 8 == 0 && (uintptr_t)p % 16 == 0); };
+    const int lds = 16 * (up32(flat) + 8 + up32(hidden) + 8) * 2;
+    k_head_fwd<<<(B + 15) / 16, 512, lds, (hipStream_t)stream>>>(B, flat, hidden, nout, X, F1, c1, F2, c2, z, zb, out,
+                                                                 vec(X, B), vec(F1, flat), vec(F2, hidden));
+    return check_launch("efm_net_head_forward");
+}
+
+extern "C" int efm_net_head_backward(const float *out, const float *target, const float *z, const uint16_t *zb,
+                                     const uint16_t *F2, float *dF2, float *dc2, float *dc1, uint16_t *dzpb,
+                                     double *loss, int B, int hidden, int nout, float inv_n, void *stream) {
+    NET_CHECK(out && target && z && zb && F2 && dF2 && dc2 && dc1 && dzpb && loss && head_fits(B, 1, hidden, nout) &&
+              B <= kHeadB && nout <= 16, "efm_net_head_backward: bad arguments");
+    k_head_bwd<<<1, 512, 0, (hipStream_t)stream>>>(B, hidden, nout, inv_n, out, target, z, zb, F2, dF2, dc2, dc1, dzpb,
+                                                   loss, B % 8 == 0 && (uintptr_t)zb % 16 == 0);
+    return check_launch("efm_net_head_backward");
 }
 
 extern "C" int efm_net_relu_backward(const float *dy, const float *y, float *dpre,

@@ -162,6 +162,7 @@ class InitNet:
                 b[f"col{i}"] = _bf((ci * s.ks, B * lo), dev)
                 b["yb_last"] = _bf((co, B * lo), dev)
         b["work"] = _f((max(work, 2048),), dev)
+        b["head"] = self.L.efm_net_head_fits(B, s.flat, s.hidden, s.nout)
         b["X"] = _bf((s.flat, B), dev)
         b["z"] = _f((s.hidden, B), dev)
         b["zb"] = _bf((s.hidden, B), dev)
@@ -203,18 +204,22 @@ class InitNet:
                 if i == last:
                     self._c(L.efm_net_flatten(_ptr(yb), _ptr(out), co, B, lo, _stream()), "efm_net_flatten")
             h = out
+        if b["head"]:
+            self._c(L.efm_net_head_forward(_ptr(b["X"]), _ptr(self.wb["F1"]), _ptr(self.w["c1"]), _ptr(self.wb["F2"]),
+                                           _ptr(self.w["c2"]), _ptr(b["z"]), _ptr(b["zb"]), _ptr(b["out"]), B, s.flat,
+                                           s.hidden, s.nout, _stream()), "efm_net_head_forward")
+            return b["out"]
         self._gemm(s.hidden, B, s.flat, self.wb["F1"], s.flat, 1, b["X"], B, 1, b["z"], B,
                    bias=self.w["c1"], Cb=b["zb"], epi=1)
         self._gemm(s.nout, B, s.hidden, self.wb["F2"], s.hidden, 1, b["zb"], B, 1, b["out"], B,
                    bias=self.w["c2"], epi=2)
         return b["out"]
 
-    def backward_buffers(self, B):
-        """MSE loss against the buffer ``t`` and every parameter gradient into self.g.
-        Returns the device loss (a 1-element float64 tensor)."""
+    def _head_backward(self, B):
+        """The loss and the last layer's backward as separate kernels."""
         s, b, L = self.spec, self._buffers(B), self.L
-        b["loss"].zero_()
         n = s.nout * B
+        b["loss"].zero_()
         self._c(L.efm_net_mse(_ptr(b["out"]), _ptr(b["t"]), _ptr(b["dout"]), _ptr(b["doutb"]),
                               _ptr(b["loss"]), n, 1.0 / n, _stream()), "efm_net_mse")
         # output layer: dF2 = dout_b · zbᵀ, dc2 = Σ dout, dz = F2ᵀ · dout_b
@@ -223,7 +228,21 @@ class InitNet:
                 "efm_net_bias_grad")
         self._gemm(s.hidden, B, s.nout, self.wb["F2"], 1, s.hidden, b["doutb"], B, 1, b["dz"], B)
         self._c(L.efm_net_relu_bias_backward(_ptr(b["dz"]), _ptr(b["z"]), _ptr(b["dzpb"]), _ptr(self.g["c1"]),
-                                             s.hidden, B, 0, 0, _ptr(b["work"]), _stream()), "efm_net_relu_bias_backward")
+                                             s.hidden, B, 0, 0, _ptr(b["work"]), _stream()),
+                "efm_net_relu_bias_backward")
+
+    def backward_buffers(self, B):
+        """MSE loss against the buffer ``t`` and every parameter gradient into self.g.
+        Returns the device loss (a 1-element float64 tensor)."""
+        s, b, L = self.spec, self._buffers(B), self.L
+        n = s.nout * B
+        if b["head"] == 3:
+            self._c(L.efm_net_head_backward(_ptr(b["out"]), _ptr(b["t"]), _ptr(b["z"]), _ptr(b["zb"]),
+                                            _ptr(self.wb["F2"]), _ptr(self.g["F2"]), _ptr(self.g["c2"]),
+                                            _ptr(self.g["c1"]), _ptr(b["dzpb"]), _ptr(b["loss"]), B, s.hidden, s.nout,
+                                            1.0 / n, _stream()), "efm_net_head_backward")
+        else:
+            self._head_backward(B)
         self._gemm(s.hidden, s.flat, B, b["dzpb"], B, 1, b["X"], 1, B, self.g["F1"], s.flat)
         self._gemm(s.flat, B, s.hidden, self.wb["F1"], 1, s.flat, b["dzpb"], B, 1, b["dX"], B)
         convs, conv = s.convs(), (s.ks, s.stride, s.pad)

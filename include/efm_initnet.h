@@ -76,6 +76,20 @@ int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, f
 int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C,
                              int B, int L, int ks, int stride, int pad, float *work, void *stream);
 
+/* The dense head.  1 if efm_net_head_forward takes these sizes, 3 if efm_net_head_backward
+ * does too (at most 128 examples and 16 outputs), else 0. */
+int efm_net_head_fits(int B, int flat, int hidden, int nout);
+/* z = max(F1·X + c1, 0), zb = bf16(z), out = F2·zb + c2: X (flat, B), F1 (hidden, flat),
+ * F2 (nout, hidden) BF16; the sums of efm_net_gemm, bit for bit. */
+int efm_net_head_forward(const uint16_t *X, const uint16_t *F1, const float *c1, const uint16_t *F2,
+                         const float *c2, float *z, uint16_t *zb, float *out, int B, int flat,
+                         int hidden, int nout, void *stream);
+/* loss = inv_n·sum (out - target)^2 (set, not added), and with dout = 2·inv_n·(out - target):
+ * dF2 = bf16(dout)·zb^T, dc2 = row sums of dout, dzpb = bf16(dz·(z > 0)) and dc1 = row sums
+ * of dz·(z > 0) for dz = F2^T·bf16(dout). */
+int efm_net_head_backward(const float *out, const float *target, const float *z, const uint16_t *zb,
+                          const uint16_t *F2, float *dF2, float *dc2, float *dc1, uint16_t *dzpb,
+                          double *loss, int B, int hidden, int nout, float inv_n, void *stream);
 /* Mean-squared error over n values: *loss += sum (out - t)^2 * inv_n (a device
  * double the caller zeroes); dout = 2 (out - t) inv_n; dout_b (nullable) = bf16(dout). */
 int efm_net_mse(const float *out, const float *target, float *dout, uint16_t *dout_b,
