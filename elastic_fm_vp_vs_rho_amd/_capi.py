@@ -48,6 +48,10 @@ class EfmShots(ctypes.Structure):
                                         "wavelet", "nt", "rec", "recmask")]
 
 
+class EfmNetSum(ctypes.Structure):
+    _fields_ = [("part", c_void_p), ("out", c_void_p), ("n", c_ll), ("si", c_ll), ("sk", c_ll), ("parts", c_int)]
+
+
 P = ctypes.POINTER
 _SIGS = {
     "efm_version": ([], c_int),
@@ -118,6 +122,10 @@ _SIGS = {
     "efm_net_col2im_relu_bias": ([c_void_p] * 4 + [c_int] * 6 + [c_void_p] * 2, c_int),
     "efm_net_relu_backward": ([c_void_p] * 4 + [c_ll, c_void_p], c_int),
     "efm_net_bias_grad": ([c_void_p, c_void_p, c_int, c_ll, c_void_p], c_int),
+    "efm_net_conv1d_back": ([c_void_p] * 5 + [c_int] * 7 + [c_void_p] * 2, c_int),
+    "efm_net_conv1d_parts": ([c_int] * 7, c_int),
+    "efm_net_row_parts": ([c_int] * 2, c_int),
+    "efm_net_sum": ([P(EfmNetSum), c_int, c_void_p], c_int),
     "efm_net_head_fits": ([c_int] * 4, c_int),
     "efm_net_head_forward": ([c_void_p] * 8 + [c_int] * 4 + [c_void_p], c_int),
     "efm_net_head_backward": ([c_void_p] * 10 + [c_int] * 3 + [c_float, c_void_p], c_int),

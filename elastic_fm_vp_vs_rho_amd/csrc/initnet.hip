@@ -188,17 +188,14 @@ __device__ __forceinline__ void gemm_stage(uint16_t *As, uint16_t *Bs, const uin
     }
 }
 
+constexpr int kGemmLds = 2 * (GBM + GBN) * GLD;      // 16-bit words
 template <bool AK, bool BN>
-__global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
-                                                  const uint16_t *__restrict__ A, long long lda,
-                                                  const uint16_t *__restrict__ B, long long ldb,
-                                                  float *__restrict__ C, long long ldc,
-                                                  const float *__restrict__ bias,
-                                                  uint16_t *__restrict__ Cb, int epi) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][GBM * GLD];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][GBN * GLD];
+__device__ __forceinline__ void gemm_tile(uint16_t *sm, int m0, int n0, int M, int N, int K,
+                                          const uint16_t *__restrict__ A, long long lda,
+                                          const uint16_t *__restrict__ B, long long ldb, float *__restrict__ C,
+                                          long long ldc, const float *__restrict__ bias, uint16_t *__restrict__ Cb,
+                                          int epi) {
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int m0 = blockIdx.y * GBM, n0 = blockIdx.x * GBN;
     const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
@@ -207,14 +204,14 @@ __global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
         for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     uint4 va, vb;
     gemm_fetch<AK, BN>(va, vb, t, m0, n0, 0, M, N, K, A, lda, B, ldb);
-    gemm_stage<AK, BN>(As[0], Bs[0], va, vb, t);
+    gemm_stage<AK, BN>(sm, sm + 2 * GBM * GLD, va, vb, t);
     __syncthreads();
     int cur = 0;
     for (int k0 = 0; k0 < K; k0 += GBK) {
         const bool more = k0 + GBK < K;
         if (more) gemm_fetch<AK, BN>(va, vb, t, m0, n0, k0 + GBK, M, N, K, A, lda, B, ldb);
-        mfma_slab(As[cur], Bs[cur], wm, wn, lane, acc);
-        if (more) gemm_stage<AK, BN>(As[cur ^ 1], Bs[cur ^ 1], va, vb, t);
+        mfma_slab(sm + cur * GBM * GLD, sm + (2 * GBM + cur * GBN) * GLD, wm, wn, lane, acc);
+        if (more) gemm_stage<AK, BN>(sm + (cur ^ 1) * GBM * GLD, sm + (2 * GBM + (cur ^ 1) * GBN) * GLD, va, vb, t);
         __syncthreads();
         cur ^= 1;
     }
@@ -235,6 +232,17 @@ __global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
                     if (Cb) Cb[o] = f2bf(v);
                 }
             }
+}
+
+template <bool AK, bool BN>
+__global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
+                                                  const uint16_t *__restrict__ A, long long lda,
+                                                  const uint16_t *__restrict__ B, long long ldb,
+                                                  float *__restrict__ C, long long ldc,
+                                                  const float *__restrict__ bias,
+                                                  uint16_t *__restrict__ Cb, int epi) {
+    __shared__ __attribute__((aligned(16))) uint16_t sm[kGemmLds];
+    gemm_tile<AK, BN>(sm, blockIdx.y * GBM, blockIdx.x * GBN, M, N, K, A, lda, B, ldb, C, ldc, bias, Cb, epi);
 }
 
 // ---- strided 1-D convolutions as implicit GEMMs ------------------------------------
@@ -407,18 +415,19 @@ __global__ __launch_bounds__(256) void k_conv_fwd(ConvShape q, const uint16_t *_
 // dW[m, c·KS + tap] = Σ_(b, l) dp[m, b·Lout + l]·x[c, b, l·stride + tap - pad].  Block tile
 // 64 rows x 16 channels' taps, slabs of 128 samples (two waves of lanes, eight channels to
 // a wave); wave w multiplies rows 16w .. 16w + 15.  The sum over (b, l) is cut over
-// gridDim.z blocks of `chunk` samples and k_sum_parts adds the parts in order: a tile to
-// a block left 229 of 256 CUs idle on the first layer's 16384-deep sum (202 us; 26.5 cut,
-// the second launch included; the four layers 278 -> 61 us).
+// gridDim.z blocks of `chunk` samples and k_sums adds the parts in order: a tile to
+// a block left 229 of 256 CUs idle on the first layer's 16384-deep sum (202 us; 22 cut).
+constexpr int kDwSlab = 128;
+template <int KS> constexpr int kDwLds = (64 + 16 * KS) * (kDwSlab + 8);      // 16-bit words
 template <int KS>
-__global__ __launch_bounds__(256) void k_conv_dw(ConvShape q, const uint16_t *__restrict__ dp,
-                                                 const uint16_t *__restrict__ x, float *__restrict__ out, int chunk,
-                                                 int avec) {
-    constexpr int SLAB = 128, LD = SLAB + 8, NT = 16 * KS;
-    __shared__ __attribute__((aligned(16))) uint16_t As[64 * LD], Bs[NT * LD];
+__device__ __forceinline__ void conv_dw_tile(uint16_t *sm, int bx, int by, int bz, const ConvShape &q,
+                                             const uint16_t *__restrict__ dp, const uint16_t *__restrict__ x,
+                                             float *__restrict__ out, int chunk, int avec) {
+    constexpr int SLAB = kDwSlab, LD = SLAB + 8;
+    uint16_t *As = sm, *Bs = sm + 64 * LD;
     const int N = q.C * KS, K = q.B * q.Lout, BL = q.B * q.L;
-    const int m0 = blockIdx.y * 64, cb = blockIdx.x * 16;
-    const int kbeg = blockIdx.z * chunk, kend = min(kbeg + chunk, K);
+    const int m0 = by * 64, cb = bx * 16;
+    const int kbeg = bz * chunk, kend = min(kbeg + chunk, K);
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int kl = (w & 1) * 64 + lane, cw = cb + (w >> 1) * 8;       // this lane's k of a slab, first channel
     uint4 fa[4], fx[8];
@@ -475,7 +484,7 @@ __global__ __launch_bounds__(256) void k_conv_dw(ConvShape q, const uint16_t *__
         }
         __syncthreads();
     }
-    out += (long long)blockIdx.z * q.M * N;
+    out += (long long)bz * q.M * N;
 #pragma unroll
     for (int j = 0; j < KS; ++j)
 #pragma unroll
@@ -485,22 +494,44 @@ __global__ __launch_bounds__(256) void k_conv_dw(ConvShape q, const uint16_t *__
         }
 }
 
-__global__ void k_sum_parts(const float *__restrict__ part, float *__restrict__ out, long long n, int parts) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float v = 0.f;
-#pragma unroll 8
-    for (int z = 0; z < parts; ++z) v += part[z * n + i];
-    out[i] = v;
+// The weight gradient's blocks, gx·gy·gz of them, and behind them those of dcol = Wᵀ·dp (its
+// gn tiles along (b, l)): both wait for dp only, and each alone leaves much of the chip
+// idle.  Layers 3, 2, 1 of 64 examples: 8.2 + 5.6, 8.6 + 4.9, 8.8 + 7.8 us apart, 8.4, 8.8
+// and 10.5 together.
+template <int KS>
+__global__ __launch_bounds__(256) void k_conv_back(ConvShape q, const uint16_t *__restrict__ dp,
+                                                   const uint16_t *__restrict__ x, float *__restrict__ out, int chunk,
+                                                   int avec, int gx, int gy, int gz, const uint16_t *__restrict__ W,
+                                                   float *__restrict__ dcol, int gn) {
+    __shared__ __attribute__((aligned(16))) uint16_t sm[kDwLds<KS> > kGemmLds ? kDwLds<KS> : kGemmLds];
+    int b = blockIdx.x;
+    if (b < gx * gy * gz) {
+        conv_dw_tile<KS>(sm, b % gx, b / gx % gy, b / (gx * gy), q, dp, x, out, chunk, avec);
+        return;
+    }
+    b -= gx * gy * gz;
+    const int K = q.C * KS, N = q.B * q.Lout;
+    gemm_tile<false, true>(sm, b / gn * GBM, b % gn * GBN, K, N, q.M, W, K, dp, N, dcol, N, nullptr, nullptr, 0);
 }
 
-// db[m] = Σ_k part[m·nb + k]
-__global__ void k_sum_rows(const float *__restrict__ part, float *__restrict__ db, int M, int nb) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M) return;
+// out[i] = Σ_k part[i·si + k·sk] for every sum of the list, in rising k.  One launch for
+// all the cut sums of a backward pass (5.2 us against 4.1 for each of five).
+struct SumList {
+    EfmNetSum s[EFM_NET_SUMS];
+    int first[EFM_NET_SUMS];        // its first block of 256 outputs
+    int n;
+};
+__global__ __launch_bounds__(256) void k_sums(SumList l) {
+    int j = 0;
+    while (j + 1 < l.n && (int)blockIdx.x >= l.first[j + 1]) ++j;
+    const EfmNetSum &s = l.s[j];
+    const long long i = (long long)(blockIdx.x - l.first[j]) * 256 + threadIdx.x;
+    if (i >= s.n) return;
+    const float *p = s.part + i * s.si;
     float v = 0.f;
-    for (int k = 0; k < nb; ++k) v += part[m * nb + k];
-    db[m] = v;
+#pragma unroll 8
+    for (int k = 0; k < s.parts; ++k) v += p[k * s.sk];
+    s.out[i] = v;
 }
 
 // ---- ReLU backward with the bias gradient --------------------------------------------
@@ -1008,7 +1039,7 @@ extern "C" int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float 
 }
 
 // Blocks a tile's sum is cut over: up to two blocks for each of the 256 CUs, of at
-// least two slabs each; sums of four slabs or fewer stay whole (no second launch).
+// least two slabs each; sums of four slabs or fewer stay whole.
 static int dw_splits(const ConvShape &q) {
     const long long tiles = (long long)((q.C + 15) / 16) * ((q.M + 63) / 64);
     const long long slabs = ((long long)q.B * q.Lout + 127) / 128;
@@ -1020,7 +1051,7 @@ static int dw_splits(const ConvShape &q) {
 
 // Blocks a row of N values is cut over: two values to a thread, at most kRowParts blocks
 // in all.  A row to a block leaves 192 of the 256 CUs idle in dependent loads: 64 rows of
-// 16384 / 4096 values 30 / 25 us, cut 11.8 / 9.7 with the launch that adds the parts.
+// 16384 / 4096 values 30 / 25 us, cut 7.5 / 5.6 and a share of the launch that adds parts.
 static constexpr int kRowParts = 2048;
 static int row_blocks(int M, long long N) {
     const long long b = N / 512 < kRowParts / M ? N / 512 : kRowParts / M;
@@ -1035,50 +1066,106 @@ extern "C" long long efm_net_conv1d_work(int C, int B, int L, int M, int ks, int
     return dw > kRowParts ? dw : kRowParts;
 }
 
-extern "C" int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M, int ks,
-                                 int stride, int pad, float *work, void *stream) {
+// The launch of the weight gradient: samples to a block and blocks along the sum.
+static void dw_cut(const ConvShape &q, int &chunk, int &z) {
+    const int K = q.B * q.Lout, want = dw_splits(q);
+    chunk = ((K + want - 1) / want + kDwSlab - 1) / kDwSlab * kDwSlab;
+    z = (K + chunk - 1) / chunk;
+}
+
+extern "C" int efm_net_sum(const EfmNetSum *sums, int n, void *stream) {
+    NET_CHECK(n >= 0 && (sums || n == 0), "efm_net_sum: bad arguments");
+    for (int j0 = 0; j0 < n; j0 += EFM_NET_SUMS) {
+        SumList l{};
+        long long blocks = 0;
+        for (; l.n < EFM_NET_SUMS && j0 + l.n < n; ++l.n) {
+            const EfmNetSum &s = sums[j0 + l.n];
+            NET_CHECK(s.part && s.out && s.n > 0 && s.parts > 0, "efm_net_sum: bad sum");
+            l.s[l.n] = s;
+            l.first[l.n] = (int)blocks;
+            blocks += (s.n + 255) / 256;
+            NET_CHECK(blocks < (1LL << 24), "efm_net_sum: too many outputs");
+        }
+        k_sums<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(l);
+        if (int rc = check_launch("efm_net_sum")) return rc;
+    }
+    return EFM_OK;
+}
+
+extern "C" int efm_net_conv1d_parts(int C, int B, int L, int M, int ks, int stride, int pad) {
     ConvShape q;
-    NET_CHECK(dp && x && dW && work && conv_shape(q, C, B, L, M, ks, stride, pad), "efm_net_conv1d_dw: bad arguments");
-    NET_CHECK((M + 63) / 64 <= 65535, "efm_net_conv1d_dw: M too large");
-    const int K = B * q.Lout, want = dw_splits(q);
-    const int chunk = ((K + want - 1) / want + 127) / 128 * 128, z = (K + chunk - 1) / chunk;
+    if (!conv_shape(q, C, B, L, M, ks, stride, pad)) return -1;
+    int chunk, z;
+    dw_cut(q, chunk, z);
+    return z;
+}
+
+extern "C" int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const uint16_t *W, float *dW, float *dcol,
+                                   int C, int B, int L, int M, int ks, int stride, int pad, float *work,
+                                   void *stream) {
+    ConvShape q;
+    NET_CHECK(dp && x && dW && work && (W || !dcol) && conv_shape(q, C, B, L, M, ks, stride, pad),
+              "efm_net_conv1d_back: bad arguments");
+    int chunk, gz;
+    dw_cut(q, chunk, gz);
+    const int K = B * q.Lout, gx = (C + 15) / 16, gy = (M + 63) / 64;
     const int avec = K % 8 == 0 && (uintptr_t)dp % 16 == 0;
-    const dim3 grid((C + 15) / 16, (M + 63) / 64, z);
-    hipStream_t st = (hipStream_t)stream;
+    // dcol rides along where its product may take 16-byte loads
+    const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0;
+    const int gn = (K + GBN - 1) / GBN;
+    const long long blocks = (long long)gx * gy * gz + (both ? (long long)gn * ((C * ks + GBM - 1) / GBM) : 0);
+    NET_CHECK(blocks < (1LL << 24), "efm_net_conv1d_back: too large");
     switch (ks) {
-#define EFM_CONV(KS) \
-    case KS: k_conv_dw<KS><<<grid, 256, 0, st>>>(q, dp, x, z > 1 ? work : dW, chunk, avec); break;
+#define EFM_CONV(KS)                                                                                              \
+    case KS:                                                                                                      \
+        k_conv_back<KS><<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(q, dp, x, gz > 1 ? work : dW, chunk,   \
+                                                                           avec, gx, gy, gz, W, dcol, gn);        \
+        break;
         EFM_CONV_SIZES(EFM_CONV)
 #undef EFM_CONV
     }
-    if (int rc = check_launch("efm_net_conv1d_dw")) return rc;
+    if (int rc = check_launch("efm_net_conv1d_back")) return rc;
+    if (!dcol || both) return EFM_OK;
+    return efm_net_gemm(C * ks, K, M, W, 1, C * ks, dp, K, 1, dcol, K, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M, int ks,
+                                 int stride, int pad, float *work, void *stream) {
+    if (int rc = efm_net_conv1d_back(dp, x, nullptr, dW, nullptr, C, B, L, M, ks, stride, pad, work, stream)) return rc;
+    const int z = efm_net_conv1d_parts(C, B, L, M, ks, stride, pad);
     if (z == 1) return EFM_OK;
     const long long n = (long long)M * C * ks;
-    k_sum_parts<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(work, dW, n, z);
-    return check_launch("efm_net_conv1d_dw");
+    const EfmNetSum sum{work, dW, n, 1, n, z};
+    return efm_net_sum(&sum, 1, stream);
+}
+
+extern "C" int efm_net_row_parts(int M, int N) { return M > 0 && N > 0 ? row_blocks(M, N) : -1; }
+
+static int sum_rows(const float *work, float *db, int M, int nb, void *stream) {
+    if (!db || nb == 1) return EFM_OK;
+    const EfmNetSum sum{work, db, M, nb, 1, nb};
+    return efm_net_sum(&sum, 1, stream);
 }
 
 extern "C" int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, int M, int N, int B,
                                           int L, float *work, void *stream) {
-    NET_CHECK(dy && y && dpb && db && work && M > 0 && N > 0 && (L <= 0 || (B > 0 && (long long)B * L == N)),
+    NET_CHECK(dy && y && dpb && work && M > 0 && N > 0 && (L <= 0 || (B > 0 && (long long)B * L == N)),
               "efm_net_relu_bias_backward: bad arguments");
     const int nb = row_blocks(M, N);
-    hipStream_t st = (hipStream_t)stream;
-    k_relu_bias<<<dim3(M, nb), 256, 0, st>>>(dy, y, dpb, nb > 1 ? work : db, N, B, L);
-    if (nb > 1) k_sum_rows<<<(M + 63) / 64, 64, 0, st>>>(work, db, M, nb);
-    return check_launch("efm_net_relu_bias_backward");
+    k_relu_bias<<<dim3(M, nb), 256, 0, (hipStream_t)stream>>>(dy, y, dpb, db && nb == 1 ? db : work, N, B, L);
+    if (int rc = check_launch("efm_net_relu_bias_backward")) return rc;
+    return sum_rows(work, db, M, nb, stream);
 }
 
 extern "C" int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C, int B, int L,
                                         int ks, int stride, int pad, float *work, void *stream) {
-    NET_CHECK(dcol && y && dpb && db && work && conv_ok(C, B, L, ks, stride, pad) && (long long)B * L < (1LL << 31),
+    NET_CHECK(dcol && y && dpb && work && conv_ok(C, B, L, ks, stride, pad) && (long long)B * L < (1LL << 31),
               "efm_net_col2im_relu_bias: bad arguments");
     const ConvShape q{C, B, L, 1, ks, stride, pad, (L + 2 * pad - ks) / stride + 1};
     const int nb = row_blocks(C, (long long)B * L);
-    hipStream_t st = (hipStream_t)stream;
-    k_col2im_relu_bias<<<dim3(C, nb), 256, 0, st>>>(dcol, y, dpb, nb > 1 ? work : db, q);
-    if (nb > 1) k_sum_rows<<<(C + 63) / 64, 64, 0, st>>>(work, db, C, nb);
-    return check_launch("efm_net_col2im_relu_bias");
+    k_col2im_relu_bias<<<dim3(C, nb), 256, 0, (hipStream_t)stream>>>(dcol, y, dpb, db && nb == 1 ? db : work, q);
+    if (int rc = check_launch("efm_net_col2im_relu_bias")) return rc;
+    return sum_rows(work, db, C, nb, stream);
 }
 
 // 16 examples' inputs and hidden values in 64 KB of LDS.

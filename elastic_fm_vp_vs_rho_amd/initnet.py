@@ -148,7 +148,14 @@ class InitNet:
             return b
         s, dev = self.spec, self.dev
         b = {"x": _bf((s.cin, B, s.length), dev)}
-        convs, work = s.convs(), 0
+        convs, sums = s.convs(), []
+
+        def add(parts, n, si, sk, out):
+            """A buffer for the parts of sums that one launch adds at the backward's end."""
+            t = _f((parts * n,), dev)
+            sums.append(_capi.EfmNetSum(_ptr(t), _ptr(out), n, si, sk, parts))
+            return t
+
         for i, (ci, co, L, lo) in enumerate(convs):
             b[f"y{i}"] = _f((co, B * lo), dev)
             if i < len(convs) - 1:               # the last block writes its output flattened (X)
@@ -156,12 +163,18 @@ class InitNet:
             b[f"dpb{i}"] = _bf((co, B * lo), dev)
             if i > 0:
                 b[f"dcol{i}"] = _f((ci * s.ks, B * lo), dev)
-            n = self.L.efm_net_conv1d_work(ci, B, L, co, s.ks, s.stride, s.pad)
-            work = max(work, n)
-            if n < 0:            # more than 9 taps or short rows: im2col matrix and GEMM
+            conv = (ci, B, L, co, s.ks, s.stride, s.pad)
+            parts = self.L.efm_net_conv1d_parts(*conv)
+            if parts < 0:        # more than 9 taps or short rows: im2col matrix and GEMM
                 b[f"col{i}"] = _bf((ci * s.ks, B * lo), dev)
                 b["yb_last"] = _bf((co, B * lo), dev)
-        b["work"] = _f((max(work, 2048),), dev)
+            elif parts > 1:
+                b[f"work{i}"] = add(parts, co * ci * s.ks, 1, co * ci * s.ks, self.g[f"W{i}"])
+            rows = self.L.efm_net_row_parts(co, B * lo)
+            if rows > 1:
+                b[f"rows{i}"] = add(rows, co, rows, 1, self.g[f"b{i}"])
+        b["work"] = _f((max(2048, *self.spec.convs()[0][:2], s.hidden),), dev)
+        b["sums"] = (_capi.EfmNetSum * len(sums))(*sums)
         b["head"] = self.L.efm_net_head_fits(B, s.flat, s.hidden, s.nout)
         b["X"] = _bf((s.flat, B), dev)
         b["z"] = _f((s.hidden, B), dev)
@@ -248,26 +261,32 @@ class InitNet:
         convs, conv = s.convs(), (s.ks, s.stride, s.pad)
         last = len(convs) - 1
         co, lo = convs[last][1], convs[last][3]
-        self._c(L.efm_net_relu_bias_backward(_ptr(b["dX"]), _ptr(b[f"y{last}"]), _ptr(b[f"dpb{last}"]),
-                                             _ptr(self.g[f"b{last}"]), co, B * lo, B, lo, _ptr(b["work"]),
-                                             _stream()),
-                "efm_net_relu_bias_backward")
+        def rows(i):
+            """Where layer i's bias gradient goes: (db, work) of the ReLU backward."""
+            return (None, _ptr(b[f"rows{i}"])) if f"rows{i}" in b else (_ptr(self.g[f"b{i}"]), _ptr(b["work"]))
+
+        db, work = rows(last)
+        self._c(L.efm_net_relu_bias_backward(_ptr(b["dX"]), _ptr(b[f"y{last}"]), _ptr(b[f"dpb{last}"]), db, co, B * lo,
+                                             B, lo, work, _stream()), "efm_net_relu_bias_backward")
         for i in range(last, -1, -1):
             ci, co, Lin, lo = convs[i]
             N, K = B * lo, ci * s.ks
             h = b["x"] if i == 0 else b[f"yb{i - 1}"]
+            # dW, and dcol = Wᵀ · dpre_b, whose transposed im2col is the previous layer's dy
             if f"col{i}" in b:
                 self._gemm(co, K, N, b[f"dpb{i}"], N, 1, b[f"col{i}"], 1, N, self.g[f"W{i}"], K)
+                if i > 0:
+                    self._gemm(K, N, co, self.wb[f"W{i}"], 1, K, b[f"dpb{i}"], N, 1, b[f"dcol{i}"], N)
             else:
-                self._c(L.efm_net_conv1d_dw(_ptr(b[f"dpb{i}"]), _ptr(h), _ptr(self.g[f"W{i}"]), ci, B, Lin, co,
-                                            *conv, _ptr(b["work"]), _stream()), "efm_net_conv1d_dw")
+                self._c(L.efm_net_conv1d_back(_ptr(b[f"dpb{i}"]), _ptr(h), _ptr(self.wb[f"W{i}"]),
+                                              _ptr(self.g[f"W{i}"]), _ptr(b[f"dcol{i}"]) if i > 0 else None, ci, B,
+                                              Lin, co, *conv, _ptr(b.get(f"work{i}", b["work"])), _stream()),
+                        "efm_net_conv1d_back")
             if i > 0:
-                # dcol = Wᵀ · dpre_b, its transposed im2col is the previous layer's dy
-                self._gemm(K, N, co, self.wb[f"W{i}"], 1, K, b[f"dpb{i}"], N, 1, b[f"dcol{i}"], N)
+                db, work = rows(i - 1)
                 self._c(L.efm_net_col2im_relu_bias(_ptr(b[f"dcol{i}"]), _ptr(b[f"y{i - 1}"]), _ptr(b[f"dpb{i - 1}"]),
-                                                   _ptr(self.g[f"b{i - 1}"]), ci, B, Lin, *conv,
-                                                   _ptr(b["work"]), _stream()),
-                        "efm_net_col2im_relu_bias")
+                                                   db, ci, B, Lin, *conv, work, _stream()), "efm_net_col2im_relu_bias")
+        self._c(L.efm_net_sum(b["sums"], len(b["sums"]), _stream()), "efm_net_sum")
         return b["loss"]
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):

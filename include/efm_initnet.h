@@ -67,14 +67,33 @@ long long efm_net_conv1d_work(int C, int B, int L, int M, int ks, int stride, in
  * blocks and its parts added in a fixed order. */
 int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M,
                       int ks, int stride, int pad, float *work, void *stream);
+/* The same, and dcol = W^T·dp (C·ks, B·Lout) beside it unless null; where the sum is cut
+ * (efm_net_conv1d_parts > 1 of them) its parts are left in work, M·C·ks floats each, and
+ * dW is not written. */
+int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const uint16_t *W, float *dW, float *dcol,
+                        int C, int B, int L, int M, int ks, int stride, int pad, float *work,
+                        void *stream);
+int efm_net_conv1d_parts(int C, int B, int L, int M, int ks, int stride, int pad);
 /* dpb = bf16(dy * (y > 0)) and db[m] = sum_n dy * (y > 0) for rows m < M of N values;
  * dy row-major, or with L > 0 flattened as efm_net_flatten (N = B·L).  work: 2048
- * floats. */
+ * floats, and at least M; with db null the row's parts stay there (efm_net_row_parts
+ * of them, one after the other for each row). */
 int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, int M,
                                int N, int B, int L, float *work, void *stream);
+int efm_net_row_parts(int M, int N);
 /* The same for dy = efm_net_col2im(dcol), y (C, B, L). */
 int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C,
                              int B, int L, int ks, int stride, int pad, float *work, void *stream);
+/* out[i] = sum over k < parts of part[i*si + k*sk], i < n, in rising k, for n sums;
+ * EFM_NET_SUMS of them to a launch. */
+#define EFM_NET_SUMS 12
+typedef struct {
+    const float *part;
+    float *out;
+    long long n, si, sk;
+    int parts;
+} EfmNetSum;
+int efm_net_sum(const EfmNetSum *sums, int n, void *stream);
 
 /* The dense head.  1 if efm_net_head_forward takes these sizes, 3 if efm_net_head_backward
  * does too (at most 128 examples and 16 outputs), else 0. */

@@ -9,6 +9,8 @@ in any order (the worst case, or four standard deviations) of u = 2^-23, twice t
 rounding to nearest, as the matrix instruction may truncate inside.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -147,3 +149,43 @@ def test_gather_batch_rows(length):
     t = torch.empty(nout, B, device="cuda")
     _ok(lib.efm_net_gather_batch(_p(data), _p(target), data.shape[0], _p(idx), B, C, length, nout, _p(x), _p(t), None))
     assert torch.equal(x, data[idx.long()].permute(1, 0, 2)) and torch.equal(t, target[idx.long()].T)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_conv_backward_in_one_launch(shape):
+    """dW's parts and dcol from one launch: the separate calls' bits (the parts left unsummed
+    where there are several, dcol through the general product where it cannot ride along)."""
+    C, B, L, M, ks, stride, pad = shape
+    lib, Lout = _capi.lib(), (L + 2 * pad - ks) // stride + 1
+    g = torch.Generator().manual_seed(2 + sum(shape))
+    x, W = torch.randn(C, B, L, generator=g).bfloat16().cuda(), torch.randn(M, C * ks, generator=g).bfloat16().cuda()
+    dp = torch.randn(M, B * Lout, generator=g).bfloat16().cuda()
+    K, N, n = C * ks, B * Lout, M * C * ks
+    conv = (C, B, L, M, ks, stride, pad)
+    parts = lib.efm_net_conv1d_parts(*conv)
+    work = torch.zeros(max(parts * n, lib.efm_net_conv1d_work(*conv)), device="cuda")
+    dW, got, dcol, want = (torch.full(s, 7.0, device="cuda") for s in ((M, K), (M, K), (K, N), (K, N)))
+    _ok(lib.efm_net_conv1d_back(_p(dp), _p(x), _p(W), _p(got), _p(dcol), *conv, _p(work), None))
+    if parts > 1:
+        assert (got == 7.0).all()
+        s = _capi.EfmNetSum(_p(work), _p(got), n, 1, n, parts)
+        _ok(lib.efm_net_sum(ctypes.byref(s), 1, None))
+    _ok(lib.efm_net_conv1d_dw(_p(dp), _p(x), _p(dW), *conv, _p(work), None))
+    _ok(lib.efm_net_gemm(K, N, M, _p(W), 1, K, _p(dp), N, 1, _p(want), N, None, None, 0, None))
+    torch.cuda.synchronize()
+    assert torch.equal(got, dW) and torch.equal(dcol, want)
+
+
+@pytest.mark.parametrize("count", [0, 1, 12, 13, 30])
+def test_sum_lists(count):
+    """Lists below, at and above a launch's twelve sums; parts side by side and one after the other."""
+    lib, rng = _capi.lib(), np.random.default_rng(count)
+    ins, outs, sums = [], [], (_capi.EfmNetSum * count)()
+    for j in range(count):
+        n, k = int(rng.integers(1, 700)), int(rng.integers(1, 9))
+        ins.append(torch.as_tensor(rng.integers(-8, 9, (k, n) if j % 2 else (n, k)).astype(np.float32)).cuda())
+        outs.append(torch.empty(n, device="cuda"))
+        sums[j] = _capi.EfmNetSum(_p(ins[j]), _p(outs[j]), n, 1 if j % 2 else k, n if j % 2 else 1, k)
+    _ok(lib.efm_net_sum(sums, count, None))
+    for j in range(count):
+        assert torch.equal(outs[j], ins[j].sum(0 if j % 2 else 1))          # whole numbers: exact
