@@ -190,12 +190,12 @@ __device__ __forceinline__ void gemm_stage(uint16_t *As, uint16_t *Bs, const uin
 
 constexpr int kGemmLds = 2 * (GBM + GBN) * GLD;      // 16-bit words
 template <bool AK, bool BN>
-__device__ __forceinline__ void gemm_tile(uint16_t *sm, int m0, int n0, int M, int N, int K,
+__device__ __forceinline__ void gemm_tile(uint16_t *sm, int t, int m0, int n0, int M, int N, int K,
                                           const uint16_t *__restrict__ A, long long lda,
                                           const uint16_t *__restrict__ B, long long ldb, float *__restrict__ C,
                                           long long ldc, const float *__restrict__ bias, uint16_t *__restrict__ Cb,
                                           int epi) {
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int lane = t & 63, w = t >> 6;
     const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
                                                   const float *__restrict__ bias,
                                                   uint16_t *__restrict__ Cb, int epi) {
     __shared__ __attribute__((aligned(16))) uint16_t sm[kGemmLds];
-    gemm_tile<AK, BN>(sm, blockIdx.y * GBM, blockIdx.x * GBN, M, N, K, A, lda, B, ldb, C, ldc, bias, Cb, epi);
+    gemm_tile<AK, BN>(sm, threadIdx.x, blockIdx.y * GBM, blockIdx.x * GBN, M, N, K, A, lda, B, ldb, C, ldc, bias, Cb, epi);
 }
 
 // ---- strided 1-D convolutions as implicit GEMMs ------------------------------------
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void k_gemm_vec(int M, int N, int K,
 // LDS as [column][k].  A slab's loads are issued before the MFMAs of the slab before
 // it.  Few wide loads also keep the kernels short: they run for one to six slabs, and
 // unrolled over 72 two-byte loads they spent their time fetching instructions (the four
-// layers of 64 examples, 192 channels of 1024: forward 33 + 3 x 13 us that way, 23 + 3 x 10.7
+// layers of 64 examples, 192 channels of 1024: forward 33 + 3 x 13 us that way, 19 + 3 x 7.9
 // now, against 192 us of im2col, GEMM and flatten over the stored matrix).
 struct ConvShape {
     int C, B, L, M, ks, stride, pad, Lout;
@@ -318,105 +318,101 @@ __device__ __forceinline__ uint16_t tap_of(const uint4 &v, uint16_t n, int k) {
 // y[m, b·Lout + l] = max(Σ W·x + bias, 0); yb = bf16(y) at the same place, or flattened
 // for the dense head (yb[(m·Lout + l)·B + b]).  Block tile 64 x 64, slabs of 32
 // channels: a multiple of 32 k for any KS, so that the MFMA steps and the bits are those
-// of the GEMM over the stored matrix, and 8 whole channels to each wave.
+// of the GEMM over the stored matrix.  16 waves, two whole channels of a slab and one MFMA
+// tile each: the kernel lasts two to six slabs, so it is the few hundred instructions and the
+// loads' latency of a slab that it waits for (first layer and the others, us: 4 waves
+// 22.7 and 10.7, 8 waves 19.6 and 8.7, 16 waves 18.8 and 7.9; with two slabs' loads in
+// flight 19.2 and 8.4).
+constexpr int kFwdWaves = 16, kFwdThreads = 64 * kFwdWaves;
 template <int KS>
-__global__ __launch_bounds__(256) void k_conv_fwd(ConvShape q, const uint16_t *__restrict__ x,
-                                                  const uint16_t *__restrict__ W, const float *__restrict__ bias,
-                                                  float *__restrict__ y, uint16_t *__restrict__ yb, int flat,
-                                                  int avec) {
-    constexpr int SLAB = 32 * KS, LD = SLAB + 8;
+struct FwdSlab {
+    static constexpr int NA = (64 * 4 * KS + kFwdThreads - 1) / kFwdThreads;
+    uint4 a[NA], x[2];
+    uint16_t x9[2];
+};
+template <int KS>
+__global__ __launch_bounds__(kFwdThreads) void k_conv_fwd(ConvShape q, const uint16_t *__restrict__ x,
+                                                          const uint16_t *__restrict__ W,
+                                                          const float *__restrict__ bias, float *__restrict__ y,
+                                                          uint16_t *__restrict__ yb, int flat, int avec) {
+    constexpr int SLAB = 32 * KS, LD = SLAB + 8, NA = FwdSlab<KS>::NA;
+    static_assert(kFwdWaves * 2 == 32, "two channels of a slab to a wave");
     __shared__ __attribute__((aligned(16))) uint16_t As[64 * LD], Bs[64 * LD];
     const int N = q.B * q.Lout, K = q.C * KS, BL = q.B * q.L;
     const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
+    const int wm = (w >> 2) * 16, wn = (w & 3) * 16;
     const int n = min(n0 + lane, N - 1), b = n / q.Lout;      // lanes past the last column repeat it
     const Taps tp = conv_taps(q, b, n - b * q.Lout);
     const bool edge = __any(tp.shift != 0 || !tp.has9);
-    uint4 fa[KS], fx[8];
-    uint16_t f9[8];
-    auto fetch = [&](int c0) {
+    auto fetch = [&](FwdSlab<KS> &f, int c0) __attribute__((always_inline)) {
+        if (c0 >= q.C) return;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint16_t *p = x + (long long)min(c0 + 8 * w + j, q.C - 1) * BL;
+        for (int j = 0; j < 2; ++j) {
+            const uint16_t *p = x + (long long)min(c0 + 2 * w + j, q.C - 1) * BL;
             const u32x4u v = *reinterpret_cast<const u32x4u *>(p + tp.first);
-            fx[j] = make_uint4(v.x, v.y, v.z, v.w);
-            if (KS > 8) f9[j] = p[tp.ninth];
+            f.x[j] = make_uint4(v.x, v.y, v.z, v.w);
+            f.x9[j] = KS > 8 ? p[tp.ninth] : (uint16_t)0;
         }
 #pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            const int j = t + 256 * i, row = j / (4 * KS), kv = (j - row * (4 * KS)) * 8;
-            fa[i] = conv_a8(W, K, q.M, m0 + row, c0 * KS + kv, K, avec);
+        for (int i = 0; i < NA; ++i) {
+            const int j = t + kFwdThreads * i, row = j / (4 * KS), kv = (j - row * (4 * KS)) * 8;
+            if (row < 64) f.a[i] = conv_a8(W, K, q.M, m0 + row, c0 * KS + kv, K, avec);
         }
     };
-    f32x4 acc[2][2] = {};
-    fetch(0);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    FwdSlab<KS> f;
+    fetch(f, 0);
 #pragma unroll 1
     for (int c0 = 0; c0 < q.C; c0 += 32) {
-        if (edge) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                fx[j] = shift_taps(fx[j], tp.shift);
-                if (!tp.has9) f9[j] = 0;
+        for (int j = 0; j < 2; ++j) {
+            if (edge) {
+                f.x[j] = shift_taps(f.x[j], tp.shift);
+                if (!tp.has9) f.x9[j] = 0;
             }
-        }
-        if (c0 + 32 > q.C) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (c0 + 8 * w + j >= q.C) { fx[j] = make_uint4(0, 0, 0, 0); f9[j] = 0; }
+            if (c0 + 2 * w + j >= q.C) { f.x[j] = make_uint4(0, 0, 0, 0); f.x9[j] = 0; }
         }
 #pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            const int j = t + 256 * i, row = j / (4 * KS), kv = (j - row * (4 * KS)) * 8;
-            *reinterpret_cast<uint4 *>(&As[row * LD + kv]) = fa[i];
-            uint16_t e[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) e[u] = tap_of(fx[(8 * i + u) / KS], f9[(8 * i + u) / KS], (8 * i + u) % KS);
-            *reinterpret_cast<uint4 *>(&Bs[lane * LD + 8 * KS * w + 8 * i]) = pack8(e);
+        for (int i = 0; i < NA; ++i) {
+            const int j = t + kFwdThreads * i, row = j / (4 * KS), kv = (j - row * (4 * KS)) * 8;
+            if (row < 64) *reinterpret_cast<uint4 *>(&As[row * LD + kv]) = f.a[i];
         }
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+            *reinterpret_cast<unsigned *>(&Bs[lane * LD + 2 * KS * w + 2 * i]) =
+                tap_of(f.x[2 * i / KS], f.x9[2 * i / KS], 2 * i % KS) |
+                (unsigned)tap_of(f.x[(2 * i + 1) / KS], f.x9[(2 * i + 1) / KS], (2 * i + 1) % KS) << 16;
         __syncthreads();
-        if (c0 + 32 < q.C) fetch(c0 + 32);
+        fetch(f, c0 + 32);
         const int ko = 8 * (lane >> 4);
 #pragma unroll 3
-        for (int kk = 0; kk < SLAB; kk += 32) {
-            bf16x8 fa2[2], fb2[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                fa2[i] = *reinterpret_cast<const bf16x8 *>(&As[(wm + 16 * i + (lane & 15)) * LD + kk + ko]);
-                fb2[i] = *reinterpret_cast<const bf16x8 *>(&Bs[(wn + 16 * i + (lane & 15)) * LD + kk + ko]);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa2[i], fb2[j], acc[i][j], 0, 0, 0);
-        }
+        for (int kk = 0; kk < SLAB; kk += 32)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                *reinterpret_cast<const bf16x8 *>(&As[(wm + (lane & 15)) * LD + kk + ko]),
+                *reinterpret_cast<const bf16x8 *>(&Bs[(wn + (lane & 15)) * LD + kk + ko]), acc, 0, 0, 0);
         __syncthreads();
     }
+    const int col = n0 + wn + (lane & 15);
+    if (col >= N) return;
+    const int bb = col / q.Lout, ll = col - bb * q.Lout;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int col = n0 + wn + 16 * j + (lane & 15);
-        if (col >= N) continue;
-        const int bb = col / q.Lout, ll = col - bb * q.Lout;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm + 16 * i + 4 * (lane >> 4) + r;
-                if (row >= q.M) continue;
-                const float v = fmaxf(acc[i][j][r] + bias[row], 0.f);
-                const long long o = (long long)row * N + col;
-                y[o] = v;
-                yb[flat ? ((long long)row * q.Lout + ll) * q.B + bb : o] = f2bf(v);
-            }
+    for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + 4 * (lane >> 4) + r;
+        if (row >= q.M) continue;
+        const float v = fmaxf(acc[r] + bias[row], 0.f);
+        const long long o = (long long)row * N + col;
+        y[o] = v;
+        yb[flat ? ((long long)row * q.Lout + ll) * q.B + bb : o] = f2bf(v);
     }
 }
 
 // dW[m, c·KS + tap] = Σ_(b, l) dp[m, b·Lout + l]·x[c, b, l·stride + tap - pad].  Block tile
-// 64 rows x 16 channels' taps, slabs of 128 samples (two waves of lanes, eight channels to
-// a wave); wave w multiplies rows 16w .. 16w + 15.  The sum over (b, l) is cut over
-// gridDim.z blocks of `chunk` samples and k_sums adds the parts in order: a tile to
-// a block left 229 of 256 CUs idle on the first layer's 16384-deep sum (202 us; 22 cut).
+// 64 rows x 16 channels' taps, slabs of 128 samples: of 16 waves two take each pair of
+// channels, 64 samples each; wave w multiplies rows 16(w/4) .. and every fourth column
+// tile from w mod 4.  The sum over (b, l) is cut over gz blocks of `chunk` samples and
+// k_sums adds the parts in order: a tile to a block left 229 of 256 CUs idle on the
+// first layer's 16384-deep sum (202 us; 22 cut).
 constexpr int kDwSlab = 128;
 template <int KS> constexpr int kDwLds = (64 + 16 * KS) * (kDwSlab + 8);      // 16-bit words
 template <int KS>
@@ -429,56 +425,52 @@ __device__ __forceinline__ void conv_dw_tile(uint16_t *sm, int bx, int by, int b
     const int m0 = by * 64, cb = bx * 16;
     const int kbeg = bz * chunk, kend = min(kbeg + chunk, K);
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int kl = (w & 1) * 64 + lane, cw = cb + (w >> 1) * 8;       // this lane's k of a slab, first channel
-    uint4 fa[4], fx[8];
-    uint16_t f9[8];
+    const int kl = (w & 1) * 64 + lane, cw = cb + (w >> 1) * 2;       // this lane's k of a slab, first channel
+    uint4 fa, fx[2];
+    uint16_t f9[2];
     Taps tp;
     auto fetch = [&](int k0) {
         const int k = min(k0 + kl, K - 1), b = k / q.Lout;
         tp = conv_taps(q, b, k - b * q.Lout);
         if (k0 + kl >= kend) { tp.shift = 8; tp.has9 = false; }       // counts as 0
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < 2; ++j) {
             const uint16_t *p = x + (long long)min(cw + j, q.C - 1) * BL;
             const u32x4u v = *reinterpret_cast<const u32x4u *>(p + tp.first);
             fx[j] = make_uint4(v.x, v.y, v.z, v.w);
             if (KS > 8) f9[j] = p[tp.ninth];
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int j = t + 256 * i;
-            fa[i] = conv_a8(dp, K, q.M, m0 + (j >> 4), k0 + (j & 15) * 8, kend, avec);
-        }
+        fa = conv_a8(dp, K, q.M, m0 + (t >> 4), k0 + (t & 15) * 8, kend, avec);
     };
-    f32x4 acc[KS] = {};
+    constexpr int NJ = (KS + 3) / 4;                   // column tiles w & 3, + 4, + 8 of KS
+    const int wm = 16 * (w >> 2), wj = w & 3;
+    f32x4 acc[NJ] = {};
     fetch(kbeg);
 #pragma unroll 1
     for (int k0 = kbeg; k0 < kend; k0 += SLAB) {
         if (__any(tp.shift != 0 || !tp.has9)) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < 2; ++j) {
                 fx[j] = shift_taps(fx[j], tp.shift);
                 if (!tp.has9) f9[j] = 0;
             }
         }
+        *reinterpret_cast<uint4 *>(&As[(t >> 4) * LD + (t & 15) * 8]) = fa;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int j = t + 256 * i;
-            *reinterpret_cast<uint4 *>(&As[(j >> 4) * LD + (j & 15) * 8]) = fa[i];
-        }
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int k = 0; k < KS; ++k) Bs[(((w >> 1) * 8 + j) * KS + k) * LD + kl] = tap_of(fx[j], f9[j], k);
+            for (int k = 0; k < KS; ++k) Bs[(((w >> 1) * 2 + j) * KS + k) * LD + kl] = tap_of(fx[j], f9[j], k);
         __syncthreads();
         if (k0 + SLAB < kend) fetch(k0 + SLAB);
         const int ko = 8 * (lane >> 4);
-#pragma unroll 1
+#pragma unroll 2
         for (int kk = 0; kk < SLAB; kk += 32) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[(16 * w + (lane & 15)) * LD + kk + ko]);
+            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[(wm + (lane & 15)) * LD + kk + ko]);
 #pragma unroll
-            for (int j = 0; j < KS; ++j) {
-                const bf16x8 v = *reinterpret_cast<const bf16x8 *>(&Bs[(16 * j + (lane & 15)) * LD + kk + ko]);
+            for (int j = 0; j < NJ; ++j) {
+                if (4 * j + wj >= KS) continue;
+                const bf16x8 v =
+                    *reinterpret_cast<const bf16x8 *>(&Bs[(16 * (4 * j + wj) + (lane & 15)) * LD + kk + ko]);
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, v, acc[j], 0, 0, 0);
             }
         }
@@ -486,32 +478,38 @@ __device__ __forceinline__ void conv_dw_tile(uint16_t *sm, int bx, int by, int b
     }
     out += (long long)bz * q.M * N;
 #pragma unroll
-    for (int j = 0; j < KS; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = m0 + 16 * w + 4 * (lane >> 4) + r, col = cb * KS + 16 * j + (lane & 15);
-            if (row < q.M && col < N) out[(long long)row * N + col] = acc[j][r];
+            const int row = m0 + wm + 4 * (lane >> 4) + r, col = cb * KS + 16 * (4 * j + wj) + (lane & 15);
+            if (4 * j + wj < KS && row < q.M && col < N) out[(long long)row * N + col] = acc[j][r];
         }
 }
 
 // The weight gradient's blocks, gx·gy·gz of them, and behind them those of dcol = Wᵀ·dp (its
 // gn tiles along (b, l)): both wait for dp only, and each alone leaves much of the chip
 // idle.  Layers 3, 2, 1 of 64 examples: 8.2 + 5.6, 8.6 + 4.9, 8.8 + 7.8 us apart, 8.4, 8.8
-// and 10.5 together.
+// and 10.5 together, 7.6, 8.0 and 9.3 with 16 waves to a block instead of 4.
+constexpr int kDwThreads = 1024;
 template <int KS>
-__global__ __launch_bounds__(256) void k_conv_back(ConvShape q, const uint16_t *__restrict__ dp,
-                                                   const uint16_t *__restrict__ x, float *__restrict__ out, int chunk,
-                                                   int avec, int gx, int gy, int gz, const uint16_t *__restrict__ W,
-                                                   float *__restrict__ dcol, int gn) {
-    __shared__ __attribute__((aligned(16))) uint16_t sm[kDwLds<KS> > kGemmLds ? kDwLds<KS> : kGemmLds];
+__global__ __launch_bounds__(kDwThreads) void k_conv_back(ConvShape q, const uint16_t *__restrict__ dp,
+                                                          const uint16_t *__restrict__ x, float *__restrict__ out,
+                                                          int chunk, int avec, int gx, int gy, int gz,
+                                                          const uint16_t *__restrict__ W, float *__restrict__ dcol,
+                                                          int gn) {
+    __shared__ __attribute__((aligned(16))) uint16_t sm[kDwLds<KS> > 4 * kGemmLds ? kDwLds<KS> : 4 * kGemmLds];
     int b = blockIdx.x;
     if (b < gx * gy * gz) {
         conv_dw_tile<KS>(sm, b % gx, b / gx % gy, b / (gx * gy), q, dp, x, out, chunk, avec);
         return;
     }
-    b -= gx * gy * gz;
-    const int K = q.C * KS, N = q.B * q.Lout;
-    gemm_tile<false, true>(sm, b / gn * GBM, b % gn * GBN, K, N, q.M, W, K, dp, N, dcol, N, nullptr, nullptr, 0);
+    // four tiles of 256 threads; they walk the same number of slabs, so their barriers agree,
+    // and waves without a tile leave before the first
+    const int K = q.C * KS, N = q.B * q.Lout, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    b = 4 * (b - gx * gy * gz) + g;
+    if (b >= gn * ((K + GBM - 1) / GBM)) return;
+    gemm_tile<false, true>(sm + g * kGemmLds, threadIdx.x & 255, b / gn * GBM, b % gn * GBN, K, N, q.M, W, K, dp, N,
+                           dcol, N, nullptr, nullptr, 0);
 }
 
 // out[i] = Σ_k part[i·si + k·sk] for every sum of the list, in rising k.  One launch for
@@ -1031,20 +1029,21 @@ extern "C" int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float 
     hipStream_t st = (hipStream_t)stream;
     switch (ks) {
 #define EFM_CONV(KS) \
-    case KS: k_conv_fwd<KS><<<grid, 256, 0, st>>>(q, x, W, bias, y, yb, flat, avec); break;
+    case KS: k_conv_fwd<KS><<<grid, kFwdThreads, 0, st>>>(q, x, W, bias, y, yb, flat, avec); break;
         EFM_CONV_SIZES(EFM_CONV)
 #undef EFM_CONV
     }
     return check_launch("efm_net_conv1d");
 }
 
-// Blocks a tile's sum is cut over: up to two blocks for each of the 256 CUs, of at
-// least two slabs each; sums of four slabs or fewer stay whole.
+// Blocks a tile's sum is cut over: about a block for each of the 256 CUs, of at least two
+// slabs each; sums of four slabs or fewer stay whole.  First layer of 64 examples with 256,
+// 512, 768 blocks: 22.2, 23.4, 20.9 us and 4.8, 5.2, 6.0 to add the parts.
 static int dw_splits(const ConvShape &q) {
     const long long tiles = (long long)((q.C + 15) / 16) * ((q.M + 63) / 64);
     const long long slabs = ((long long)q.B * q.Lout + 127) / 128;
     if (slabs <= 4) return 1;
-    long long z = (512 + tiles - 1) / tiles;
+    long long z = (256 + tiles - 1) / tiles;
     if (z > slabs / 2) z = slabs / 2;
     return (int)(z < 1 ? 1 : z > 65535 ? 65535 : z);
 }
@@ -1113,13 +1112,13 @@ extern "C" int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const 
     // dcol rides along where its product may take 16-byte loads
     const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0;
     const int gn = (K + GBN - 1) / GBN;
-    const long long blocks = (long long)gx * gy * gz + (both ? (long long)gn * ((C * ks + GBM - 1) / GBM) : 0);
+    const long long blocks = (long long)gx * gy * gz + (both ? ((long long)gn * ((C * ks + GBM - 1) / GBM) + 3) / 4 : 0);
     NET_CHECK(blocks < (1LL << 24), "efm_net_conv1d_back: too large");
     switch (ks) {
 #define EFM_CONV(KS)                                                                                              \
     case KS:                                                                                                      \
-        k_conv_back<KS><<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(q, dp, x, gz > 1 ? work : dW, chunk,   \
-                                                                           avec, gx, gy, gz, W, dcol, gn);        \
+        k_conv_back<KS><<<(unsigned)blocks, kDwThreads, 0, (hipStream_t)stream>>>(                                \
+            q, dp, x, gz > 1 ? work : dW, chunk, avec, gx, gy, gz, W, dcol, gn);                                  \
         break;
         EFM_CONV_SIZES(EFM_CONV)
 #undef EFM_CONV
