@@ -48,8 +48,8 @@ class EfmShots(ctypes.Structure):
                                         "wavelet", "nt", "rec", "recmask")]
 
 
-class EfmNetSum(ctypes.Structure):
-    _fields_ = [("part", c_void_p), ("out", c_void_p), ("n", c_ll), ("si", c_ll), ("sk", c_ll), ("parts", c_int)]
+class EfmNetBias(ctypes.Structure):
+    _fields_ = [("chains", c_void_p), ("db", c_void_p), ("M", c_int)]
 
 
 P = ctypes.POINTER
@@ -116,16 +116,14 @@ _SIGS = {
     "efm_net_im2col": ([c_void_p, c_void_p] + [c_int] * 6 + [c_void_p], c_int),
     "efm_net_col2im": ([c_void_p, c_void_p] + [c_int] * 6 + [c_void_p], c_int),
     "efm_net_conv1d": ([c_void_p] * 5 + [c_int] * 8 + [c_void_p], c_int),
-    "efm_net_conv1d_work": ([c_int] * 7, c_ll),
-    "efm_net_conv1d_dw": ([c_void_p] * 3 + [c_int] * 7 + [c_void_p] * 2, c_int),
-    "efm_net_relu_bias_backward": ([c_void_p] * 4 + [c_int] * 4 + [c_void_p] * 2, c_int),
-    "efm_net_col2im_relu_bias": ([c_void_p] * 4 + [c_int] * 6 + [c_void_p] * 2, c_int),
     "efm_net_relu_backward": ([c_void_p] * 4 + [c_ll, c_void_p], c_int),
     "efm_net_bias_grad": ([c_void_p, c_void_p, c_int, c_ll, c_void_p], c_int),
-    "efm_net_conv1d_back": ([c_void_p] * 5 + [c_int] * 7 + [c_void_p] * 2, c_int),
-    "efm_net_conv1d_parts": ([c_int] * 7, c_int),
-    "efm_net_row_parts": ([c_int] * 2, c_int),
-    "efm_net_sum": ([P(EfmNetSum), c_int, c_void_p], c_int),
+    "efm_net_conv1d_fits": ([c_int] * 7, c_int),
+    "efm_net_conv1d_back": ([c_void_p] * 5 + [c_int] * 8 + [c_void_p], c_int),
+    "efm_net_relu_bias_backward": ([c_void_p] * 5 + [c_int] * 5 + [c_void_p], c_int),
+    "efm_net_col2im_relu_bias": ([c_void_p] * 5 + [c_int] * 7 + [c_void_p], c_int),
+    "efm_net_bias_split": ([c_int] * 2, c_int),
+    "efm_net_bias_sums": ([P(EfmNetBias), c_int, c_void_p], c_int),
     "efm_net_head_fits": ([c_int] * 4, c_int),
     "efm_net_head_forward": ([c_void_p] * 8 + [c_int] * 4 + [c_void_p], c_int),
     "efm_net_head_backward": ([c_void_p] * 10 + [c_int] * 3 + [c_float, c_void_p], c_int),

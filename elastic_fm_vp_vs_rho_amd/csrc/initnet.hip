@@ -37,6 +37,11 @@ inline int blocks_for(long long n, int bs) {
 // and B[8(l/16)+j][l%16], j < 8, and receives D[4(l/16)+j][l%16], j < 4.
 constexpr int GBM = 64, GBN = 64, GBK = 32, GLD = GBK + 8;
 
+__device__ __forceinline__ f32x4 mfma_1(const uint4 &a, const uint4 &b, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(&a),
+                                                   *reinterpret_cast<const bf16x8 *>(&b), acc, 0, 0, 0);
+}
+
 // The 2 x 2 MFMA tiles of one k-slab from the LDS stages.
 __device__ __forceinline__ void mfma_slab(const uint16_t *As, const uint16_t *Bs, int wm, int wn,
                                           int lane, f32x4 (&acc)[2][2]) {
@@ -407,181 +412,244 @@ __global__ __launch_bounds__(kFwdThreads) void k_conv_fwd(ConvShape q, const uin
     }
 }
 
-// dW[m, c·KS + tap] = Σ_(b, l) dp[m, b·Lout + l]·x[c, b, l·stride + tap - pad].  Block tile
-// 64 rows x 16 channels' taps, slabs of 128 samples: of 16 waves two take each pair of
-// channels, 64 samples each; wave w multiplies rows 16(w/4) .. and every fourth column
-// tile from w mod 4.  The sum over (b, l) is cut over gz blocks of `chunk` samples and
-// k_sums adds the parts in order: a tile to a block left 229 of 256 CUs idle on the
-// first layer's 16384-deep sum (202 us; 22 cut).
-constexpr int kDwSlab = 128;
-template <int KS> constexpr int kDwLds = (64 + 16 * KS) * (kDwSlab + 8);      // 16-bit words
-template <int KS>
-__device__ __forceinline__ void conv_dw_tile(uint16_t *sm, int bx, int by, int bz, const ConvShape &q,
-                                             const uint16_t *__restrict__ dp, const uint16_t *__restrict__ x,
-                                             float *__restrict__ out, int chunk, int avec) {
-    constexpr int SLAB = kDwSlab, LD = SLAB + 8;
-    uint16_t *As = sm, *Bs = sm + 64 * LD;
-    const int N = q.C * KS, K = q.B * q.Lout, BL = q.B * q.L;
-    const int m0 = by * 64, cb = bx * 16;
-    const int kbeg = bz * chunk, kend = min(kbeg + chunk, K);
+// dW[m, c·ks + tap] = Σ_(b, l) dp[m, b·Lout + l]·x[c, b, l·stride + tap - pad].  A block makes
+// 32 rows x 16 channels of one tap in one pass over (b, l), slabs of 256 samples: the sum
+// of an entry stays one accumulator over rising 32-deep MFMA steps, as in the product with
+// the stored matrix, since another order moves the last bit of a gradient, and Adam's
+// first steps turn that into other BF16 weights.  Waves 0 and 1 multiply, a row tile each,
+// with dp straight from memory (no other wave of the block wants it); 4 to 7 put the
+// 16 channels of the next slab into the other of two LDS buffers, a sample to a lane, so
+// that every lane's tap is in the row or not for all channels at once.  Three slabs of loads
+// are in flight.  What binds it is the vector memory path of a CU, which each slab's dp (0.28
+// us) and taps (0.38 us) share: 32 rows a block for 64 (the first layer's chain of 64
+// slabs 92 -> 63 us on 216 CUs), 16 go twice to a CU (101).  Four layers of 64 examples: 97 us
+// against 278 of 64 x 64 tiles over the stored matrix, its im2col not counted.
+constexpr int kDwSlab = 256, kDwLd = kDwSlab + 8, kDwThreads = 512, kDwRows = 32;
+constexpr int kDwLds = 2 * 16 * kDwLd;                // 16-bit words
+template <bool AVEC>
+__device__ __forceinline__ void conv_dw_tile(uint16_t *Bs, int c0, int tap, int m0, const ConvShape &q,
+                                             const uint16_t *__restrict__ dp, int ldp,
+                                             const uint16_t *__restrict__ x, float *__restrict__ out) {
+    constexpr int AHEAD = AVEC ? 3 : 1, NK = kDwSlab / 32;        // slabs of loads in flight
+    const int K = q.B * q.Lout, BL = q.B * q.L;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int kl = (w & 1) * 64 + lane, cw = cb + (w >> 1) * 2;       // this lane's k of a slab, first channel
-    uint4 fa, fx[2];
-    uint16_t f9[2];
-    Taps tp;
-    auto fetch = [&](int k0) {
-        const int k = min(k0 + kl, K - 1), b = k / q.Lout;
-        tp = conv_taps(q, b, k - b * q.Lout);
-        if (k0 + kl >= kend) { tp.shift = 8; tp.has9 = false; }       // counts as 0
+    // slabs, whole rounds of AHEAD: those past the end add nothing, and with no condition on a
+    // load the compiler can wait for the oldest one alone
+    const int nslab = (K + kDwSlab * AHEAD - 1) / (kDwSlab * AHEAD) * AHEAD;
+    if (w >= 4) {
+        const int kl = t - 256;
+        const uint16_t *px[16];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint16_t *p = x + (long long)min(cw + j, q.C - 1) * BL;
-            const u32x4u v = *reinterpret_cast<const u32x4u *>(p + tp.first);
-            fx[j] = make_uint4(v.x, v.y, v.z, v.w);
-            if (KS > 8) f9[j] = p[tp.ninth];
-        }
-        fa = conv_a8(dp, K, q.M, m0 + (t >> 4), k0 + (t & 15) * 8, kend, avec);
-    };
-    constexpr int NJ = (KS + 3) / 4;                   // column tiles w & 3, + 4, + 8 of KS
-    const int wm = 16 * (w >> 2), wj = w & 3;
-    f32x4 acc[NJ] = {};
-    fetch(kbeg);
+        for (int j = 0; j < 16; ++j) px[j] = x + (long long)min(c0 + j, q.C - 1) * BL;
+        uint16_t f[AHEAD][16];
+        bool in[AHEAD];
+        auto fetch = [&](uint16_t (&g)[16], bool &valid, int i) __attribute__((always_inline)) {
+            const int k = min(i, nslab) * kDwSlab + kl, kc = min(k, K - 1), b = kc / q.Lout;
+            const int pos = (kc - b * q.Lout) * q.stride - q.pad + tap;
+            valid = k < K && (unsigned)pos < (unsigned)q.L;
+            const unsigned off = (unsigned)(b * q.L + min(max(pos, 0), q.L - 1));
+#pragma unroll
+            for (int j = 0; j < 16; ++j) g[j] = px[j][off];
+        };
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) fetch(f[d], in[d], d);
 #pragma unroll 1
-    for (int k0 = kbeg; k0 < kend; k0 += SLAB) {
-        if (__any(tp.shift != 0 || !tp.has9)) {
+        for (int i = 0; i < nslab; i += AHEAD)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                fx[j] = shift_taps(fx[j], tp.shift);
-                if (!tp.has9) f9[j] = 0;
+            for (int d = 0; d < AHEAD; ++d) {
+                uint16_t *B = Bs + ((i + d) & 1) * 16 * kDwLd + kl;
+#pragma unroll
+                for (int j = 0; j < 16; ++j) B[j * kDwLd] = in[d] ? f[d][j] : (uint16_t)0;
+                fetch(f[d], in[d], i + d + AHEAD);
+                __syncthreads();
             }
-        }
-        *reinterpret_cast<uint4 *>(&As[(t >> 4) * LD + (t & 15) * 8]) = fa;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int k = 0; k < KS; ++k) Bs[(((w >> 1) * 2 + j) * KS + k) * LD + kl] = tap_of(fx[j], f9[j], k);
-        __syncthreads();
-        if (k0 + SLAB < kend) fetch(k0 + SLAB);
-        const int ko = 8 * (lane >> 4);
-#pragma unroll 2
-        for (int kk = 0; kk < SLAB; kk += 32) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&As[(wm + (lane & 15)) * LD + kk + ko]);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                if (4 * j + wj >= KS) continue;
-                const bf16x8 v =
-                    *reinterpret_cast<const bf16x8 *>(&Bs[(16 * (4 * j + wj) + (lane & 15)) * LD + kk + ko]);
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, v, acc[j], 0, 0, 0);
-            }
-        }
-        __syncthreads();
-    }
-    out += (long long)bz * q.M * N;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = m0 + wm + 4 * (lane >> 4) + r, col = cb * KS + 16 * (4 * j + wj) + (lane & 15);
-            if (4 * j + wj < KS && row < q.M && col < N) out[(long long)row * N + col] = acc[j][r];
-        }
-}
-
-// The weight gradient's blocks, gx·gy·gz of them, and behind them those of dcol = Wᵀ·dp (its
-// gn tiles along (b, l)): both wait for dp only, and each alone leaves much of the chip
-// idle.  Layers 3, 2, 1 of 64 examples: 8.2 + 5.6, 8.6 + 4.9, 8.8 + 7.8 us apart, 8.4, 8.8
-// and 10.5 together, 7.6, 8.0 and 9.3 with 16 waves to a block instead of 4.
-constexpr int kDwThreads = 1024;
-template <int KS>
-__global__ __launch_bounds__(kDwThreads) void k_conv_back(ConvShape q, const uint16_t *__restrict__ dp,
-                                                          const uint16_t *__restrict__ x, float *__restrict__ out,
-                                                          int chunk, int avec, int gx, int gy, int gz,
-                                                          const uint16_t *__restrict__ W, float *__restrict__ dcol,
-                                                          int gn) {
-    __shared__ __attribute__((aligned(16))) uint16_t sm[kDwLds<KS> > 4 * kGemmLds ? kDwLds<KS> : 4 * kGemmLds];
-    int b = blockIdx.x;
-    if (b < gx * gy * gz) {
-        conv_dw_tile<KS>(sm, b % gx, b / gx % gy, b / (gx * gy), q, dp, x, out, chunk, avec);
         return;
     }
-    // four tiles of 256 threads; they walk the same number of slabs, so their barriers agree,
+    if (w >= kDwRows / 16) return;
+    const int row = m0 + 16 * w + (lane & 15), ko = 8 * (lane >> 4);
+    const uint16_t *rowp = dp + (long long)min(row, q.M - 1) * ldp;      // rows past M: sums nobody stores
+    uint4 a[AHEAD][NK];
+    auto load = [&](uint4 (&g)[NK], int i) __attribute__((always_inline)) {
+        const int k0 = min(i, nslab) * kDwSlab + ko;
+        if (AVEC) {          // rows of whole vectors: in range or past the end as one
+#pragma unroll
+            for (int k = 0; k < NK; ++k) g[k] = *reinterpret_cast<const uint4 *>(rowp + min(k0 + 32 * k, K - 8));
+        } else {
+#pragma unroll
+            for (int k = 0; k < NK; ++k) g[k] = conv_a8(rowp, K, 1, 0, k0 + 32 * k, K, false);
+        }
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) load(a[d], d);
+#pragma unroll 1
+    for (int i = 0; i < nslab; i += AHEAD)
+#pragma unroll
+        for (int d = 0; d < AHEAD; ++d) {
+            __syncthreads();
+            const uint16_t *B = Bs + ((i + d) & 1) * 16 * kDwLd + (lane & 15) * kDwLd + ko;
+            uint4 v[NK];
+#pragma unroll
+            for (int k = 0; k < NK; ++k) v[k] = *reinterpret_cast<const uint4 *>(B + 32 * k);
+            if (AVEC && (i + d + 1) * kDwSlab > K) {
+#pragma unroll
+                for (int k = 0; k < NK; ++k)
+                    if ((i + d) * kDwSlab + 32 * k + ko >= K) a[d][k] = make_uint4(0, 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);        // all reads before the first product
+#pragma unroll
+            for (int k = 0; k < NK; ++k) acc = mfma_1(a[d][k], v[k], acc);
+            load(a[d], i + d + AHEAD);
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int m = m0 + 16 * w + 4 * (lane >> 4) + r, c = c0 + (lane & 15);
+        if (m < q.M && c < q.C) out[((long long)m * q.C + c) * q.ks + tap] = acc[r];
+    }
+}
+
+// The weight gradient's blocks, dw_blocks of them, and behind them those of dcol = Wᵀ·dp
+// (its gn tiles along (b, l)): both wait for dp only, and each alone leaves much of the chip
+// idle.  Row tiles and taps of 16 channels follow one another on an XCD, whose L2 then holds
+// those channels.
+__host__ __device__ inline int dw_rows(const ConvShape &q) { return (q.M + kDwRows - 1) / kDwRows; }
+__host__ __device__ inline int dw_tiles(const ConvShape &q) { return (q.C + 15) / 16 * q.ks * dw_rows(q); }
+template <bool AVEC>
+__global__ __launch_bounds__(kDwThreads) void k_conv_back(ConvShape q, const uint16_t *__restrict__ dp, int ldp,
+                                                          const uint16_t *__restrict__ x, float *__restrict__ dW,
+                                                          int dw_blocks, const uint16_t *__restrict__ W,
+                                                          float *__restrict__ dcol, int gn) {
+    __shared__ __attribute__((aligned(16))) uint16_t sm[kDwLds > 2 * kGemmLds ? kDwLds : 2 * kGemmLds];
+    int b = blockIdx.x;
+    if (b < dw_blocks) {
+        const int tile = b % 8 * (dw_blocks / 8) + b / 8, rows = dw_rows(q);
+        if (tile < dw_tiles(q))
+            conv_dw_tile<AVEC>(sm, tile / (rows * q.ks) * 16, tile / rows % q.ks, tile % rows * kDwRows, q, dp, ldp, x,
+                               dW);
+        return;
+    }
+    // two tiles of 256 threads; they walk the same number of slabs, so their barriers agree,
     // and waves without a tile leave before the first
-    const int K = q.C * KS, N = q.B * q.Lout, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-    b = 4 * (b - gx * gy * gz) + g;
+    const int K = q.C * q.ks, N = q.B * q.Lout, g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    b = 2 * (b - dw_blocks) + g;
     if (b >= gn * ((K + GBM - 1) / GBM)) return;
-    gemm_tile<false, true>(sm + g * kGemmLds, threadIdx.x & 255, b / gn * GBM, b % gn * GBN, K, N, q.M, W, K, dp, N,
+    gemm_tile<false, true>(sm + g * kGemmLds, threadIdx.x & 255, b / gn * GBM, b % gn * GBN, K, N, q.M, W, K, dp, ldp,
                            dcol, N, nullptr, nullptr, 0);
 }
 
-// out[i] = Σ_k part[i·si + k·sk] for every sum of the list, in rising k.  One launch for
-// all the cut sums of a backward pass (5.2 us against 4.1 for each of five).
-struct SumList {
-    EfmNetSum s[EFM_NET_SUMS];
-    int first[EFM_NET_SUMS];        // its first block of 256 outputs
-    int n;
-};
-__global__ __launch_bounds__(256) void k_sums(SumList l) {
-    int j = 0;
-    while (j + 1 < l.n && (int)blockIdx.x >= l.first[j + 1]) ++j;
-    const EfmNetSum &s = l.s[j];
-    const long long i = (long long)(blockIdx.x - l.first[j]) * 256 + threadIdx.x;
-    if (i >= s.n) return;
-    const float *p = s.part + i * s.si;
-    float v = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < s.parts; ++k) v += p[k * s.sk];
-    s.out[i] = v;
-}
-
 // ---- ReLU backward with the bias gradient --------------------------------------------
-// Row m = blockIdx.x of dp = dy·(y > 0), in gridDim.y blocks; sums[m·gridDim.y + blockIdx.y]
-// = the block's sum (db itself for one block a row).  `value(m, n)` gives dy.
-template <typename F>
-__device__ __forceinline__ void relu_bias_row(const float *__restrict__ y, uint16_t *__restrict__ dpb,
-                                              float *__restrict__ sums, int N, F value) {
-    __shared__ float red[256];
-    const int m = blockIdx.x, chunk = (N + gridDim.y - 1) / gridDim.y;
-    const int n0 = blockIdx.y * chunk, n1 = min(n0 + chunk, N);
-    const long long row = (long long)m * N;
-    float s = 0.f;
-#pragma unroll 4
-    for (int n = n0 + threadIdx.x; n < n1; n += 256) {
-        const float d = value(m, n);
-        const float v = y[row + n] > 0.f ? d : 0.f;
-        dpb[row + n] = f2bf(v);
-        s += v;
-    }
-    red[threadIdx.x] = s;
+// A bias gradient is 256 chains (chain i: the row's values i, i + 256, ... in rising order)
+// and a tree over them; the order is kept whatever computes it (see conv_dw_tile).
+__device__ __forceinline__ float tree256(float *red, float v) {
+    red[threadIdx.x] = v;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) sums[m * gridDim.y + blockIdx.y] = red[0];
+    return red[0];
+}
+
+// dp = dy·(y > 0) of row m = blockIdx.x; `value(m, n)` gives dy.  One block to a row
+// (chains null): db[m].  Else gridDim.y = 16 blocks to a row, kChains chains each: their sums
+// to chains[256·m ..], added up by k_bias_sums.  64 rows of 16384 / 4096 values through
+// col2im: 30 / 25 us in one block a row, 10.8 / 7.4 in blocks of 16 chains (14.9 / 9.4 of
+// 32, 23.7 / 14.2 of 64).
+constexpr int kChains = 16;
+template <typename F>
+__device__ __forceinline__ void relu_bias_row(const float *__restrict__ y, uint16_t *__restrict__ dpb,
+                                              float *__restrict__ db, float *__restrict__ chains, int N, int ldp,
+                                              F value) {
+    const int m = blockIdx.x, t = threadIdx.x;
+    const long long row = (long long)m * N;
+    dpb += (long long)m * ldp;
+    if (!chains) {
+        __shared__ float red[256];
+        float s = 0.f;
+#pragma unroll 4
+        for (int n = t; n < N; n += 256) {
+            const float d = value(m, n);
+            const float v = y[row + n] > 0.f ? d : 0.f;
+            dpb[n] = f2bf(v);
+            s += v;
+        }
+        s = tree256(red, s);
+        if (t == 0) db[m] = s;
+        return;
+    }
+    __shared__ float v[64][kChains + 1];    // 64 values of each of the block's chains
+    const int i = t % kChains, c = kChains * blockIdx.y + i;
+    float s = 0.f;
+    for (long long n0 = 0; n0 < N; n0 += 64 * 256) {
+#pragma unroll
+        for (int jj = 0; jj < kChains / 4; ++jj) {
+            const int j = t / kChains + 256 / kChains * jj;
+            const long long n = n0 + 256 * j + c;
+            const int nc = (int)(n < N ? n : N - 1);         // past the end: computed, not kept
+            const float d = value(m, nc);
+            const float p = y[row + nc] > 0.f ? d : 0.f;
+            v[j][i] = p;
+            if (n < N) dpb[n] = f2bf(p);
+        }
+        __syncthreads();
+        if (t < kChains)
+#pragma unroll 8
+            for (int j = 0; j < 64; ++j)
+                if (n0 + 256 * j + c < N) s += v[j][i];
+        __syncthreads();
+    }
+    if (t < kChains) chains[256LL * m + c] = s;
+}
+
+// db[m] from the chains of rows m < M, for every bias of the list.
+struct BiasList {
+    EfmNetBias s[EFM_NET_BIASES];
+    int first[EFM_NET_BIASES];        // its first block, a row each
+    int n;
+};
+__global__ __launch_bounds__(256) void k_bias_sums(BiasList l) {
+    __shared__ float red[256];
+    int j = 0;
+    while (j + 1 < l.n && (int)blockIdx.x >= l.first[j + 1]) ++j;
+    const int m = blockIdx.x - l.first[j];
+    const float s = tree256(red, l.s[j].chains[256LL * m + threadIdx.x]);
+    if (threadIdx.x == 0) l.s[j].db[m] = s;
 }
 
 // dy (M, N) row-major, or flattened (dy[(m·L + l)·B + b] for n = b·L + l) when L > 0.
 __global__ __launch_bounds__(256) void k_relu_bias(const float *__restrict__ dy, const float *__restrict__ y,
-                                                   uint16_t *__restrict__ dpb, float *__restrict__ sums, int N,
-                                                   int B, int L) {
-    relu_bias_row(y, dpb, sums, N, [&](int m, int n) {
+                                                   uint16_t *__restrict__ dpb, float *__restrict__ db,
+                                                   float *__restrict__ chains, int N, int B, int L, int ldp) {
+    relu_bias_row(y, dpb, db, chains, N, ldp, [&](int m, int n) {
         if (L <= 0) return dy[(long long)m * N + n];
         const int b = n / L, l = n - b * L;
         return dy[((long long)m * L + l) * B + b];
     });
 }
 
-// dy = the transposed im2col of dcol (see k_col2im) at channel c, n = b·L + j.
+// dy = the transposed im2col of dcol (see k_col2im) at channel c, n = b·L + j: the taps with
+// j + pad - k a multiple of the stride, in rising k, at most T of them (0: any number).
+template <int T>
 __global__ __launch_bounds__(256) void k_col2im_relu_bias(const float *__restrict__ dcol, const float *__restrict__ y,
-                                                          uint16_t *__restrict__ dpb, float *__restrict__ sums,
-                                                          ConvShape q) {
-    const int ncol = q.B * q.Lout;
-    relu_bias_row(y, dpb, sums, q.B * q.L, [&](int c, int n) {
-        const int b = n / q.L, j = n - b * q.L;
+                                                          uint16_t *__restrict__ dpb, float *__restrict__ db,
+                                                          float *__restrict__ chains, ConvShape q, int ldp) {
+    const unsigned ncol = q.B * q.Lout, L = q.L, stride = q.stride;
+    relu_bias_row(y, dpb, db, chains, q.B * q.L, ldp, [&](int c, int n) __attribute__((always_inline)) {
+        const unsigned b = (unsigned)n / L, j = n - b * L + q.pad;
+        int l = j / stride, k = j - l * stride;
+        const float *col = dcol + (long long)c * q.ks * ncol + b * q.Lout;
         float s = 0.f;
-        // taps with (j + pad - k) a multiple of the stride, in rising k
-        int k = (j + q.pad) % q.stride, l = (j + q.pad) / q.stride;
-        for (; k < q.ks && l >= 0; k += q.stride, --l)
-            if (l < q.Lout) s += dcol[(long long)(c * q.ks + k) * ncol + b * q.Lout + l];
+        if (T == 0) {
+            for (; k < q.ks && l >= 0; k += stride, --l)
+                if (l < q.Lout) s += col[(long long)k * ncol + l];
+            return s;
+        }
+        // every tap loaded from a place inside the row, counted if it is its own
+#pragma unroll
+        for (int i = 0; i < T; ++i, k += stride, --l) {
+            const float v = col[(long long)min(k, q.ks - 1) * ncol + min(max(l, 0), q.Lout - 1)];
+            s += k < q.ks && (unsigned)l < (unsigned)q.Lout ? v : 0.f;
+        }
         return s;
     });
 }
@@ -593,10 +661,6 @@ __global__ __launch_bounds__(256) void k_col2im_relu_bias(const float *__restric
 // its waves 16 rows each, eight slabs of a row's sum in flight at once: 8.5 us; and one
 // block takes the loss and the last layer back to the hidden layer: 10.3 us in place of six
 // launches (25 us).  MFMA steps of 32 k in rising order, as the general product's.
-__device__ __forceinline__ f32x4 mfma_1(const uint4 &a, const uint4 &b, f32x4 acc) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8 *>(&a),
-                                                   *reinterpret_cast<const bf16x8 *>(&b), acc, 0, 0, 0);
-}
 __host__ __device__ constexpr int up32(int n) { return (n + 31) & ~31; }
 
 __global__ __launch_bounds__(512) void k_head_fwd(int B, int flat, int hidden, int nout,
@@ -712,25 +776,28 @@ __global__ __launch_bounds__(512) void k_head_bwd(int B, int hidden, int nout, f
         for (int u = 0; u < 8; ++u)
             e[u] = ko + u < nout && r0 + i < hidden ? F2[(ko + u) * hidden + r0 + i] : (uint16_t)0;
         const uint4 a = pack8(e);
-        float sum[4] = {0.f, 0.f, 0.f, 0.f};
-        for (int n0 = 0; n0 < B; n0 += 16) {
-            const f32x4 dz = mfma_1(a, *reinterpret_cast<const uint4 *>(&Dn[(n0 + i) * LN + ko]),
-                                    f32x4{0.f, 0.f, 0.f, 0.f});
+        float p[kHeadB / 16][4];
+#pragma unroll
+        for (int j = 0; j < kHeadB / 16; ++j) {
+            const int n = 16 * j + i;
+            f32x4 dz = {0.f, 0.f, 0.f, 0.f};
+            if (16 * j < B) dz = mfma_1(a, *reinterpret_cast<const uint4 *>(&Dn[n * LN + ko]), dz);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = r0 + 4 * (lane >> 4) + r;
-                if (row >= hidden || n0 + i >= B) continue;
-                const int p = row * B + n0 + i;
-                const float v = z[p] > 0.f ? dz[r] : 0.f;
-                dzpb[p] = f2bf(v);
-                sum[r] += v;
+                const int row = r0 + 4 * (lane >> 4) + r, at = row * B + n;
+                p[j][r] = 0.f;
+                if (row >= hidden || n >= B) continue;
+                p[j][r] = z[at] > 0.f ? dz[r] : 0.f;
+                dzpb[at] = f2bf(p[j][r]);
             }
         }
+        // the bias gradient's tree over examples: 64 apart, 32, 16, then within the 16 lanes
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            for (int d = 8; d > 0; d >>= 1) sum[r] += __shfl_xor(sum[r], d);
+            float v = ((p[0][r] + p[4][r]) + (p[2][r] + p[6][r])) + ((p[1][r] + p[5][r]) + (p[3][r] + p[7][r]));
+            for (int d = 8; d > 0; d >>= 1) v += __shfl_xor(v, d);
             const int row = r0 + 4 * (lane >> 4) + r;
-            if (i == 0 && row < hidden) dc1[row] = sum[r];
+            if (i == 0 && row < hidden) dc1[row] = v;
         }
     }
 }
@@ -1036,135 +1103,73 @@ extern "C" int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float 
     return check_launch("efm_net_conv1d");
 }
 
-// Blocks a tile's sum is cut over: about a block for each of the 256 CUs, of at least two
-// slabs each; sums of four slabs or fewer stay whole.  First layer of 64 examples with 256,
-// 512, 768 blocks: 22.2, 23.4, 20.9 us and 4.8, 5.2, 6.0 to add the parts.
-static int dw_splits(const ConvShape &q) {
-    const long long tiles = (long long)((q.C + 15) / 16) * ((q.M + 63) / 64);
-    const long long slabs = ((long long)q.B * q.Lout + 127) / 128;
-    if (slabs <= 4) return 1;
-    long long z = (256 + tiles - 1) / tiles;
-    if (z > slabs / 2) z = slabs / 2;
-    return (int)(z < 1 ? 1 : z > 65535 ? 65535 : z);
-}
-
-// Blocks a row of N values is cut over: two values to a thread, at most kRowParts blocks
-// in all.  A row to a block leaves 192 of the 256 CUs idle in dependent loads: 64 rows of
-// 16384 / 4096 values 30 / 25 us, cut 7.5 / 5.6 and a share of the launch that adds parts.
-static constexpr int kRowParts = 2048;
-static int row_blocks(int M, long long N) {
-    const long long b = N / 512 < kRowParts / M ? N / 512 : kRowParts / M;
-    return b < 4 ? 1 : (int)b;
-}
-
-extern "C" long long efm_net_conv1d_work(int C, int B, int L, int M, int ks, int stride, int pad) {
+extern "C" int efm_net_conv1d_fits(int C, int B, int L, int M, int ks, int stride, int pad) {
     ConvShape q;
-    if (!conv_shape(q, C, B, L, M, ks, stride, pad)) return -1;
-    const int z = dw_splits(q);
-    const long long dw = z > 1 ? (long long)z * M * C * ks : 0;
-    return dw > kRowParts ? dw : kRowParts;
+    return conv_shape(q, C, B, L, M, ks, stride, pad);
 }
 
-// The launch of the weight gradient: samples to a block and blocks along the sum.
-static void dw_cut(const ConvShape &q, int &chunk, int &z) {
-    const int K = q.B * q.Lout, want = dw_splits(q);
-    chunk = ((K + want - 1) / want + kDwSlab - 1) / kDwSlab * kDwSlab;
-    z = (K + chunk - 1) / chunk;
+extern "C" int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const uint16_t *W, float *dW, float *dcol,
+                                   int C, int B, int L, int M, int ks, int stride, int pad, int ldp, void *stream) {
+    ConvShape q;
+    NET_CHECK(dp && x && dW && (W || !dcol) && conv_shape(q, C, B, L, M, ks, stride, pad) && ldp >= B * q.Lout,
+              "efm_net_conv1d_back: bad arguments");
+    const int K = B * q.Lout, gn = (K + GBN - 1) / GBN;
+    const bool avec = K % 8 == 0 && ldp % 8 == 0 && (uintptr_t)dp % 16 == 0;
+    // dcol rides along where its product may take 16-byte loads
+    const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0;
+    const long long tiles = (C + 15LL) / 16 * ks * ((M + kDwRows - 1) / kDwRows), dw = (tiles + 7) / 8 * 8;
+    const long long blocks = dw + (both ? ((long long)gn * ((C * ks + GBM - 1) / GBM) + 1) / 2 : 0);
+    NET_CHECK(blocks < (1LL << 22), "efm_net_conv1d_back: too large");
+    (avec ? k_conv_back<true> : k_conv_back<false>)<<<(unsigned)blocks, kDwThreads, 0, (hipStream_t)stream>>>(
+        q, dp, ldp, x, dW, (int)dw, W, dcol, gn);
+    if (int rc = check_launch("efm_net_conv1d_back")) return rc;
+    if (!dcol || both) return EFM_OK;
+    return efm_net_gemm(C * ks, K, M, W, 1, C * ks, dp, ldp, 1, dcol, K, nullptr, nullptr, 0, stream);
 }
 
-extern "C" int efm_net_sum(const EfmNetSum *sums, int n, void *stream) {
-    NET_CHECK(n >= 0 && (sums || n == 0), "efm_net_sum: bad arguments");
-    for (int j0 = 0; j0 < n; j0 += EFM_NET_SUMS) {
-        SumList l{};
+// Rows of at least 1024 values, fewer of them than fill the chip a block to a row.
+extern "C" int efm_net_bias_split(int M, int N) { return M <= 512 && N >= 1024; }
+
+extern "C" int efm_net_bias_sums(const EfmNetBias *biases, int n, void *stream) {
+    NET_CHECK(n >= 0 && (biases || n == 0), "efm_net_bias_sums: bad arguments");
+    for (int j0 = 0; j0 < n; j0 += EFM_NET_BIASES) {
+        BiasList l{};
         long long blocks = 0;
-        for (; l.n < EFM_NET_SUMS && j0 + l.n < n; ++l.n) {
-            const EfmNetSum &s = sums[j0 + l.n];
-            NET_CHECK(s.part && s.out && s.n > 0 && s.parts > 0, "efm_net_sum: bad sum");
+        for (; l.n < EFM_NET_BIASES && j0 + l.n < n; ++l.n) {
+            const EfmNetBias &s = biases[j0 + l.n];
+            NET_CHECK(s.chains && s.db && s.M > 0, "efm_net_bias_sums: bad bias");
             l.s[l.n] = s;
             l.first[l.n] = (int)blocks;
-            blocks += (s.n + 255) / 256;
-            NET_CHECK(blocks < (1LL << 24), "efm_net_sum: too many outputs");
+            blocks += s.M;
+            NET_CHECK(blocks < (1LL << 22), "efm_net_bias_sums: too many rows");
         }
-        k_sums<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(l);
-        if (int rc = check_launch("efm_net_sum")) return rc;
+        k_bias_sums<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(l);
+        if (int rc = check_launch("efm_net_bias_sums")) return rc;
     }
     return EFM_OK;
 }
 
-extern "C" int efm_net_conv1d_parts(int C, int B, int L, int M, int ks, int stride, int pad) {
-    ConvShape q;
-    if (!conv_shape(q, C, B, L, M, ks, stride, pad)) return -1;
-    int chunk, z;
-    dw_cut(q, chunk, z);
-    return z;
-}
-
-extern "C" int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const uint16_t *W, float *dW, float *dcol,
-                                   int C, int B, int L, int M, int ks, int stride, int pad, float *work,
-                                   void *stream) {
-    ConvShape q;
-    NET_CHECK(dp && x && dW && work && (W || !dcol) && conv_shape(q, C, B, L, M, ks, stride, pad),
-              "efm_net_conv1d_back: bad arguments");
-    int chunk, gz;
-    dw_cut(q, chunk, gz);
-    const int K = B * q.Lout, gx = (C + 15) / 16, gy = (M + 63) / 64;
-    const int avec = K % 8 == 0 && (uintptr_t)dp % 16 == 0;
-    // dcol rides along where its product may take 16-byte loads
-    const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0;
-    const int gn = (K + GBN - 1) / GBN;
-    const long long blocks = (long long)gx * gy * gz + (both ? ((long long)gn * ((C * ks + GBM - 1) / GBM) + 3) / 4 : 0);
-    NET_CHECK(blocks < (1LL << 24), "efm_net_conv1d_back: too large");
-    switch (ks) {
-#define EFM_CONV(KS)                                                                                              \
-    case KS:                                                                                                      \
-        k_conv_back<KS><<<(unsigned)blocks, kDwThreads, 0, (hipStream_t)stream>>>(                                \
-            q, dp, x, gz > 1 ? work : dW, chunk, avec, gx, gy, gz, W, dcol, gn);                                  \
-        break;
-        EFM_CONV_SIZES(EFM_CONV)
-#undef EFM_CONV
-    }
-    if (int rc = check_launch("efm_net_conv1d_back")) return rc;
-    if (!dcol || both) return EFM_OK;
-    return efm_net_gemm(C * ks, K, M, W, 1, C * ks, dp, K, 1, dcol, K, nullptr, nullptr, 0, stream);
-}
-
-extern "C" int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M, int ks,
-                                 int stride, int pad, float *work, void *stream) {
-    if (int rc = efm_net_conv1d_back(dp, x, nullptr, dW, nullptr, C, B, L, M, ks, stride, pad, work, stream)) return rc;
-    const int z = efm_net_conv1d_parts(C, B, L, M, ks, stride, pad);
-    if (z == 1) return EFM_OK;
-    const long long n = (long long)M * C * ks;
-    const EfmNetSum sum{work, dW, n, 1, n, z};
-    return efm_net_sum(&sum, 1, stream);
-}
-
-extern "C" int efm_net_row_parts(int M, int N) { return M > 0 && N > 0 ? row_blocks(M, N) : -1; }
-
-static int sum_rows(const float *work, float *db, int M, int nb, void *stream) {
-    if (!db || nb == 1) return EFM_OK;
-    const EfmNetSum sum{work, db, M, nb, 1, nb};
-    return efm_net_sum(&sum, 1, stream);
-}
-
-extern "C" int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, int M, int N, int B,
-                                          int L, float *work, void *stream) {
-    NET_CHECK(dy && y && dpb && work && M > 0 && N > 0 && (L <= 0 || (B > 0 && (long long)B * L == N)),
+extern "C" int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, float *chains,
+                                          int M, int N, int B, int L, int ldp, void *stream) {
+    NET_CHECK(dy && y && dpb && (db || chains) && M > 0 && N > 0 && ldp >= N && (L <= 0 || (B > 0 && (long long)B * L == N)),
               "efm_net_relu_bias_backward: bad arguments");
-    const int nb = row_blocks(M, N);
-    k_relu_bias<<<dim3(M, nb), 256, 0, (hipStream_t)stream>>>(dy, y, dpb, db && nb == 1 ? db : work, N, B, L);
-    if (int rc = check_launch("efm_net_relu_bias_backward")) return rc;
-    return sum_rows(work, db, M, nb, stream);
+    k_relu_bias<<<dim3(M, chains ? 256 / kChains : 1), 256, 0, (hipStream_t)stream>>>(dy, y, dpb, db, chains, N, B, L, ldp);
+    return check_launch("efm_net_relu_bias_backward");
 }
 
-extern "C" int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C, int B, int L,
-                                        int ks, int stride, int pad, float *work, void *stream) {
-    NET_CHECK(dcol && y && dpb && work && conv_ok(C, B, L, ks, stride, pad) && (long long)B * L < (1LL << 31),
+extern "C" int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, float *chains,
+                                        int C, int B, int L, int ks, int stride, int pad, int ldp, void *stream) {
+    NET_CHECK(dcol && y && dpb && (db || chains) && conv_ok(C, B, L, ks, stride, pad) &&
+                  (long long)B * L < (1LL << 31) && ldp >= B * L,
               "efm_net_col2im_relu_bias: bad arguments");
     const ConvShape q{C, B, L, 1, ks, stride, pad, (L + 2 * pad - ks) / stride + 1};
-    const int nb = row_blocks(C, (long long)B * L);
-    k_col2im_relu_bias<<<dim3(C, nb), 256, 0, (hipStream_t)stream>>>(dcol, y, dpb, db && nb == 1 ? db : work, q);
-    if (int rc = check_launch("efm_net_col2im_relu_bias")) return rc;
-    return sum_rows(work, db, C, nb, stream);
+    const int taps = (ks + stride - 1) / stride;
+    const auto kernel = taps == 1   ? k_col2im_relu_bias<1>
+                        : taps == 2 ? k_col2im_relu_bias<2>
+                        : taps == 3 ? k_col2im_relu_bias<3>
+                                    : k_col2im_relu_bias<0>;
+    kernel<<<dim3(C, chains ? 256 / kChains : 1), 256, 0, (hipStream_t)stream>>>(dcol, y, dpb, db, chains, q, ldp);
+    return check_launch("efm_net_col2im_relu_bias");
 }
 
 // 16 examples' inputs and hidden values in 64 KB of LDS.

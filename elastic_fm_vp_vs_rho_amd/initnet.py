@@ -148,33 +148,24 @@ class InitNet:
             return b
         s, dev = self.spec, self.dev
         b = {"x": _bf((s.cin, B, s.length), dev)}
-        convs, sums = s.convs(), []
-
-        def add(parts, n, si, sk, out):
-            """A buffer for the parts of sums that one launch adds at the backward's end."""
-            t = _f((parts * n,), dev)
-            sums.append(_capi.EfmNetSum(_ptr(t), _ptr(out), n, si, sk, parts))
-            return t
-
+        convs, biases = s.convs(), []
         for i, (ci, co, L, lo) in enumerate(convs):
             b[f"y{i}"] = _f((co, B * lo), dev)
             if i < len(convs) - 1:               # the last block writes its output flattened (X)
                 b[f"yb{i}"] = _bf((co, B * lo), dev)
-            b[f"dpb{i}"] = _bf((co, B * lo), dev)
+            # rows a cache line apart from a power of two: the weight gradient reads all of
+            # them at one offset, which would fall to one channel of the L2
+            b[f"dpb{i}"] = _bf((co, -(-B * lo // 8) * 8 + 64), dev)
             if i > 0:
                 b[f"dcol{i}"] = _f((ci * s.ks, B * lo), dev)
-            conv = (ci, B, L, co, s.ks, s.stride, s.pad)
-            parts = self.L.efm_net_conv1d_parts(*conv)
-            if parts < 0:        # more than 9 taps or short rows: im2col matrix and GEMM
+            if not self.L.efm_net_conv1d_fits(ci, B, L, co, s.ks, s.stride, s.pad):
+                # more than 9 taps or short rows: im2col matrix and GEMM
                 b[f"col{i}"] = _bf((ci * s.ks, B * lo), dev)
                 b["yb_last"] = _bf((co, B * lo), dev)
-            elif parts > 1:
-                b[f"work{i}"] = add(parts, co * ci * s.ks, 1, co * ci * s.ks, self.g[f"W{i}"])
-            rows = self.L.efm_net_row_parts(co, B * lo)
-            if rows > 1:
-                b[f"rows{i}"] = add(rows, co, rows, 1, self.g[f"b{i}"])
-        b["work"] = _f((max(2048, *self.spec.convs()[0][:2], s.hidden),), dev)
-        b["sums"] = (_capi.EfmNetSum * len(sums))(*sums)
+            if self.L.efm_net_bias_split(co, B * lo):
+                b[f"chains{i}"] = _f((co, 256), dev)
+                biases.append(_capi.EfmNetBias(_ptr(b[f"chains{i}"]), _ptr(self.g[f"b{i}"]), co))
+        b["biases"] = (_capi.EfmNetBias * len(biases))(*biases)
         b["head"] = self.L.efm_net_head_fits(B, s.flat, s.hidden, s.nout)
         b["X"] = _bf((s.flat, B), dev)
         b["z"] = _f((s.hidden, B), dev)
@@ -240,9 +231,8 @@ class InitNet:
         self._c(L.efm_net_bias_grad(_ptr(b["dout"]), _ptr(self.g["c2"]), s.nout, B, _stream()),
                 "efm_net_bias_grad")
         self._gemm(s.hidden, B, s.nout, self.wb["F2"], 1, s.hidden, b["doutb"], B, 1, b["dz"], B)
-        self._c(L.efm_net_relu_bias_backward(_ptr(b["dz"]), _ptr(b["z"]), _ptr(b["dzpb"]), _ptr(self.g["c1"]),
-                                             s.hidden, B, 0, 0, _ptr(b["work"]), _stream()),
-                "efm_net_relu_bias_backward")
+        self._c(L.efm_net_relu_bias_backward(_ptr(b["dz"]), _ptr(b["z"]), _ptr(b["dzpb"]), _ptr(self.g["c1"]), None,
+                                             s.hidden, B, 0, 0, B, _stream()), "efm_net_relu_bias_backward")
 
     def backward_buffers(self, B):
         """MSE loss against the buffer ``t`` and every parameter gradient into self.g.
@@ -261,32 +251,28 @@ class InitNet:
         convs, conv = s.convs(), (s.ks, s.stride, s.pad)
         last = len(convs) - 1
         co, lo = convs[last][1], convs[last][3]
-        def rows(i):
-            """Where layer i's bias gradient goes: (db, work) of the ReLU backward."""
-            return (None, _ptr(b[f"rows{i}"])) if f"rows{i}" in b else (_ptr(self.g[f"b{i}"]), _ptr(b["work"]))
-
-        db, work = rows(last)
-        self._c(L.efm_net_relu_bias_backward(_ptr(b["dX"]), _ptr(b[f"y{last}"]), _ptr(b[f"dpb{last}"]), db, co, B * lo,
-                                             B, lo, work, _stream()), "efm_net_relu_bias_backward")
+        self._c(L.efm_net_relu_bias_backward(_ptr(b["dX"]), _ptr(b[f"y{last}"]), _ptr(b[f"dpb{last}"]),
+                                             _ptr(self.g[f"b{last}"]), _ptr(b.get(f"chains{last}")), co, B * lo, B, lo,
+                                             b[f"dpb{last}"].stride(0), _stream()), "efm_net_relu_bias_backward")
         for i in range(last, -1, -1):
             ci, co, Lin, lo = convs[i]
-            N, K = B * lo, ci * s.ks
+            N, K, ldp = B * lo, ci * s.ks, b[f"dpb{i}"].stride(0)
             h = b["x"] if i == 0 else b[f"yb{i - 1}"]
             # dW, and dcol = Wᵀ · dpre_b, whose transposed im2col is the previous layer's dy
             if f"col{i}" in b:
-                self._gemm(co, K, N, b[f"dpb{i}"], N, 1, b[f"col{i}"], 1, N, self.g[f"W{i}"], K)
+                self._gemm(co, K, N, b[f"dpb{i}"], ldp, 1, b[f"col{i}"], 1, N, self.g[f"W{i}"], K)
                 if i > 0:
-                    self._gemm(K, N, co, self.wb[f"W{i}"], 1, K, b[f"dpb{i}"], N, 1, b[f"dcol{i}"], N)
+                    self._gemm(K, N, co, self.wb[f"W{i}"], 1, K, b[f"dpb{i}"], ldp, 1, b[f"dcol{i}"], N)
             else:
                 self._c(L.efm_net_conv1d_back(_ptr(b[f"dpb{i}"]), _ptr(h), _ptr(self.wb[f"W{i}"]),
                                               _ptr(self.g[f"W{i}"]), _ptr(b[f"dcol{i}"]) if i > 0 else None, ci, B,
-                                              Lin, co, *conv, _ptr(b.get(f"work{i}", b["work"])), _stream()),
-                        "efm_net_conv1d_back")
+                                              Lin, co, *conv, ldp, _stream()), "efm_net_conv1d_back")
             if i > 0:
-                db, work = rows(i - 1)
                 self._c(L.efm_net_col2im_relu_bias(_ptr(b[f"dcol{i}"]), _ptr(b[f"y{i - 1}"]), _ptr(b[f"dpb{i - 1}"]),
-                                                   db, ci, B, Lin, *conv, work, _stream()), "efm_net_col2im_relu_bias")
-        self._c(L.efm_net_sum(b["sums"], len(b["sums"]), _stream()), "efm_net_sum")
+                                                   _ptr(self.g[f"b{i - 1}"]), _ptr(b.get(f"chains{i - 1}")), ci, B, Lin,
+                                                   *conv, b[f"dpb{i - 1}"].stride(0), _stream()),
+                        "efm_net_col2im_relu_bias")
+        self._c(L.efm_net_bias_sums(b["biases"], len(b["biases"]), _stream()), "efm_net_bias_sums")
         return b["loss"]
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
@@ -355,13 +341,16 @@ class InitNet:
         """(N, nout) float32 outputs for the examples ``idx`` (default all) of a dataset."""
         N = data.shape[0]
         idx = torch.arange(N, dtype=torch.int32, device=self.dev) if idx is None else idx
-        dummy = torch.zeros((N, self.spec.nout), device=self.dev)
-        outs = []
-        for i in range(0, idx.numel(), batch):
-            part = idx[i:i + batch]
-            B = self.load_batch(data, dummy, part)
-            outs.append(self.forward_buffers(B).t().clone())
-        return torch.cat(outs)
+        n = idx.numel()
+        if n == 0:
+            raise RuntimeError("predict needs at least one example")
+        # targets that nothing reads, and every batch's outputs written where they belong
+        dummy = torch.empty((N, self.spec.nout), device=self.dev)
+        out = torch.empty((n, self.spec.nout), device=self.dev)
+        for i in range(0, n, batch):
+            B = self.load_batch(data, dummy, idx[i:i + batch])
+            out[i:i + B].copy_(self.forward_buffers(B).t())
+        return out
 
     def evaluate(self, data, targets, idx=None, batch=256):
         """Mean squared error over examples ``idx`` (float, synchronises)."""

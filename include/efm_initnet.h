@@ -51,7 +51,7 @@ int efm_net_relu_backward(const float *dy, const float *y, float *dpre, uint16_t
 /* db[m] = sum_n dpre[m*N + n]. */
 int efm_net_bias_grad(const float *dpre, float *db, int M, long long N, void *stream);
 
-/* A convolution with bias and ReLU, its weight gradient, and the ReLU and bias
+/* A convolution with bias and ReLU, its backward products, and the ReLU and bias
  * backward of a layer, without the im2col matrix in memory.  Kernel sizes 1 to 9 over
  * rows of at least 8 samples (else EFM_E_ARG).
  * x (C, B, L) BF16, W (M, C·ks) BF16; y[m, b*Lout + l] = max(sum_(c,k) W[m, c*ks + k] *
@@ -60,40 +60,32 @@ int efm_net_bias_grad(const float *dpre, float *db, int M, long long N, void *st
  * flattened as efm_net_flatten. */
 int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float *bias, float *y, uint16_t *yb,
                    int C, int B, int L, int M, int ks, int stride, int pad, int flat, void *stream);
-/* Floats of the workspace that suffices for the three calls below on this
- * convolution's arrays (-1: not a convolution efm_net_conv1d takes). */
-long long efm_net_conv1d_work(int C, int B, int L, int M, int ks, int stride, int pad);
-/* dW (M, C·ks) of dp (M, B·Lout) BF16 against x; a long sum over (b, l) is cut over
- * blocks and its parts added in a fixed order. */
-int efm_net_conv1d_dw(const uint16_t *dp, const uint16_t *x, float *dW, int C, int B, int L, int M,
-                      int ks, int stride, int pad, float *work, void *stream);
-/* The same, and dcol = W^T·dp (C·ks, B·Lout) beside it unless null; where the sum is cut
- * (efm_net_conv1d_parts > 1 of them) its parts are left in work, M·C·ks floats each, and
- * dW is not written. */
+/* 1 if efm_net_conv1d and efm_net_conv1d_back take this convolution, else 0. */
+int efm_net_conv1d_fits(int C, int B, int L, int M, int ks, int stride, int pad);
+/* ldp below: the distance of dp's (dpb's) rows.  dW (M, C·ks) of dp (M, B·Lout) BF16 against x, and dcol = W^T·dp (C·ks, B·Lout) beside
+ * it unless null: the sums of efm_net_gemm over efm_net_im2col's matrix, bit for bit. */
 int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const uint16_t *W, float *dW, float *dcol,
-                        int C, int B, int L, int M, int ks, int stride, int pad, float *work,
-                        void *stream);
-int efm_net_conv1d_parts(int C, int B, int L, int M, int ks, int stride, int pad);
-/* dpb = bf16(dy * (y > 0)) and db[m] = sum_n dy * (y > 0) for rows m < M of N values;
- * dy row-major, or with L > 0 flattened as efm_net_flatten (N = B·L).  work: 2048
- * floats, and at least M; with db null the row's parts stay there (efm_net_row_parts
- * of them, one after the other for each row). */
-int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, int M,
-                               int N, int B, int L, float *work, void *stream);
-int efm_net_row_parts(int M, int N);
+                        int C, int B, int L, int M, int ks, int stride, int pad, int ldp, void *stream);
+/* dpb = bf16(dy * (y > 0)) and db[m] = sum_n dy * (y > 0) for rows m < M of N values (the
+ * sum of efm_net_bias_grad, bit for bit); dy row-major, or with L > 0 flattened as
+ * efm_net_flatten (N = B·L).  With chains (256·M floats, see efm_net_bias_split) the sums'
+ * chains are left there for efm_net_bias_sums and db is not written. */
+int efm_net_relu_bias_backward(const float *dy, const float *y, uint16_t *dpb, float *db, float *chains,
+                               int M, int N, int B, int L, int ldp, void *stream);
 /* The same for dy = efm_net_col2im(dcol), y (C, B, L). */
-int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, int C,
-                             int B, int L, int ks, int stride, int pad, float *work, void *stream);
-/* out[i] = sum over k < parts of part[i*si + k*sk], i < n, in rising k, for n sums;
- * EFM_NET_SUMS of them to a launch. */
-#define EFM_NET_SUMS 12
+int efm_net_col2im_relu_bias(const float *dcol, const float *y, uint16_t *dpb, float *db, float *chains,
+                             int C, int B, int L, int ks, int stride, int pad, int ldp,
+                             void *stream);
+/* Whether M rows of N values are faster through chains. */
+int efm_net_bias_split(int M, int N);
+/* db[m] from chains[256·m ..] for rows m < M of each of n biases, EFM_NET_BIASES to a launch. */
+#define EFM_NET_BIASES 16
 typedef struct {
-    const float *part;
-    float *out;
-    long long n, si, sk;
-    int parts;
-} EfmNetSum;
-int efm_net_sum(const EfmNetSum *sums, int n, void *stream);
+    const float *chains;
+    float *db;
+    int M;
+} EfmNetBias;
+int efm_net_bias_sums(const EfmNetBias *biases, int n, void *stream);
 
 /* The dense head.  1 if efm_net_head_forward takes these sizes, 3 if efm_net_head_backward
  * does too (at most 128 examples and 16 outputs), else 0. */

@@ -1,12 +1,11 @@
 """The implicit-convolution kernels of the initializer at the edges of their tiles and
 dispatch: taps 1, 3, 8 and 9, row ends and padding wider than a load, channels and samples
-that do not fill a slab, sums over (b, l) short, long and cut over blocks, rows cut over
-blocks, and the shapes that keep the stored im2col matrix.
+that do not fill a slab, sums over (b, l) of one slab and of many, rows summed in one
+block and in chains, and the shapes that keep the stored im2col matrix.
 
-The forward pass is the stored-matrix path bit for bit (same sums).  Gradients are sums
-of n float32 terms against float64: |error| <= min(n, 4·sqrt(n))·u·sum|terms|, n roundings
-in any order (the worst case, or four standard deviations) of u = 2^-23, twice the
-rounding to nearest, as the matrix instruction may truncate inside.
+Every sum keeps the order of the stored-matrix path, so the two agree bit for bit; col2im,
+which has no counterpart of the same bits, is held to a float64 sum of its at most ks
+float32 terms: |error| <= ks·2^-24·sum|terms|.
 """
 
 import ctypes
@@ -29,8 +28,9 @@ SHAPES = [
     (17, 5, 31, 64, 3, 1, 0),       # no padding, odd rows
     (16, 2, 32, 130, 1, 3, 0),      # one tap
     (6, 2, 9, 8, 9, 1, 20),         # padding past the row: whole outputs of zeros
-    (16, 40, 64, 64, 9, 2, 4),      # sum of 1280: cut over blocks; rows of 2560: cut
-    (24, 7, 700, 16, 9, 1, 4),      # ragged last part of a cut sum, 8 does not divide it
+    (16, 40, 64, 64, 9, 2, 4),      # whole slabs of the backward sum
+    (24, 7, 700, 16, 9, 1, 4),      # a ragged last slab, 8 does not divide it
+    (3, 9, 4000, 20, 2, 3, 1),      # rows of 36000 values: chains longer than a round
 ]
 
 
@@ -40,10 +40,6 @@ def _p(t):
 
 def _ok(rc):
     _capi.check(rc, "net")
-
-
-def _bound(n, mag):
-    return min(n, 4 * np.sqrt(n)) * 2.0 ** -23 * mag + 1e-30
 
 
 def _dbl(t):
@@ -73,46 +69,67 @@ def test_conv_forward_is_the_stored_matrix_product(shape):
 
 
 @pytest.mark.parametrize("shape", SHAPES)
-def test_conv_gradients(shape):
+def test_conv_backward_products(shape):
     C, B, L, M, ks, stride, pad = shape
     lib, Lout = _capi.lib(), (L + 2 * pad - ks) // stride + 1
+    assert lib.efm_net_conv1d_fits(*shape) == 1
     g = torch.Generator().manual_seed(1 + sum(shape))
-    x = torch.randn(C, B, L, generator=g).bfloat16()
-    dp = torch.randn(M, B * Lout, generator=g).bfloat16()
-    y = torch.randn(C, B, L, generator=g)
-    dcol = torch.randn(C * ks, B * Lout, generator=g)
-    n = lib.efm_net_conv1d_work(C, B, L, M, ks, stride, pad)
-    work = torch.full((n,), float("nan"), device="cuda")
-    # weight gradient: dp · colᵀ
-    xp = torch.nn.functional.pad(x.double(), (pad, pad))
-    col = xp.unfold(2, ks, stride)[:, :, :Lout].permute(0, 3, 1, 2).reshape(C * ks, B * Lout)
-    dW = torch.empty(M, C * ks, device="cuda")
-    xd, dpd, dcold, yd = x.cuda(), dp.cuda(), dcol.cuda(), y.cuda()
-    _ok(lib.efm_net_conv1d_dw(_p(dpd), _p(xd), _p(dW), C, B, L, M, ks, stride, pad, _p(work), None))
-    err, mag = (_dbl(dW) - dp.double() @ col.T).abs(), dp.double().abs() @ col.abs().T
-    assert (err <= _bound(B * Lout, mag)).all()
-    # dy = col2im(dcol), then ReLU and the bias sum
-    dy = torch.zeros(C, B, L + 2 * pad + ks, dtype=torch.float64)
-    mg = torch.zeros_like(dy)
+    x, W = torch.randn(C, B, L, generator=g).bfloat16().cuda(), torch.randn(M, C * ks, generator=g).bfloat16().cuda()
+    dp = torch.randn(M, B * Lout, generator=g).bfloat16().cuda()
+    K, N = C * ks, B * Lout
+    col = torch.empty(K, N, dtype=torch.bfloat16, device="cuda")
+    _ok(lib.efm_net_im2col(_p(x), _p(col), C, B, L, ks, stride, pad, None))
+    wW, wcol = torch.empty(M, K, device="cuda"), torch.empty(K, N, device="cuda")
+    _ok(lib.efm_net_gemm(M, K, N, _p(dp), N, 1, _p(col), 1, N, _p(wW), K, None, None, 0, None))
+    _ok(lib.efm_net_gemm(K, N, M, _p(W), 1, K, _p(dp), N, 1, _p(wcol), N, None, None, 0, None))
+    wide = torch.full((M, N + 72), float("nan"), dtype=torch.bfloat16, device="cuda")       # rows further apart
+    wide[:, :N] = dp
+    for both, d in ((True, dp), (False, dp), (True, wide)):
+        dW, dcol = torch.full((M, K), 7.0, device="cuda"), torch.full((K, N), 7.0, device="cuda")
+        _ok(lib.efm_net_conv1d_back(_p(d), _p(x), _p(W), _p(dW), _p(dcol) if both else None, *shape,
+                                    d.stride(0), None))
+        torch.cuda.synchronize()
+        assert torch.equal(dW, wW)
+        assert torch.equal(dcol, wcol) if both else (dcol == 7.0).all()
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_relu_and_bias_rows(shape):
+    C, B, L, M, ks, stride, pad = shape
+    lib, Lout = _capi.lib(), (L + 2 * pad - ks) // stride + 1
+    g = torch.Generator().manual_seed(2 + sum(shape))
+    y, dcol = torch.randn(C, B, L, generator=g), torch.randn(C * ks, B * Lout, generator=g)
+    yd, dcold = y.cuda(), dcol.cuda()
+    dy = torch.empty(C, B, L, device="cuda")
+    _ok(lib.efm_net_col2im(_p(dcold), _p(dy), C, B, L, ks, stride, pad, None))
+    # the transposed im2col itself against float64
+    ref = torch.zeros(C, B, L + 2 * pad + ks, dtype=torch.float64)
+    mag = torch.zeros_like(ref)
     d4 = dcol.double().reshape(C, ks, B, Lout)
     for k in range(ks):
-        dy[:, :, k:k + stride * Lout:stride][:, :, :Lout] += d4[:, k]
-        mg[:, :, k:k + stride * Lout:stride][:, :, :Lout] += d4[:, k].abs()
-    dy, mg = dy[:, :, pad:pad + L], mg[:, :, pad:pad + L]
-    dpb, db = torch.empty(C, B, L, dtype=torch.bfloat16, device="cuda"), torch.empty(C, device="cuda")
-    _ok(lib.efm_net_col2im_relu_bias(_p(dcold), _p(yd), _p(dpb), _p(db), C, B, L, ks, stride, pad, _p(work), None))
-    on = (y > 0).double()
-    assert ((_dbl(dpb) - dy * on).abs() <= 2.0 ** -8 * (dy * on).abs() + _bound(ks, mg)).all()
-    assert ((_dbl(db) - (dy * on).sum((1, 2))).abs() <= _bound(ks * B * L, (mg * on).sum((1, 2)))).all()
-    # the same from a plain and a flattened dy
-    dyf = dy.float()
-    dyf_d = dyf.reshape(C, B * L).cuda()
-    flat = dyf.permute(0, 2, 1).reshape(C * L, B).contiguous().cuda()
-    for d, l in ((dyf_d, 0), (flat, L)):
-        _ok(lib.efm_net_relu_bias_backward(_p(d), _p(yd), _p(dpb), _p(db), C, B * L, B, l, _p(work), None))
-        assert torch.equal(dpb.cpu(), torch.where(y > 0, dyf, torch.zeros(())).bfloat16())
-        ref = dyf.double() * on
-        assert ((_dbl(db) - ref.sum((1, 2))).abs() <= _bound(B * L, ref.abs().sum((1, 2)))).all()
+        ref[:, :, k:k + stride * Lout:stride][:, :, :Lout] += d4[:, k]
+        mag[:, :, k:k + stride * Lout:stride][:, :, :Lout] += d4[:, k].abs()
+    ref, mag = ref[:, :, pad:pad + L], mag[:, :, pad:pad + L]
+    assert ((_dbl(dy) - ref).abs() <= ks * 2.0 ** -24 * mag).all()
+    dp = torch.where(yd > 0, dy, torch.zeros((), device="cuda"))
+    want = torch.empty(C, device="cuda")
+    _ok(lib.efm_net_bias_grad(_p(dp), _p(want), C, B * L, None))
+    flat = dy.permute(0, 2, 1).reshape(C * L, B).contiguous()
+    rows = lambda d, n: lambda *out: lib.efm_net_relu_bias_backward(_p(d), _p(yd), *out, C, B * L, B, n, B * L + 9, None)
+    for call in (lambda *out: lib.efm_net_col2im_relu_bias(_p(dcold), _p(yd), *out, C, B, L, ks, stride, pad, B * L + 9,
+                                                            None),
+                 rows(dy, 0), rows(flat, L)):
+        for chained in (False, True):
+            dpb = torch.full((C, B * L + 9), 7.0, dtype=torch.bfloat16, device="cuda")
+            db = torch.full((C,), 7.0, device="cuda")
+            chains = torch.full((C, 256), float("nan"), device="cuda")
+            _ok(call(_p(dpb), _p(db), _p(chains) if chained else None))
+            if chained:
+                assert (db == 7.0).all()
+                _ok(lib.efm_net_bias_sums(ctypes.byref(_capi.EfmNetBias(_p(chains), _p(db), C)), 1, None))
+            torch.cuda.synchronize()
+            assert torch.equal(dpb[:, :B * L], dp.bfloat16().reshape(C, B * L)) and (dpb[:, B * L:] == 7.0).all()
+            assert torch.equal(db, want)
 
 
 @pytest.mark.parametrize("spec,implicit", [
@@ -151,41 +168,16 @@ def test_gather_batch_rows(length):
     assert torch.equal(x, data[idx.long()].permute(1, 0, 2)) and torch.equal(t, target[idx.long()].T)
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_conv_backward_in_one_launch(shape):
-    """dW's parts and dcol from one launch: the separate calls' bits (the parts left unsummed
-    where there are several, dcol through the general product where it cannot ride along)."""
-    C, B, L, M, ks, stride, pad = shape
-    lib, Lout = _capi.lib(), (L + 2 * pad - ks) // stride + 1
-    g = torch.Generator().manual_seed(2 + sum(shape))
-    x, W = torch.randn(C, B, L, generator=g).bfloat16().cuda(), torch.randn(M, C * ks, generator=g).bfloat16().cuda()
-    dp = torch.randn(M, B * Lout, generator=g).bfloat16().cuda()
-    K, N, n = C * ks, B * Lout, M * C * ks
-    conv = (C, B, L, M, ks, stride, pad)
-    parts = lib.efm_net_conv1d_parts(*conv)
-    work = torch.zeros(max(parts * n, lib.efm_net_conv1d_work(*conv)), device="cuda")
-    dW, got, dcol, want = (torch.full(s, 7.0, device="cuda") for s in ((M, K), (M, K), (K, N), (K, N)))
-    _ok(lib.efm_net_conv1d_back(_p(dp), _p(x), _p(W), _p(got), _p(dcol), *conv, _p(work), None))
-    if parts > 1:
-        assert (got == 7.0).all()
-        s = _capi.EfmNetSum(_p(work), _p(got), n, 1, n, parts)
-        _ok(lib.efm_net_sum(ctypes.byref(s), 1, None))
-    _ok(lib.efm_net_conv1d_dw(_p(dp), _p(x), _p(dW), *conv, _p(work), None))
-    _ok(lib.efm_net_gemm(K, N, M, _p(W), 1, K, _p(dp), N, 1, _p(want), N, None, None, 0, None))
-    torch.cuda.synchronize()
-    assert torch.equal(got, dW) and torch.equal(dcol, want)
-
-
-@pytest.mark.parametrize("count", [0, 1, 12, 13, 30])
-def test_sum_lists(count):
-    """Lists below, at and above a launch's twelve sums; parts side by side and one after the other."""
+@pytest.mark.parametrize("count", [0, 1, 16, 17, 40])
+def test_bias_lists(count):
+    """Lists below, at and above a launch's sixteen biases."""
     lib, rng = _capi.lib(), np.random.default_rng(count)
-    ins, outs, sums = [], [], (_capi.EfmNetSum * count)()
+    ins, outs, biases = [], [], (_capi.EfmNetBias * count)()
     for j in range(count):
-        n, k = int(rng.integers(1, 700)), int(rng.integers(1, 9))
-        ins.append(torch.as_tensor(rng.integers(-8, 9, (k, n) if j % 2 else (n, k)).astype(np.float32)).cuda())
-        outs.append(torch.empty(n, device="cuda"))
-        sums[j] = _capi.EfmNetSum(_p(ins[j]), _p(outs[j]), n, 1 if j % 2 else k, n if j % 2 else 1, k)
-    _ok(lib.efm_net_sum(sums, count, None))
+        m = int(rng.integers(1, 70))
+        ins.append(torch.as_tensor(rng.integers(-8, 9, (m, 256)).astype(np.float32)).cuda())
+        outs.append(torch.empty(m, device="cuda"))
+        biases[j] = _capi.EfmNetBias(_p(ins[j]), _p(outs[j]), m)
+    _ok(lib.efm_net_bias_sums(biases, count, None))
     for j in range(count):
-        assert torch.equal(outs[j], ins[j].sum(0 if j % 2 else 1))          # whole numbers: exact
+        assert torch.equal(outs[j], ins[j].sum(1))                  # whole numbers: exact
