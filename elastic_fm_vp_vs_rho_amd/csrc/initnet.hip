@@ -416,21 +416,22 @@ __global__ __launch_bounds__(kFwdThreads) void k_conv_fwd(ConvShape q, const uin
 // 32 rows x 16 channels of one tap in one pass over (b, l), slabs of 256 samples: the sum
 // of an entry stays one accumulator over rising 32-deep MFMA steps, as in the product with
 // the stored matrix, since another order moves the last bit of a gradient, and Adam's
-// first steps turn that into other BF16 weights.  Waves 0 and 1 multiply, a row tile each,
-// with dp straight from memory (no other wave of the block wants it); 4 to 7 put the
-// 16 channels of the next slab into the other of two LDS buffers, a sample to a lane, so
-// that every lane's tap is in the row or not for all channels at once.  Three slabs of loads
-// are in flight.  What binds it is the vector memory path of a CU, which each slab's dp (0.28
-// us) and taps (0.38 us) share: 32 rows a block for 64 (the first layer's chain of 64
-// slabs 92 -> 63 us on 216 CUs), 16 go twice to a CU (101).  Four layers of 64 examples: 97 us
-// against 278 of 64 x 64 tiles over the stored matrix, its im2col not counted.
+// first steps turn that into other BF16 weights.  Waves 0 and 1 multiply, a row tile each;
+// 2 and 3 put the next slab's dp into the other of two LDS buffers, whole rows at a time,
+// and 4 to 7 its 16 channels, a sample to a lane, so that every lane's tap is in the row or
+// not for all channels at once.  Three slabs of loads are in flight.  What binds it is the
+// vector memory path of a CU, the taps' 2-byte loads above all (0.4 of 0.8 us a slab): 32 rows
+// a block for 64 (the first layer's chain of 64 slabs 92 -> 63 us on 216 CUs; blocks of 16
+// rows go twice to a CU, 101), dp in whole rows instead of MFMA fragments 63 -> 56.  Four
+// layers of 64 examples: 87 us against 278 of 64 x 64 tiles over the stored matrix, its
+// im2col not counted.
 constexpr int kDwSlab = 256, kDwLd = kDwSlab + 8, kDwThreads = 512, kDwRows = 32;
-constexpr int kDwLds = 2 * 16 * kDwLd;                // 16-bit words
+constexpr int kDwLds = 2 * (16 + kDwRows) * kDwLd;                // 16-bit words
 template <bool AVEC>
 __device__ __forceinline__ void conv_dw_tile(uint16_t *Bs, int c0, int tap, int m0, const ConvShape &q,
                                              const uint16_t *__restrict__ dp, int ldp,
                                              const uint16_t *__restrict__ x, float *__restrict__ out) {
-    constexpr int AHEAD = AVEC ? 3 : 1, NK = kDwSlab / 32;        // slabs of loads in flight
+    constexpr int AHEAD = AVEC ? 3 : 1, NK = kDwSlab / 32, NA = kDwRows * kDwSlab / 8 / 128;        // slabs of loads in flight
     const int K = q.B * q.Lout, BL = q.B * q.L;
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     // slabs, whole rounds of AHEAD: those past the end add nothing, and with no condition on a
@@ -465,42 +466,53 @@ __device__ __forceinline__ void conv_dw_tile(uint16_t *Bs, int c0, int tap, int 
             }
         return;
     }
-    if (w >= kDwRows / 16) return;
-    const int row = m0 + 16 * w + (lane & 15), ko = 8 * (lane >> 4);
-    const uint16_t *rowp = dp + (long long)min(row, q.M - 1) * ldp;      // rows past M: sums nobody stores
-    uint4 a[AHEAD][NK];
-    auto load = [&](uint4 (&g)[NK], int i) __attribute__((always_inline)) {
-        const int k0 = min(i, nslab) * kDwSlab + ko;
-        if (AVEC) {          // rows of whole vectors: in range or past the end as one
+    uint16_t *As = Bs + 2 * 16 * kDwLd;
+    if (w >= 2) {
+        // rows of dp, 512 contiguous bytes each
+        const int u = t - 128, kk = (u & 31) * 8;
+        uint4 a[AHEAD][NA];
+        auto load = [&](uint4 (&g)[NA], int i) __attribute__((always_inline)) {
+            const int k = min(i, nslab) * kDwSlab + kk;
 #pragma unroll
-            for (int k = 0; k < NK; ++k) g[k] = *reinterpret_cast<const uint4 *>(rowp + min(k0 + 32 * k, K - 8));
-        } else {
-#pragma unroll
-            for (int k = 0; k < NK; ++k) g[k] = conv_a8(rowp, K, 1, 0, k0 + 32 * k, K, false);
-        }
-    };
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int d = 0; d < AHEAD; ++d) load(a[d], d);
-#pragma unroll 1
-    for (int i = 0; i < nslab; i += AHEAD)
-#pragma unroll
-        for (int d = 0; d < AHEAD; ++d) {
-            __syncthreads();
-            const uint16_t *B = Bs + ((i + d) & 1) * 16 * kDwLd + (lane & 15) * kDwLd + ko;
-            uint4 v[NK];
-#pragma unroll
-            for (int k = 0; k < NK; ++k) v[k] = *reinterpret_cast<const uint4 *>(B + 32 * k);
-            if (AVEC && (i + d + 1) * kDwSlab > K) {
-#pragma unroll
-                for (int k = 0; k < NK; ++k)
-                    if ((i + d) * kDwSlab + 32 * k + ko >= K) a[d][k] = make_uint4(0, 0, 0, 0);
+            for (int j = 0; j < NA; ++j) {
+                const uint16_t *row = dp + (long long)min(m0 + (u >> 5) + 4 * j, q.M - 1) * ldp;     // past M: not stored
+                // a row of whole vectors is in range or past the end as one
+                g[j] = AVEC ? *reinterpret_cast<const uint4 *>(row + min(k, K - 8)) : conv_a8(row, K, 1, 0, k, K, false);
             }
-            __builtin_amdgcn_sched_barrier(0);        // all reads before the first product
+        };
 #pragma unroll
-            for (int k = 0; k < NK; ++k) acc = mfma_1(a[d][k], v[k], acc);
-            load(a[d], i + d + AHEAD);
+        for (int d = 0; d < AHEAD; ++d) load(a[d], d);
+#pragma unroll 1
+        for (int i = 0; i < nslab; i += AHEAD)
+#pragma unroll
+            for (int d = 0; d < AHEAD; ++d) {
+                const bool in = (i + d) * kDwSlab + kk < K;
+#pragma unroll
+                for (int j = 0; j < NA; ++j)
+                    *reinterpret_cast<uint4 *>(As + (((i + d) & 1) * kDwRows + (u >> 5) + 4 * j) * kDwLd + kk) =
+                        in ? a[d][j] : make_uint4(0, 0, 0, 0);
+                load(a[d], i + d + AHEAD);
+                __syncthreads();
+            }
+        return;
+    }
+    const int ko = 8 * (lane >> 4);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int i = 0; i < nslab; ++i) {
+        __syncthreads();
+        const uint16_t *A = As + ((i & 1) * kDwRows + 16 * w + (lane & 15)) * kDwLd + ko;
+        const uint16_t *B = Bs + ((i & 1) * 16 + (lane & 15)) * kDwLd + ko;
+        uint4 a[NK], v[NK];
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+            a[k] = *reinterpret_cast<const uint4 *>(A + 32 * k);
+            v[k] = *reinterpret_cast<const uint4 *>(B + 32 * k);
         }
+        __builtin_amdgcn_sched_barrier(0);        // all reads before the first product
+#pragma unroll
+        for (int k = 0; k < NK; ++k) acc = mfma_1(a[k], v[k], acc);
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = m0 + 16 * w + 4 * (lane >> 4) + r, c = c0 + (lane & 15);
