@@ -36,14 +36,17 @@ HBM_PEAK_GBS = 8000.0
 # traffic excluded):
 #   stress     v×3, λ, μ read; τ×6 read+write                    = 17 words
 #   velocity   τ×6, ρ read; v×3 read+write                        = 13 words
-#   adj_vel    v̄×3, forward v^{n+1}, v^n ×3 each, b̄×3 read; τ̄×6 and
-#              the ρ sum r+w                                       = 26 words
-#   adj_str    τ̄×6, forward v×3, λ, μ, μ̄×3 read; v̄×3, λμ-sums×5 r+w = 30 words
-ALG_BYTES = {"stress": 68, "velocity": 52, "adj_velocity": 104, "adj_stress": 120}
+# The reverse sweep images two steps at a time, so every second launch of an adjoint
+# sweep moves more; the mean of the two:
+#   adj_vel    v̄×3, b̄×3 read; τ̄×6 r+w                             = 18 words
+#              with the images: forward v×3 of two steps read, λμ-sums×5 r+w = 34
+#   adj_str    τ̄×6, λ, μ, μ̄×3 read; v̄×3 r+w                       = 17 words
+#              with the images: forward v×3 of three steps read, ρ sums×3 r+w = 32
+ALG_BYTES = {"stress": 68, "velocity": 52, "adj_velocity": 104, "adj_stress": 98}
 # The byte model of the metric counts an adjoint time step as 120 B (the adjoint
 # state's sweeps) + 24 B (three imaging accumulators read and written) = 144 B
-# per interior cell; the two-sweep design moves 224 B (its τ̄ crosses HBM
-# between the sweeps, it reads the derived medium and keeps 6 sums).
+# per interior cell; the two-sweep design moves 202 B (its τ̄ crosses HBM
+# between the sweeps, it reads the derived medium and keeps 8 sums).
 ADJ_STEP_MODEL_BYTES = 144
 FIXTURE_C2 = os.path.join(ROOT, "tests", "golden", "c2_gathers_400.npz")
 FIXTURE_C2_GRADIENT = os.path.join(ROOT, "tests", "golden", "c2_gradient_40.npz")
@@ -51,36 +54,36 @@ FIXTURE_C2_GRADIENT = os.path.join(ROOT, "tests", "golden", "c2_gradient_40.npz"
 # HBM bytes per dispatch on the 128^3 C2 grid, by tile "bx,bz,ny,map": rocprofv3
 # FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 (the factors that make the counters read
 # 256 MiB each way for a 256 MiB copy), medians over the dispatches of
-# `bench.py --profile-kernels`.  Only valid for the kernels' current sources and
+# `bench.py --profile-kernels`; adjoint sweeps: the mean of a plain and an imaging launch.  Only valid for the kernels' current sources and
 # the 128^3 grid; any other size reports traffic null.
 MEASURED_TRAFFIC = {
     "stress": {
-        "128,1,1,0": 191197637, "128,2,1,0": 171724689, "64,1,1,0": 208424926, "64,2,1,0": 187271551,
-        "64,4,1,0": 177759425, "64,4,2,0": 183068655, "128,1,1,8": 155800165, "128,2,1,8": 155800773,
-        "256,1,1,8": 155798693, "64,1,1,8": 155800069, "64,2,1,8": 155797926, "64,4,1,8": 155799461,
-        "64,4,2,8": 156048560, "64,8,1,8": 155785703, "128,1,1,16": 155861316, "128,1,2,16": 157314835,
-        "256,1,1,16": 155860004, "64,1,1,16": 155954500,
+        "128,1,1,0": 191223776, "128,2,1,0": 171734880, "64,1,1,0": 208441600, "64,2,1,0": 187298592,
+        "64,4,1,0": 177763136, "64,4,2,0": 182736192, "128,1,1,8": 155808832, "128,2,1,8": 155809216,
+        "256,1,1,8": 155798144, "64,1,1,8": 155808608, "64,2,1,8": 155802592, "64,4,1,8": 155807936,
+        "64,4,2,8": 155917984, "64,8,1,8": 155807520, "128,1,1,16": 155814912, "128,1,2,16": 155944608,
+        "256,1,1,16": 155815200, "64,1,1,16": 155816768,
     },
     "velocity": {
-        "128,1,1,0": 161603185, "128,2,1,0": 140184167, "64,1,1,0": 174893508, "64,2,1,0": 154752523,
-        "64,4,1,0": 145708997, "64,4,2,0": 148252102, "128,1,1,8": 124300601, "128,2,1,8": 124302857,
-        "256,1,1,8": 124293337, "64,1,1,8": 124300505, "64,2,1,8": 124301241, "64,4,1,8": 124293081,
-        "64,4,2,8": 124414799, "64,8,1,8": 124302617, "128,1,1,16": 124601857, "128,1,2,16": 125905375,
-        "256,1,1,16": 124322808, "64,1,1,16": 124376568,
+        "128,1,1,0": 159647456, "128,2,1,0": 140209152, "64,1,1,0": 174902912, "64,2,1,0": 154772352,
+        "64,4,1,0": 145724160, "64,4,2,0": 148228288, "128,1,1,8": 124312672, "128,2,1,8": 124314688,
+        "256,1,1,8": 124297984, "64,1,1,8": 124307296, "64,2,1,8": 124302720, "64,4,1,8": 124569920,
+        "64,4,2,8": 124533216, "64,8,1,8": 124313856, "128,1,1,16": 124578240, "128,1,2,16": 124572896,
+        "256,1,1,16": 124319840, "64,1,1,16": 124320288,
     },
     "adj_velocity": {
-        "128,1,1,0": 297996656, "128,2,1,0": 260773961, "64,1,1,0": 321601941, "64,2,1,0": 283630696,
-        "64,4,1,0": 265993074, "64,4,2,0": 312446312, "128,1,1,8": 231463820, "128,2,1,8": 231460153,
-        "256,1,1,8": 230669693, "64,1,1,8": 231400148, "64,2,1,8": 231437298, "64,4,1,8": 231500798,
-        "64,4,2,8": 253276609, "64,8,1,8": 232402444, "128,1,1,16": 239307653, "128,1,2,16": 266988764,
-        "256,1,1,16": 237318627, "64,1,1,16": 239244164,
+        "128,1,1,0": 329532192, "128,2,1,0": 283719280, "64,1,1,0": 358302208, "64,2,1,0": 314967504,
+        "64,4,1,0": 293014936, "64,4,2,0": 320474400, "128,1,1,8": 268284112, "128,2,1,8": 265236432,
+        "256,1,1,8": 265231568, "64,1,1,8": 269349808, "64,2,1,8": 268280304, "64,4,1,8": 265569216,
+        "64,4,2,8": 272011664, "64,8,1,8": 265270496, "128,1,1,16": 268242768, "128,1,2,16": 274238176,
+        "256,1,1,16": 264331984, "64,1,1,16": 268795792,
     },
     "adj_stress": {
-        "128,1,1,0": 388869317, "128,2,1,0": 333875468, "64,1,1,0": 422968550, "64,2,1,0": 370303011,
-        "64,4,1,0": 343344816, "64,4,2,0": 474192917, "128,1,1,8": 304226871, "128,2,1,8": 302532747,
-        "256,1,1,8": 302041446, "64,1,1,8": 305047935, "64,2,1,8": 304884462, "64,4,1,8": 304141087,
-        "64,4,2,8": 412439331, "64,8,1,8": 302609413, "128,1,1,16": 327087078, "128,1,2,16": 468075640,
-        "256,1,1,16": 323230582, "64,1,1,16": 327790592,
+        "128,1,1,0": 299155968, "128,2,1,0": 254146592, "64,1,1,0": 327458688, "64,2,1,0": 280861440,
+        "64,4,1,0": 259872160, "64,4,2,0": 283227936, "128,1,1,8": 219415520, "128,2,1,8": 219317104,
+        "256,1,1,8": 218819760, "64,1,1,8": 219518592, "64,2,1,8": 219461200, "64,4,1,8": 219215504,
+        "64,4,2,8": 224016704, "64,8,1,8": 218905024, "128,1,1,16": 219565520, "128,1,2,16": 225199792,
+        "256,1,1,16": 219458624, "64,1,1,16": 219382832,
     },
 }
 
