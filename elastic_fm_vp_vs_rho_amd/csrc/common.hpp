@@ -27,6 +27,7 @@ struct Geo {
     int pxc, pyc, pzc;                 // per-component strides of the ψ slabs
     const int *itp;                    // device time-step counter added to `it` (graph replay), or null
     int recw;                          // words per shot of the receiver bitmask, ceil(N/32)
+    int dense;                         // compact sweeps walk the interior cells only (see tile_coords)
 };
 
 struct StatePtrs {
@@ -61,6 +62,7 @@ inline Geo make_geo(const EfmDims &d) {
     g.pzc = d.ny * g.Lz * d.nx;
     g.itp = nullptr;
     g.recw = (int)((g.N + 31) / 32);
+    g.dense = 0;
     return g;
 }
 
@@ -119,20 +121,30 @@ __device__ __forceinline__ bool is_receiver(const Geo &g, const ShotPtrs &sh, in
     return (sh.recmask[(long long)s * g.recw + (t >> 5)] >> (t & 31)) & 1u;
 }
 
-// The receivers among a wave's cells, which follow one another in memory: t is the lane's
-// cell.  The active lanes take the list one receiver each; f(r, lane, hit) is called by all
-// of them for each share of the list, with the lane that owns the cell of this lane's
-// receiver r where there is one (hit).  A lane with a receiver that walked the list by
-// itself kept its wave, and with it the sweep, for 6.5 us per 100 receivers: velocity sweep
-// of 100^3 with 200 receivers 25.7 -> 13.0 us, 64^3 with 16 receivers 6.2 -> 5.7.
+// The receivers among a wave's cells, which follow one another in memory (or, in a dense
+// walk, among the interior cells of their plane): t is the lane's cell.  The active lanes
+// take the list one receiver each; f(r, lane, hit) is called by all of them for each
+// share of the list, with the lane that owns the cell of this lane's receiver r where there
+// is one (hit).  A lane with a receiver that walked the list by itself kept its wave, and
+// with it the sweep, for 6.5 us per 100 receivers: velocity sweep of 100^3 with 200
+// receivers 25.7 -> 13.0 us, 64^3 with 16 receivers 6.2 -> 5.7.
 template <typename F>
 __device__ __forceinline__ void wave_receivers(const Geo &g, const ShotPtrs &sh, int s, int t, F f) {
     const unsigned long long on = __ballot(1);
     const int lane = __lane_id(), n = __popcll(on), rank = __popcll(on & ((1ull << lane) - 1));
     const int *rs = sh.rec + (long long)s * g.nrec;
+    // place of cell c in the walk; another plane's or a guard cell of a dense walk: far away
+    const int y0 = g.dense ? t / g.sxz32 : 0;
+    auto place = [&](int c) {
+        if (!g.dense) return c;
+        const int p = c - y0 * g.sxz32, z = p / g.nx, x = p - z * g.nx;
+        const bool in = p >= 0 && p < g.sxz32 && x >= H && x < g.nx - H && z >= H && z < g.nz - H;
+        return in ? (z - H) * (g.nx - 2 * H) + x - H : -(1 << 30);
+    };
+    const int first = place(t) - lane;
     for (int r0 = 0; r0 < g.nrec; r0 += n) {
         const int r = r0 + rank;
-        const int j = (r < g.nrec ? rs[r] : -1) - (t - lane);
+        const int j = place(r < g.nrec ? rs[r] : -1) - first;
         f(r, j & 63, (unsigned)j < 64u && (on >> (j & 63) & 1));
     }
 }
@@ -212,8 +224,17 @@ __host__ __device__ constexpr int map_xcds(int map) { return map == 16 ? 8 : map
 // Floats of a 128-byte cache line, and the cells a compact sweep walks in a plane:
 // from the line of the first interior cell to the last interior cell.
 constexpr int kLine = 32;
+
+// A forward step over many cells in short rows loses more to the guard lanes (4 of nx) than
+// to lines shared by two waves, and walks the interior cells only (Geo::dense); aligned and
+// dense walks, us per step: 105.1 and 103.1 for 10 shots of 36x138x89, 49.6 and 48.4 for 8 of
+// 40x80x80, 94.9 and 94.0 for 9 of 52x124x78; even from 66 cells a row on.  Steps that take
+// little more than their launches (one shot of 41x37x33, 48^3) keep the aligned walk, whose
+// index arithmetic is shorter: 10.8 and 11.15, 11.0 and 11.3.
+constexpr int kDenseRow = 64;
+constexpr long long kDenseCells = 1 << 20;
 __host__ __device__ inline int plane_span(const Geo &g) {
-    return (g.nz - 2 * H) * g.nx - 2 * H + kLine - 1;
+    return g.dense ? (g.nz - 2 * H) * (g.nx - 2 * H) : (g.nz - 2 * H) * g.nx - 2 * H + kLine - 1;
 }
 
 // Number of tiles (blocks × y-chunks × shots) of a sweep: x-blocks × z-blocks,
@@ -276,6 +297,12 @@ __device__ __forceinline__ bool tile_coords(const Geo &g, int &x, int &z, int &s
         s = g.s0 + sl;
         const int qb = gi % nqb;
         yb = gi / nqb;
+        if (g.dense) {
+            const int q = qb * (BX * BZ) + threadIdx.y * BX + threadIdx.x, w = g.nx - 2 * H;
+            z = H + q / w;
+            x = H + q - (z - H) * w;
+            return z < g.nz - H;
+        }
         // position in the plane of the line-aligned cell the plane's walk starts at
         const int row0 = (H + yb * NYC) * g.sxz32;
         const int p = ((row0 + H * g.nx + H) & ~(kLine - 1)) - row0 + qb * (BX * BZ) + threadIdx.y * BX + threadIdx.x;
@@ -330,11 +357,13 @@ int set_tile(int kernel, Tile t);
 // Measured on the two sweeps, ns per thousand interior cell-steps by shots per
 // launch: 96^3 25.6 at 4 shots (190 MB), 25.8 at 5 (237 MB), 32.1 at 6 (281 MB), 35.0
 // at 32; 64^3 29.0 at 16 (248 MB), 42.0 at 24 (371 MB); 128^3 22.7 at 2 (223 MB),
-// 34.2 at 3.  32 shots of 96^3 went from 872 to 682 us per step.  Where even one shot
-// exceeds the cache all shots stay in one launch (fewer, longer launches).  The
-// adjoint sweeps gain nothing from groups (96^3: 71 ns with 8 shots in a launch,
-// 74-83 in groups of 2 or 1), so they take the whole batch.
-constexpr long long kCacheBytes = 240LL * 1000 * 1000;
+// 34.2 at 3.  32 shots of 96^3 went from 872 to 682 us per step.  The line lies where the
+// cache (268 MB) begins to miss more than a second round of launches costs: batches of
+// 240, 249, 258 and 263 MB took 98, 97, 102 and 123 us per step in one launch, 104, 106,
+// 108 and 114 in two.  Where even one shot exceeds the cache all shots stay in one launch
+// (fewer, longer launches).  The adjoint sweeps gain nothing from groups (96^3: 71 ns with
+// 8 shots in a launch, 74-83 in groups of 2 or 1), so they take the whole batch.
+constexpr long long kCacheBytes = 260LL * 1000 * 1000;
 
 // Bytes of one shot's nine fields and of its ψ slabs.
 inline long long field_bytes(const Geo &g) { return 36 * g.N; }

@@ -5,15 +5,13 @@
 // (M:1728-1734), kernel_Vx_Vy_Vz (M:133-188), kernel_get_Station (M:324-335),
 // kernel_get_border / kernel_set_border (M:378-462).
 //
-// Mapping: a block is BX (x, one 64-lane wave per row) × BZ (z) threads; each
-// thread owns one (x, z) column and marches NYC cells along y.  x is the
-// contiguous axis, so every wave issues fully coalesced 256-byte row loads; the
-// ±1 neighbours along x and z are the same rows shifted and are served from the
-// L1/LDS-backed vector cache of the CU, the ±y neighbour from the previous
-// march step.  ψ memory variables live only in CPML slabs (identically zero
-// elsewhere, where a = b = 0).  The moment-tensor source is added by the thread
-// that owns the source cell right after it writes τ (the reference adds it with
-// six separate gpuarray launches).
+// Mapping: a block is BX (x) × BZ (z) threads and each thread owns NYC cells along y; the
+// compact mapping (the default) deals a plane's cells to the lanes in memory order.  x is
+// the contiguous axis, so every wave issues coalesced row loads; a cell's ±1 neighbours are
+// other lanes' cells and come from the CU's vector cache or the XCD's L2.  ψ memory
+// variables live only in CPML slabs (identically zero elsewhere, where a = b = 0).  The
+// moment-tensor source is added by the thread that owns the source cell right after it
+// writes τ (the reference adds it with six separate gpuarray launches).
 #include "sweeps.hpp"
 
 namespace efm {
@@ -208,7 +206,9 @@ int run_forward(const Geo &g0, const EfmMedium &m, const ShotPtrs &sh, const Efm
                 bool in_place, float *gathers, float *borders, int W, int it0, int nsteps,
                 hipStream_t st) {
     const int group = group_shots(g0, field_bytes(g0) + psi_bytes(g0), 12 * g0.N);
-    return for_shot_groups(g0, group, [&](const Geo &g) {
+    Geo gd = g0;
+    gd.dense = gd.nx < kDenseRow && gd.N * gd.S >= kDenseCells;
+    return for_shot_groups(gd, group, [&](const Geo &g) {
         bool unsaved = false;       // the borders of the step before
         for (int k = 0; k < nsteps; ++k) {
             const int it = it0 + k;

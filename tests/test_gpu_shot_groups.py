@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("fuse", [True, False])
 def test_grouped_batch_equals_single_shots(gpu_lib, fuse):
     from elastic_fm_vp_vs_rho_amd.propagator import Propagator, ShotBatch
-    nt, S = 14, 13        # a 92^3 shot takes 33 MB with its CPML slabs: 13 make groups of 5, 5 and 3
+    nt, S = 14, 13        # a 92^3 shot takes 33 MB with its CPML slabs: 13 make groups of 7 and 6
     p = tiny(n=(92, 92, 92), nt=nt, W=4, seed=5, nrec=6)
     grid = grid_of(p)
     f = lambda a: torch.as_tensor(np.ascontiguousarray(a, np.float32), device="cuda")
