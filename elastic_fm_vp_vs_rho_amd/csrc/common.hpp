@@ -361,9 +361,13 @@ int set_tile(int kernel, Tile t);
 // cache (268 MB) begins to miss more than a second round of launches costs: batches of
 // 240, 249, 258 and 263 MB took 98, 97, 102 and 123 us per step in one launch, 104, 106,
 // 108 and 114 in two.  Where even one shot exceeds the cache all shots stay in one launch
-// (fewer, longer launches).  The adjoint sweeps gain nothing from groups (96^3: 71 ns with
+// (fewer, longer launches).  A batch only just larger than that also stays whole: 26 shots of
+// 73x64x37 (261 MB) take 100.5 us per step whole and 107.6 in two groups, with records of
+// 2/3 to all of the steps 88.6 and 95.1; 27 (271 MB) 112.3 and 111.6, 97.0 and 98.3; 29
+// (291 MB) 132.4 and 118.6, 111.2 and 102.8.  The adjoint sweeps gain nothing from groups (96^3: 71 ns with
 // 8 shots in a launch, 74-83 in groups of 2 or 1), so they take the whole batch.
 constexpr long long kCacheBytes = 260LL * 1000 * 1000;
+constexpr long long kWholeBytes = 272LL * 1000 * 1000;
 
 // Bytes of one shot's nine fields and of its ψ slabs.
 inline long long field_bytes(const Geo &g) { return 36 * g.N; }
@@ -373,7 +377,7 @@ inline long long psi_bytes(const Geo &g) { return 24LL * ((long long)g.pxc + g.p
 // `shared` bytes of the medium in every step; groups are as equal as possible.
 inline int group_shots(const Geo &g, long long per_shot, long long shared) {
     const long long fit = (kCacheBytes - shared) / (per_shot > 0 ? per_shot : 1);
-    if (fit < 1 || fit >= g.S) return g.S;
+    if (fit < 1 || fit >= g.S || g.S * per_shot + shared <= kWholeBytes) return g.S;
     const int groups = (int)((g.S + fit - 1) / fit);
     return (g.S + groups - 1) / groups;
 }
