@@ -28,10 +28,10 @@ int check_launch(const char *what) {
 }
 
 // Tiles: 0 stress, 1 velocity, 2 adjoint velocity, 3 adjoint stress.  The
-// default, blocks of 128 consecutive interior cells in the XCD-aware order
-// (map 16), keeps every wave full whatever nx is: measured within 0-2 % of the
-// best row tile at 128^3, 4-8 % behind it where rows fill whole waves
-// (256 wide), and 15-25 % ahead where they do not (200 and 132 wide).
+// default, blocks of 128 consecutive cells of a plane in the XCD-aware order
+// (map 16), gives every wave whole cache lines whatever nx is: within 0-2 % of
+// the best tile at 128^3 and 256 wide, and 15-25 % ahead of the row tiles where
+// rows do not fill whole waves (200 and 132 wide).
 static std::mutex g_tile_mu;
 static Tile g_tiles[4] = {{128, 1, 1, 16}, {128, 1, 1, 16}, {128, 1, 1, 16}, {128, 1, 1, 16}};
 #define EFM_TILE_ENTRY(a, b, c, o) {a, b, c, o},

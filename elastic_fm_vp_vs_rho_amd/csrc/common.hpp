@@ -361,11 +361,12 @@ int set_tile(int kernel, Tile t);
 // cache (268 MB) begins to miss more than a second round of launches costs: batches of
 // 240, 249, 258 and 263 MB took 98, 97, 102 and 123 us per step in one launch, 104, 106,
 // 108 and 114 in two.  Where even one shot exceeds the cache all shots stay in one launch
-// (fewer, longer launches).  A batch only just larger than that also stays whole: 26 shots of
-// 73x64x37 (261 MB) take 100.5 us per step whole and 107.6 in two groups, with records of
-// 2/3 to all of the steps 88.6 and 95.1; 27 (271 MB) 112.3 and 111.6, 97.0 and 98.3; 29
-// (291 MB) 132.4 and 118.6, 111.2 and 102.8.  The adjoint sweeps gain nothing from groups (96^3: 71 ns with
-// 8 shots in a launch, 74-83 in groups of 2 or 1), so they take the whole batch.
+// (fewer, longer launches).  A batch only just larger than that also stays whole: 26
+// shots of 73x64x37 (261 MB) take 100.5 us per step whole and 107.6 in two groups, with
+// records of 2/3 to all of the steps 88.6 and 95.1; 27 (271 MB) 112.3 and 111.6, 97.0 and
+// 98.3; 29 (291 MB) 132.4 and 118.6, 111.2 and 102.8.  The adjoint sweeps gain nothing from
+// groups (96^3: 71 ns with 8 shots in a launch, 74-83 in groups of 2 or 1), so they take
+// the whole batch.
 constexpr long long kCacheBytes = 260LL * 1000 * 1000;
 constexpr long long kWholeBytes = 272LL * 1000 * 1000;
 
