@@ -42,8 +42,8 @@ def shots_per_dispatch(grid):
     worst = 0
     for bx, bz, ny, mp in variants():
         nyc = -(-(grid.ny - 4) // ny)
-        if mp == 16:    # the plane's cells from the first interior one's cache line to the last
-            per = -(-((grid.nz - 4) * grid.nx - 4 + 31) // (bx * bz)) * bx * bz
+        if mp == 16:    # compact interior plane (what a sweep near the limit walks)
+            per = -(-(grid.nx - 4) * (grid.nz - 4) // (bx * bz)) * bx * bz
         else:
             per = -(-grid.nx // bx) * bx * -(-grid.nz // bz) * bz
         worst = max(worst, per * nyc)

@@ -11,6 +11,7 @@
 namespace efm {
 
 constexpr int H = 2;  // interior guard: 2 <= x,y,z < n-2 (reference M:54, 77, 152)
+constexpr int kLine = 32;  // floats of a 128-byte cache line
 
 // Everything a sweep kernel needs, passed by value (kernel-argument memory).
 struct Geo {
@@ -62,7 +63,11 @@ inline Geo make_geo(const EfmDims &d) {
     g.pzc = d.ny * g.Lz * d.nx;
     g.itp = nullptr;
     g.recw = (int)((g.N + 31) / 32);
-    g.dense = 0;
+    // the line-aligned walk takes the guard cells of its rows along: a batch that would pass a
+    // dispatch's 2^32 work-items with them (bound for blocks of up to 256 cells, 8 runs of
+    // blocks a shot) walks the interior cells only
+    const long long per_plane = (long long)(d.nz - 2 * H) * d.nx + kLine + 255;
+    g.dense = g.S * (per_plane * (d.ny - 2 * H) + 7 * 256) > (long long)UINT32_MAX;
     return g;
 }
 
@@ -221,10 +226,6 @@ struct Tile {
 // XCDs the blocks of an XCD-aware mapping are dealt over.
 __host__ __device__ constexpr int map_xcds(int map) { return map == 16 ? 8 : map; }
 
-// Floats of a 128-byte cache line, and the cells a compact sweep walks in a plane:
-// from the line of the first interior cell to the last interior cell.
-constexpr int kLine = 32;
-
 // A forward step over many cells in short rows loses more to the guard lanes (4 of nx) than
 // to lines shared by two waves, and walks the interior cells only (Geo::dense); aligned and
 // dense walks, us per step: 105.1 and 103.1 for 10 shots of 36x138x89, 49.6 and 48.4 for 8 of
@@ -233,6 +234,8 @@ constexpr int kLine = 32;
 // index arithmetic is shorter: 10.8 and 11.15, 11.0 and 11.3.
 constexpr int kDenseRow = 64;
 constexpr long long kDenseCells = 1 << 20;
+// The cells a compact sweep walks in a plane: from the line of the first interior cell to
+// the last interior cell, or the interior ones.
 __host__ __device__ inline int plane_span(const Geo &g) {
     return g.dense ? (g.nz - 2 * H) * (g.nx - 2 * H) : (g.nz - 2 * H) * g.nx - 2 * H + kLine - 1;
 }

@@ -207,7 +207,7 @@ int run_forward(const Geo &g0, const EfmMedium &m, const ShotPtrs &sh, const Efm
                 hipStream_t st) {
     const int group = group_shots(g0, field_bytes(g0) + psi_bytes(g0), 12 * g0.N);
     Geo gd = g0;
-    gd.dense = gd.nx < kDenseRow && gd.N * gd.S >= kDenseCells;
+    gd.dense |= gd.nx < kDenseRow && gd.N * gd.S >= kDenseCells;
     return for_shot_groups(gd, group, [&](const Geo &g) {
         bool unsaved = false;       // the borders of the step before
         for (int k = 0; k < nsteps; ++k) {

@@ -201,3 +201,19 @@ def test_efm_adjoint_checks_every_state(L, hole):
     by = ctypes.byref
     rc = L.efm_adjoint(by(d), by(m), 1, 1, by(sh), fwd, by(adj), by(adj2), 1, 1, 1, 5, 8, 0, None)
     assert rc == -1 and "null" in _capi.last_error(), _capi.last_error()
+
+
+def test_batches_up_to_the_dispatch_limit_are_accepted(L):
+    """A compact sweep of a batch just under 2^32 interior work-items walks the interior
+    cells when the line-aligned walk, guard cells included, would pass the limit; just over
+    it the batch is refused as before."""
+    from elastic_fm_vp_vs_rho_amd import _capi
+    from elastic_fm_vp_vs_rho_amd._capi import EfmDims
+    for nx, ny, nz in ((32, 460, 460), (8, 40, 40), (64, 200, 200), (512, 300, 300)):
+        # the default tile: 128 interior cells of a plane to a block, 8 runs of a shot's blocks
+        blocks = -(-(nx - 4) * (nz - 4) // 128) * (ny - 4)
+        most = ((1 << 32) - 1) // (128 * 8 * -(-blocks // 8))
+        dims = lambda S: EfmDims(nx, ny, nz, S, 0, 0, 0, 0, 0, 0, 10, 0, 0.1)
+        assert L.efm_border_floats(ctypes.byref(dims(most)), 2) > 0, (nx, _capi.last_error())
+        assert L.efm_border_floats(ctypes.byref(dims(most + 1)), 2) == -1
+        assert "shot batch too large" in _capi.last_error()
