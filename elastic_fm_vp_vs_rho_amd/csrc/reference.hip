@@ -123,25 +123,6 @@ __device__ __forceinline__ void image_cell(const Geo &g, const ImageRef &im, Cel
     im.grho[so + i] += r;
 }
 
-// The images of a range's last iteration.
-__global__ void k_image_ref(Geo g, Med m, StatePtrs a, ImageRef im) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = g.s0 + blockIdx.y;
-    if (i >= g.N) return;
-    const int row = i / g.nx;
-    const int x = i - row * g.nx;
-    const int y = row / g.nz;
-    const int z = row - y * g.nz;
-    if (!interior(x, y, z, g)) return;
-    const int nx = g.nx, sxz = g.sxz32;
-    const long long so = (long long)s * g.N, t = so + i;
-    const float *mu = m.mu;
-    image_cell(g, im, CellOld{a.v[0][t], a.v[1][t], a.v[2][t], a.t[0][t], a.t[1][t], a.t[2][t], a.t[3][t], a.t[4][t],
-                              a.t[5][t], m.lam[i], mu[i], frcp(mu[i]), frcp(mu[i + 1]), frcp(mu[i + nx]),
-                              frcp(mu[i + sxz]), frcp(mu[i + 1 + nx]), frcp(mu[i + nx + sxz]), frcp(mu[i + 1 + sxz])},
-               so, i);
-}
-
 // Jobs of a shared launch: the adjoint's sweep and the reconstruction's, as shots
 // s0 .. s0+S-1 of the first and then of the second (job0: the first job present).
 __device__ __forceinline__ int split_job(const Geo &g, int job0, int &s) {
@@ -164,19 +145,20 @@ constexpr int kAdjoint = 0, kRemake = 1;
 // bottom CPML zones: τ there only reaches velocities that the restored borders
 // and the zeroing replace.  100^3, W = 10: 27 us for both, against 15 + 15 + 17 us
 // of the sweeps and the images alone (each about 4 us of launch, and the images read
-// again what the sweep holds).
+// again what the sweep holds).  Without `step` the adjoint's job forms the images alone
+// (behind a range's last iteration).
 template <int BX, int BZ, int NYC, int MAP>
 __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_ref_stress(Geo g, Med m, ShotPtrs sh, StatePtrs a, StatePtrs f, int it,
-                                                           ImageRef im, int W, int job0, int njobs) {
+                                                           int step, ImageRef im, int W, int job0, int njobs) {
     int x, z, s, yb;
     if (!tile_coords<BX, BZ, NYC, MAP>(with_jobs(g, njobs), x, z, s, yb)) return;
     if (x < H || x >= g.nx - H || z < H || z >= g.nz - H) return;
     const int y0 = H + yb * NYC, y1 = min(y0 + NYC, g.ny - H);
     if (split_job(g, job0, s) == kAdjoint) {
         const long long sa = (long long)s * g.N;
-        const bool step = it < sh.nt[s];
-        if (!step && !im.glam) return;
-        stress_cells<NYC>(g, m, sh, a, a, it, 0, x, z, s, yb, step, [&](int t, CellOld o) EFM_INLINE {
+        const bool write = step && it < sh.nt[s];
+        if (!write && !im.glam) return;
+        stress_cells<NYC>(g, m, sh, a, a, it, 0, x, z, s, yb, write, [&](int t, CellOld o) EFM_INLINE {
             if (im.glam) image_cell(g, im, o, sa, t);
         });
     } else {
@@ -385,16 +367,16 @@ static bool jobs_fit(const Geo &g, const Tile &t, long long extra) {
 }
 
 static int launch_ref_stress(const Geo &g, const Med &md, const ShotPtrs &sh, const StatePtrs &a, const StatePtrs &f,
-                             int it, const ImageRef &im, int W, int job0, int njobs, hipStream_t st) {
+                             int it, bool step, const ImageRef &im, int W, int job0, int njobs, hipStream_t st) {
     const Tile t = get_tile(0);
     if (njobs == 2 && !jobs_fit(g, t, 0)) {
-        if (int rc = launch_ref_stress(g, md, sh, a, f, it, im, W, kAdjoint, 1, st)) return rc;
-        return launch_ref_stress(g, md, sh, a, f, it, im, W, kRemake, 1, st);
+        if (int rc = launch_ref_stress(g, md, sh, a, f, it, step, im, W, kAdjoint, 1, st)) return rc;
+        return launch_ref_stress(g, md, sh, a, f, it, step, im, W, kRemake, 1, st);
     }
     const dim3 grid = sweep_grid(with_jobs(g, njobs), t);
     bool launched = false;
 #define X(a_, b_, c_, o_) \
-    EFM_LAUNCH_GRID_IF(a_, b_, c_, o_, grid, k_ref_stress, g, md, sh, a, f, it, im, W, job0, njobs)
+    EFM_LAUNCH_GRID_IF(a_, b_, c_, o_, grid, k_ref_stress, g, md, sh, a, f, it, step, im, W, job0, njobs)
     EFM_TILE_LIST(X)
 #undef X
     if (!launched) return fail(EFM_E_UNSUPPORTED, "unsupported stress tile");
@@ -428,18 +410,19 @@ static int launch_ref_velocity(const Geo &g, const Med &md, const ShotPtrs &sh, 
 // Iterations it0 .. it0+nsteps-1 of the reverse loop.  The present velocity
 // alternates between the forward state's v and vpres (swapped every
 // iteration), so iteration `it` finds it in fwd.v when it is even and in vpres
-// when it is odd: a run split into ranges gives the same results as one run over
-// all nt-1 iterations.
+// when it is odd.
 //
 // Iteration it: [adjoint stress, images of it-1 | reconstruction's stress of it-1],
-// [adjoint velocity, residual | reconstruction's velocity, borders, zones].  The
+// [adjoint velocity, residual | reconstruction's velocity, borders].  The
 // reconstruction's stress sweep and the images of an iteration need what both of its
 // velocity sweeps wrote and nothing after them, so they wait for the next launch; the
-// last iteration's get launches of their own.  The zones of both velocity buffers are
-// zeroed, guard cells included, in a range's first two iterations, which keep the
-// reconstruction's velocity sweep, border and zeroing as separate launches; later ones
-// leave the zones untouched.  A CPML narrower than the guard layer keeps the separate
-// launches throughout, as does a batch whose two sweeps exceed one dispatch.
+// last iteration's get one of their own.  The zones of both velocity buffers are
+// zeroed, guard cells included, behind a range's first two iterations; no later one
+// writes them.  Every iteration's sweeps and images are the same kernels wherever a
+// range starts or ends, so a run split into ranges leaves the bits of one run over all
+// nt-1 iterations.  A CPML narrower than the guard layer has the reconstruction's
+// velocity sweep, the borders and the zeroing as separate launches throughout, as does
+// a batch whose two sweeps exceed one dispatch.
 static int backward_remake_ref(const EfmDims *d, const EfmMedium *m, const EfmShots *sh,
                                const EfmState *fwd, float *vpres, const float *borders, int W,
                                const EfmState *adj, const float *res, float dt, float dx, float dy,
@@ -476,25 +459,24 @@ static int backward_remake_ref(const EfmDims *d, const EfmMedium *m, const EfmSh
     };
     for (int it = it0; it < it0 + nsteps; ++it) {
         const bool first = it == it0;
-        if ((rc = launch_ref_stress(ga, md, shp, a, cur, it, first ? ImageRef{} : images(), W, kAdjoint,
+        if ((rc = launch_ref_stress(ga, md, shp, a, cur, it, true, first ? ImageRef{} : images(), W, kAdjoint,
                                     first ? 1 : 2, st)))
             return rc;
-        const bool fused = fits && it >= it0 + 2;
         const int slot = nt - it - 2;
-        if ((rc = launch_ref_velocity(ga, md, shp, a, cur, nxt, it, res, borders, W, slot, fused ? 2 : 1, st)))
+        if ((rc = launch_ref_velocity(ga, md, shp, a, cur, nxt, it, res, borders, W, slot, fits ? 2 : 1, st)))
             return rc;
-        if (!fused) {
+        if (!fits) {
             if ((rc = launch_velocity(gf, *m, shp, cur, nxt, it, st))) return rc;
             if ((rc = launch_border(gf, shp, nxt, const_cast<float *>(borders), W, slot, 0, -1, st))) return rc;
+        }
+        if (!fits || it < it0 + 2) {
             hipLaunchKernelGGL(k_zero_cpml, dim3(nblk(ga.N, 256), ga.S), dim3(256), 0, st, ga, nxt, W);
             if ((rc = check_launch("zero cpml"))) return rc;
         }
         std::swap(cur.v, nxt.v);
     }
     if (nsteps == 0) return EFM_OK;
-    if ((rc = launch_stress_src(gf, *m, shp, cur, cur, it0 + nsteps - 1, -1, st))) return rc;
-    hipLaunchKernelGGL(k_image_ref, dim3(nblk(ga.N, 256), ga.S), dim3(256), 0, st, ga, md, a, images());
-    return check_launch("image");
+    return launch_ref_stress(ga, md, shp, a, cur, it0 + nsteps, false, images(), W, kAdjoint, 2, st);
 }
 
 extern "C" int efm_backward_remake_ref(const EfmDims *d, const EfmMedium *m, const EfmShots *sh,

@@ -219,7 +219,8 @@ int efm_backward_mt_ref(const EfmDims *d, const EfmMedium *m, const EfmShots *sh
                         const EfmState *adj, const float *res, double *gm6, int nsteps,
                         void *stream);
 /* backwardFields_FowardFieldsRemake (M:1929-2054, mode 1), nt-1 iterations.
- * fwd is the final forward state (consumed), vpres is a 3-volume scratch
+ * fwd is the final forward state (consumed: its stresses and ψ within W cells
+ * of the x, y and bottom faces are not rebuilt), vpres is a 3-volume scratch
  * (S, 3, ny, nz, nx), borders from efm_forward, adj zero on entry.  Imaging
  * kernel_Gradients_Rho/_Lambda/_Mu (M:191-294) accumulated into glam, gmu,
  * grho (S, ny, nz, nx) in float32 like the reference's host sums. */
@@ -230,8 +231,8 @@ int efm_backward_remake_ref(const EfmDims *d, const EfmMedium *m, const EfmShots
                             void *stream);
 /* Iterations it0 .. it0+nsteps-1 of efm_backward_remake_ref (the body of the
  * reference's per-step loop, M:1939-2054, which it drives from Python one
- * iteration at a time).  Ranges that cover 0 .. nt-2 in order give the
- * launches of one efm_backward_remake_ref call. */
+ * iteration at a time).  Ranges that cover 0 .. nt-2 in order leave adj, vpres,
+ * fwd and the images as one efm_backward_remake_ref call does, bit for bit. */
 int efm_backward_remake_ref_steps(const EfmDims *d, const EfmMedium *m, const EfmShots *sh,
                                   const EfmState *fwd, float *vpres, const float *borders, int W,
                                   const EfmState *adj, const float *res, float dt, float dx,

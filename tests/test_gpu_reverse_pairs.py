@@ -138,3 +138,36 @@ def test_border_save_beside_the_next_sweep(case):
         got.append((borders.cpu(), gat.cpu()))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
     assert (got[0][0] != 7.0).any()
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_ranges_leave_the_bits_of_one_run(case):
+    """What a run over all iterations leaves (images, adjoint, both velocity buffers, stresses
+    and memory variables of the reconstruction) is left bit for bit by any ranges."""
+    nx, ny, nz, W, nts, free_top, fuse, tiles = case
+    _with_tiles(tiles)
+    S, L = len(nts), _capi.lib()
+    left = []
+    for ranges in ([(0, NT - 1)], [(i, 1) for i in range(NT - 1)], [(0, 4), (4, 0), (4, NT - 5)], [(0, 1), (1, 2), (3, NT - 4)]):
+        prop, batch, rng = _prop(nx, ny, nz, W, S, nts, free_top, fuse)
+        d, m, sh = prop.dims(), prop.medium(), batch.struct()
+        fwd, adj = _state(prop, rng, 1e-3), _state(prop, rng, 1e-3)
+        vol = rng.standard_normal((S, NT, 3) + prop.grid.shape).astype(np.float32) * 1e-3
+        borders = torch.as_tensor(np.stack([_faces(v, W) for v in vol.reshape((-1,) + prop.grid.shape)]), device="cuda")
+        res = torch.as_tensor(rng.standard_normal((S, 3, NT, 9)).astype(np.float32) * 1e-3, device="cuda")
+        if not fuse:
+            res[..., 1] = 0.0            # receivers that share a cell add in any order
+        vpres = torch.zeros(S * 3 * prop.grid.N, device="cuda")
+        g3 = [torch.zeros((S,) + prop.grid.shape, device="cuda") for _ in range(3)]
+        for it0, n in ranges:
+            _capi.check(L.efm_backward_remake_ref_steps(
+                by(d), by(m), by(sh), by(fwd.struct()), _ptr(vpres), _ptr(borders), W, by(adj.struct()), _ptr(res),
+                DT, 10.0, 10.0, 10.0, *[_ptr(t) for t in g3], it0, n, _stream()), "remake")
+        torch.cuda.synchronize()
+        parts = [vpres, *g3]
+        for w in (fwd, adj):
+            parts += [w.fields, w.psi_x, w.psi_y, w.psi_z]
+        left.append([t.cpu() for t in parts])
+    for other in left[1:]:
+        for a, b in zip(left[0], other):
+            assert torch.equal(a, b)
