@@ -359,17 +359,17 @@ extern "C" long long efm_border_floats(const EfmDims *d, int W) {
     return border_floats(make_geo(*d), W);
 }
 
-// Whether the sweeps of both jobs, and `extra` blocks, fit one dispatch (< 2^32
+// Whether the sweeps of njobs jobs, and `extra` blocks, fit one dispatch (< 2^32
 // work-items, 65535 blocks along z).
-static bool jobs_fit(const Geo &g, const Tile &t, long long extra) {
-    const dim3 d = sweep_grid_plus(with_jobs(g, 2), t, extra);
+static bool jobs_fit(const Geo &g, int njobs, const Tile &t, long long extra) {
+    const dim3 d = sweep_grid_plus(with_jobs(g, njobs), t, extra);
     return grid_blocks(d) * t.bx * t.bz <= (long long)UINT32_MAX && d.z <= 65535;
 }
 
 static int launch_ref_stress(const Geo &g, const Med &md, const ShotPtrs &sh, const StatePtrs &a, const StatePtrs &f,
                              int it, bool step, const ImageRef &im, int W, int job0, int njobs, hipStream_t st) {
     const Tile t = get_tile(0);
-    if (njobs == 2 && !jobs_fit(g, t, 0)) {
+    if (njobs == 2 && !jobs_fit(g, 2, t, 0)) {
         if (int rc = launch_ref_stress(g, md, sh, a, f, it, step, im, W, kAdjoint, 1, st)) return rc;
         return launch_ref_stress(g, md, sh, a, f, it, step, im, W, kRemake, 1, st);
     }
@@ -383,14 +383,16 @@ static int launch_ref_stress(const Geo &g, const Med &md, const ShotPtrs &sh, co
     return check_launch("reverse stress sweeps");
 }
 
-// njobs 1: the adjoint's sweep alone.
+// njobs 1: the adjoint's sweep alone; the residual then takes a launch of its own where the
+// blocks for its receivers would pass a dispatch's limit.
 static int launch_ref_velocity(const Geo &g, const Med &md, const ShotPtrs &sh, const StatePtrs &a,
                                const StatePtrs &cur, const StatePtrs &nxt, int it, const float *res,
                                const float *borders, int W, int slot, int njobs, hipStream_t st) {
     const Tile t = get_tile(1);
-    const bool fused = sh.recmask && g.nrec > 0;
+    const auto blocks = [&](long long n) { return (n + t.bx * t.bz - 1) / (t.bx * t.bz); };
+    const bool fused = sh.recmask && g.nrec > 0 && (njobs == 2 || jobs_fit(g, 1, t, blocks((long long)g.S * g.nrec)));
     const long long n = (fused ? (long long)g.S * g.nrec : 0) + (njobs == 2 ? 3LL * guard_borders(g) * g.S : 0);
-    const long long extra = (n + t.bx * t.bz - 1) / (t.bx * t.bz);
+    const long long extra = blocks(n);
     const Geo gj = with_jobs(g, njobs);
     const dim3 grid = sweep_grid_plus(gj, t, extra);
     const long long nsweep = grid_blocks(sweep_grid(gj, t));
@@ -451,7 +453,7 @@ static int backward_remake_ref(const EfmDims *d, const EfmMedium *m, const EfmSh
     const long long vol = (long long)ga.S * ga.N;
     nxt.v[0] = vpres; nxt.v[1] = vpres + vol; nxt.v[2] = vpres + 2 * vol;
     if (it0 & 1) std::swap(cur.v, nxt.v);
-    const bool fits = W >= H && jobs_fit(ga, get_tile(1), (long long)ga.S * (ga.nrec + 3LL * guard_borders(ga)));
+    const bool fits = W >= H && jobs_fit(ga, 2, get_tile(1), (long long)ga.S * (ga.nrec + 3LL * guard_borders(ga)));
     // cur and nxt after an iteration's swap: the reconstruction's new and old velocities
     auto images = [&]() {
         return ImageRef{{cur.v[0], cur.v[1], cur.v[2]}, {nxt.v[0], nxt.v[1], nxt.v[2]}, 1.f / dt, 1.f / dx, 1.f / dy,
