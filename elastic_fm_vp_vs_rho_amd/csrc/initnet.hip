@@ -1088,21 +1088,26 @@ extern "C" int efm_net_col2im(const float *dcol, float *dx, int C, int B, int L,
 }
 
 // A convolution the implicit kernels take: at most 9 taps, rows of at least 8 samples,
-// 32-bit offsets into x.
+// 32-bit offsets into x, and launches within a dispatch's limits.
 #define EFM_CONV_SIZES(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
+constexpr long long kConvBlocks = 1LL << 22;
+static long long dw_blocks(const ConvShape &q) {
+    const long long tiles = (q.C + 15LL) / 16 * q.ks * ((q.M + kDwRows - 1) / kDwRows);
+    return (tiles + 7) / 8 * 8;
+}
 static bool conv_shape(ConvShape &q, int C, int B, int L, int M, int ks, int stride, int pad) {
     if (!conv_ok(C, B, L, ks, stride, pad) || M <= 0 || ks > 9 || L < 8) return false;
     const long long lim = 1LL << 31, Lout = (L + 2LL * pad - ks) / stride + 1;
     q = ConvShape{C, B, L, M, ks, stride, pad, (int)Lout};
     return (long long)C * B * L < lim && (long long)C * ks < lim - 1024 && B * Lout < lim - 1024 &&
-           L + 2LL * pad + ks < lim;
+           L + 2LL * pad + ks < lim && (M + 63LL) / 64 <= 65535 &&
+           (B * Lout + 63) / 64 * kFwdThreads <= (long long)UINT32_MAX && dw_blocks(q) < kConvBlocks;
 }
 
 extern "C" int efm_net_conv1d(const uint16_t *x, const uint16_t *W, const float *bias, float *y, uint16_t *yb,
                               int C, int B, int L, int M, int ks, int stride, int pad, int flat, void *stream) {
     ConvShape q;
     NET_CHECK(x && W && bias && y && yb && conv_shape(q, C, B, L, M, ks, stride, pad), "efm_net_conv1d: bad arguments");
-    NET_CHECK((M + 63) / 64 <= 65535, "efm_net_conv1d: M too large");
     const int avec = (C * ks) % 8 == 0 && (uintptr_t)W % 16 == 0;
     const dim3 grid((B * q.Lout + 63) / 64, (M + 63) / 64);
     hipStream_t st = (hipStream_t)stream;
@@ -1127,11 +1132,10 @@ extern "C" int efm_net_conv1d_back(const uint16_t *dp, const uint16_t *x, const 
               "efm_net_conv1d_back: bad arguments");
     const int K = B * q.Lout, gn = (K + GBN - 1) / GBN;
     const bool avec = K % 8 == 0 && ldp % 8 == 0 && (uintptr_t)dp % 16 == 0;
-    // dcol rides along where its product may take 16-byte loads
-    const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0;
-    const long long tiles = (C + 15LL) / 16 * ks * ((M + kDwRows - 1) / kDwRows), dw = (tiles + 7) / 8 * 8;
-    const long long blocks = dw + (both ? ((long long)gn * ((C * ks + GBM - 1) / GBM) + 1) / 2 : 0);
-    NET_CHECK(blocks < (1LL << 22), "efm_net_conv1d_back: too large");
+    // dcol rides along where its product may take 16-byte loads and the launch holds both
+    const long long dw = dw_blocks(q), with = dw + ((long long)gn * ((C * ks + GBM - 1) / GBM) + 1) / 2;
+    const bool both = dcol && avec && C * ks % 8 == 0 && (uintptr_t)W % 16 == 0 && with < kConvBlocks;
+    const long long blocks = both ? with : dw;
     (avec ? k_conv_back<true> : k_conv_back<false>)<<<(unsigned)blocks, kDwThreads, 0, (hipStream_t)stream>>>(
         q, dp, ldp, x, dW, (int)dw, W, dcol, gn);
     if (int rc = check_launch("efm_net_conv1d_back")) return rc;

@@ -217,3 +217,16 @@ def test_batches_up_to_the_dispatch_limit_are_accepted(L):
         assert L.efm_border_floats(ctypes.byref(dims(most)), 2) > 0, (nx, _capi.last_error())
         assert L.efm_border_floats(ctypes.byref(dims(most + 1)), 2) == -1
         assert "shot batch too large" in _capi.last_error()
+
+
+def test_implicit_convolution_limits(L):
+    """A convolution that the implicit kernels' launches cannot hold (rows of a 64 x 64 tile
+    grid, 2^32 work-items of 64 columns a 1024-thread block, blocks of the weight gradient)
+    is not taken by them: such a network keeps the stored im2col matrix."""
+    #        C, B, L, M, ks, stride, pad
+    for n, shape in enumerate([(1, 1, 8, 64 * 65535 + 1, 1, 1, 0), (1, 1 << 25, 8, 1, 1, 1, 0),
+                               (16384, 1, 8, 16384, 9, 1, 4)]):
+        assert L.efm_net_conv1d_fits(*shape) == 0, shape
+    for shape in [(1, 1, 8, 64 * 65535, 1, 1, 0), (1, (1 << 25) - 8, 8, 1, 1, 1, 0), (8192, 1, 8, 16384, 9, 1, 4),
+                  (192, 64, 1024, 64, 9, 4, 4)]:
+        assert L.efm_net_conv1d_fits(*shape) == 1, shape
