@@ -579,8 +579,8 @@ __device__ __forceinline__ void relu_bias_row(const float *__restrict__ y, uint1
         __shared__ float red[256];
         float s = 0.f;
 #pragma unroll 4
-        for (int n = t; n < N; n += 256) {
-            const float d = value(m, n);
+        for (unsigned n = t; n < (unsigned)N; n += 256) {      // N may be within 256 of 2^31
+            const float d = value(m, (int)n);
             const float v = y[row + n] > 0.f ? d : 0.f;
             dpb[n] = f2bf(v);
             s += v;
@@ -645,7 +645,7 @@ template <int T>
 __global__ __launch_bounds__(256) void k_col2im_relu_bias(const float *__restrict__ dcol, const float *__restrict__ y,
                                                           uint16_t *__restrict__ dpb, float *__restrict__ db,
                                                           float *__restrict__ chains, ConvShape q, int ldp) {
-    const unsigned ncol = q.B * q.Lout, L = q.L, stride = q.stride;
+    const unsigned ncol = (unsigned)q.B * q.Lout, L = q.L, stride = q.stride;
     relu_bias_row(y, dpb, db, chains, q.B * q.L, ldp, [&](int c, int n) __attribute__((always_inline)) {
         const unsigned b = (unsigned)n / L, j = n - b * L + q.pad;
         int l = j / stride, k = j - l * stride;

@@ -181,3 +181,19 @@ def test_bias_lists(count):
     _ok(lib.efm_net_bias_sums(biases, count, None))
     for j in range(count):
         assert torch.equal(outs[j], ins[j].sum(1))                  # whole numbers: exact
+
+
+def test_longest_row():
+    """A row of 2^31 - 1 values in one block: the last round of 256 passes 2^31.  Each chain is
+    a whole number below 2^24, the tree over them within 8 roundings."""
+    lib, N = _capi.lib(), 2 ** 31 - 1
+    if torch.cuda.mem_get_info()[0] < 25 * 10 ** 9:
+        pytest.skip("needs 25 GB of free GPU memory")
+    dy, y = torch.ones(N, device="cuda"), torch.ones(N, device="cuda")
+    dpb, db = torch.zeros(N + 1, dtype=torch.bfloat16, device="cuda"), torch.zeros(1, device="cuda")
+    _ok(lib.efm_net_relu_bias_backward(_p(dy), _p(y), _p(dpb), _p(db), None, 1, N, 0, 0, N, None))
+    torch.cuda.synchronize()
+    assert abs(float(db) - N) <= 8 * 2.0 ** -24 * N
+    for at in (0, N // 2, N - 300):
+        assert (dpb[at:min(at + 300, N)] == 1).all()
+    assert float(dpb[N]) == 0
