@@ -254,16 +254,22 @@ def summarize_ab(ab, iters):
 
 
 def gemm_rate(net: InitNet, B, reps=50):
-    """Throughput of the first convolution's forward pass (the largest GEMM) at batch B,
-    timed with HIP events on the library's stream."""
+    """Throughput of the first convolution's forward pass (the largest GEMM; over the
+    stored im2col matrix where the net keeps one) at batch B, timed with HIP events on
+    the library's stream."""
     s = net.spec
     ci, co, Lin, lo = s.convs()[0]
     b = net._buffers(B)
     K, N = ci * s.ks, B * lo
-    yb = b["yb0"] if s.nblocks > 1 else b["X"]
-    call = lambda: _capi.check(net.L.efm_net_conv1d(_ptr(b["x"]), _ptr(net.wb["W0"]), _ptr(net.w["b0"]), _ptr(b["y0"]),
-                                                    _ptr(yb), ci, B, Lin, co, s.ks, s.stride, s.pad,
-                                                    int(s.nblocks == 1), _stream()), "efm_net_conv1d")
+    if "col0" in b:
+        yb = b["yb0"] if s.nblocks > 1 else b["yb_last"]
+        call = lambda: net._gemm(co, N, K, net.wb["W0"], K, 1, b["col0"], N, 1, b["y0"], N, bias=net.w["b0"],
+                                 Cb=yb, epi=1)
+    else:
+        yb = b["yb0"] if s.nblocks > 1 else b["X"]
+        call = lambda: _capi.check(net.L.efm_net_conv1d(
+            _ptr(b["x"]), _ptr(net.wb["W0"]), _ptr(net.w["b0"]), _ptr(b["y0"]), _ptr(yb), ci, B, Lin, co, s.ks,
+            s.stride, s.pad, int(s.nblocks == 1), _stream()), "efm_net_conv1d")
     call()
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     e0.record()

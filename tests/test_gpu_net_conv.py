@@ -197,3 +197,18 @@ def test_longest_row():
     for at in (0, N // 2, N - 300):
         assert (dpb[at:min(at + 300, N)] == 1).all()
     assert float(dpb[N]) == 0
+
+
+@pytest.mark.parametrize("spec", [
+    NetSpec(cin=9, length=64, channels=8, ks=9, stride=2, pad=4, nblocks=2, hidden=16),
+    NetSpec(cin=9, length=64, channels=8, ks=11, stride=2, pad=5, nblocks=2, hidden=16),
+    NetSpec(cin=9, length=64, channels=8, ks=11, stride=2, pad=5, nblocks=1, hidden=16),
+    NetSpec(cin=9, length=7, channels=8, ks=3, stride=1, pad=1, nblocks=2, hidden=16),
+])
+def test_gemm_rate_times_either_path(spec):
+    """The rate of the first convolution, implicit or over the stored matrix."""
+    from elastic_fm_vp_vs_rho_amd.initnet_data import gemm_rate
+    net = InitNet(spec, device="cuda", seed=4)
+    r = gemm_rate(net, 5, reps=3)
+    ci, co, _, lo = spec.convs()[0]
+    assert (r["M"], r["N"], r["K"]) == (co, 5 * lo, ci * spec.ks) and r["ms"] > 0 and r["tflops"] > 0
