@@ -243,3 +243,39 @@ def test_network_start_needs_fewer_lbfgs_iterations(gpu_lib):
     print(f"iterations to 1e-2 J0, plain {plain.tolist()} network {network.tolist()}")
     assert np.median(network) < np.median(plain), (plain, network)
     assert int(np.sum(network > plain)) <= 2, (plain, network)
+
+
+@pytest.mark.parametrize("small", [
+    dict(SMALL, ks=11, pad=5),                                    # more than 9 taps: every layer
+    dict(SMALL, length=40, ks=9, pad=4, nblocks=4),               # rows of 5 samples in the last layer
+    dict(SMALL, length=40, ks=9, pad=4, nblocks=5),               # ... of 5 and 3 in the last two
+    dict(SMALL, length=1100, ks=11, pad=5, nblocks=2),            # biases summed through chains
+])
+def test_stored_matrix_layers_against_oracle(gpu_lib, small):
+    """The layers that keep the im2col matrix, and the implicit ones before them: outputs, loss and
+    every gradient against the oracle, as in test_forward_backward_against_oracle."""
+    from elastic_fm_vp_vs_rho_amd.initnet import InitNet, NetSpec
+    spec, ospec = NetSpec(**small), R.Spec(**small)
+    rng = np.random.default_rng(12)
+    B = 6
+    p = R.init_params(ospec, seed=3)
+    for k in p:
+        if k[0] in "bc":
+            p[k] = (0.05 * rng.standard_normal(p[k].shape)).astype(np.float32)
+    net = InitNet(spec, params=p, device="cuda")
+    x = R.bf16(rng.standard_normal((spec.cin, B, spec.length)))
+    t = rng.standard_normal((spec.nout, B)).astype(np.float32)
+    net.set_input(_bf(x))
+    b = net._buffers(B)
+    assert f"col{spec.nblocks - 1}" in b
+    b["t"].copy_(torch.as_tensor(t, device="cuda"))
+    out = net.forward_buffers(B)
+    loss = net.backward_buffers(B)
+    torch.cuda.synchronize()
+    ro, cache = R.forward(ospec, p, x, emulate=True)
+    rl, rg = R.backward(ospec, p, cache, t.astype(np.float64), emulate=True)
+    assert _rel(out.cpu().numpy(), ro) < 2e-3
+    assert abs(float(loss) - rl) <= 2e-3 * rl
+    for k, g in rg.items():
+        e = _rel(net.g[k].cpu().numpy(), g)
+        assert e < 2e-3, (k, e)
