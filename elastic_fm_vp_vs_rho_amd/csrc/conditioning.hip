@@ -338,13 +338,6 @@ extern "C" int efm_condition_gradient(const EfmSmooth *p, int nx, int ny, int nz
     for (int j = -r; j <= r; ++j) sum += (phi[j + r] = std::exp(-0.5 / s2 * (double)j * (double)j));
     for (int j = 0; j <= r; ++j) taps.w[j] = phi[j + r] / sum;
     const Margins none{0, 0, 0, 0, 0, 0};
-    auto launch = [&](auto kernel, int dx, int dy, int dz, const float *src, float *dst, int mask, const Margins &m) {
-        const int cells = (nx + dx - 1) / dx, rows = (nz + dz - 1) / dz, planes = (ny + dy - 1) / dy;
-        // rows of 32 lanes where that leaves fewer of them idle than 64
-        const int bx = (cells + 31) / 32 % 2 ? 32 : 64, bz = 256 / bx;
-        hipLaunchKernelGGL(kernel, dim3((cells + bx - 1) / bx, std::min((rows + bz - 1) / bz, 65535),
-                                        std::min(planes, 65535)), dim3(bx, bz), 0, st, src, dst, nx, ny, nz, taps, mask, m);
-    };
     if (r == kR4 && nx >= r && ny >= r && nz >= r) {
         const long long ntx = (nx + kTX - 1) / kTX, ntz = (nz + kTZ - 1) / kTZ, nty = (ny + kTY - 1) / kTY;
         if (ntx * ntz * nty <= (long long)UINT32_MAX / kGaussThreads) {
