@@ -360,18 +360,19 @@ int set_tile(int kernel, Tile t);
 // Measured on the two sweeps, ns per thousand interior cell-steps by shots per
 // launch: 96^3 25.6 at 4 shots (190 MB), 25.8 at 5 (237 MB), 32.1 at 6 (281 MB), 35.0
 // at 32; 64^3 29.0 at 16 (248 MB), 42.0 at 24 (371 MB); 128^3 22.7 at 2 (223 MB),
-// 34.2 at 3.  32 shots of 96^3 went from 872 to 682 us per step.  The line lies where the
-// cache (268 MB) begins to miss more than a second round of launches costs: batches of
-// 240, 249, 258 and 263 MB took 98, 97, 102 and 123 us per step in one launch, 104, 106,
-// 108 and 114 in two.  Where even one shot exceeds the cache all shots stay in one launch
-// (fewer, longer launches).  A batch only just larger than that also stays whole: 26
-// shots of 73x64x37 (261 MB) take 100.5 us per step whole and 107.6 in two groups, with
-// records of 2/3 to all of the steps 88.6 and 95.1; 27 (271 MB) 112.3 and 111.6, 97.0 and
-// 98.3; 29 (291 MB) 132.4 and 118.6, 111.2 and 102.8.  The adjoint sweeps gain nothing from
+// 34.2 at 3.  32 shots of 96^3 went from 872 to 682 us per step.  The line lies at the
+// cache's own size, 256 MiB: over 24 grids of 50 thousand to 1.1 million cells, all and
+// part of the steps recorded, whole and in two groups (us per step): 64^3 106.5 and 115.2 at 263
+// MB, 130.2 and 121.5 at 279; 48^3 105.9 and 112.7 at 260, 119.2 and 121.1 at 280; 73x64x37 98.8
+// and 108.4 at 263, 106.3 and 111.7 at 272, 126.5 and 119.0 at 290; 57x169x47 98.6 and 105.7 at
+// 248, 134.9 and 115.7 at 271; 36x138x89 123.0 and 120.2 at 266.  Bytes do not tell all:
+// the sides cross between 255 and 280 MB by grid (33x150x60 already 131.3 and 117.7 at
+// 263), and a line anywhere from 265 to 277 MB loses 0.3 % to the better side on
+// average (12 % at worst from here, 17 % from 272 on), at 260 or 280 MB 0.7 %.  Where even one shot exceeds the cache all
+// shots stay in one launch (fewer, longer launches).  The adjoint sweeps gain nothing from
 // groups (96^3: 71 ns with 8 shots in a launch, 74-83 in groups of 2 or 1), so they take
 // the whole batch.
-constexpr long long kCacheBytes = 260LL * 1000 * 1000;
-constexpr long long kWholeBytes = 272LL * 1000 * 1000;
+constexpr long long kCacheBytes = 268LL * 1000 * 1000;
 
 // Bytes of one shot's nine fields and of its ψ slabs.
 inline long long field_bytes(const Geo &g) { return 36 * g.N; }
@@ -381,7 +382,7 @@ inline long long psi_bytes(const Geo &g) { return 24LL * ((long long)g.pxc + g.p
 // `shared` bytes of the medium in every step; groups are as equal as possible.
 inline int group_shots(const Geo &g, long long per_shot, long long shared) {
     const long long fit = (kCacheBytes - shared) / (per_shot > 0 ? per_shot : 1);
-    if (fit < 1 || fit >= g.S || g.S * per_shot + shared <= kWholeBytes) return g.S;
+    if (fit < 1 || fit >= g.S) return g.S;
     const int groups = (int)((g.S + fit - 1) / fit);
     return (g.S + groups - 1) / groups;
 }
