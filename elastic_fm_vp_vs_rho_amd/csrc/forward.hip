@@ -205,7 +205,7 @@ int launch_border(const Geo &g, const ShotPtrs &sh, const StatePtrs &s, float *b
 int run_forward(const Geo &g0, const EfmMedium &m, const ShotPtrs &sh, const EfmState *const *states,
                 bool in_place, float *gathers, float *borders, int W, int it0, int nsteps,
                 hipStream_t st) {
-    const int group = group_shots(g0, field_bytes(g0) + psi_bytes(g0), 12 * g0.N);
+    const int group = forward_group(g0, nsteps);
     Geo gd = g0;
     gd.dense |= gd.nx < kDenseRow && gd.N * gd.S >= kDenseCells;
     return for_shot_groups(gd, group, [&](const Geo &g) {

@@ -75,3 +75,41 @@ def test_a_batch_stays_whole_as_long_as_it_fits_the_cache(program):
 
 def test_shots_beyond_the_cache_stay_together(program):
     assert _groups(program, (256, 256, 128, 4, 20, 20, 20), (200, 200, 200, 3, 0, 0, 0)) == [[4], [3]]
+
+
+STEPS_SOURCE = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "common.hpp"
+using namespace efm;
+// nx ny nz S Lx Ly Lz nsteps: the shots of each group of a forward call of nsteps steps
+int main(int argc, char **argv) {
+    for (int i = 1; i + 7 < argc; i += 8) {
+        int v[8];
+        for (int k = 0; k < 8; ++k) v[k] = atoi(argv[i + k]);
+        EfmDims d{};
+        d.nx = v[0]; d.ny = v[1]; d.nz = v[2]; d.nshot = v[3];
+        d.wx_hi = v[4]; d.wy_hi = v[5]; d.wz_hi = v[6]; d.ntmax = 1;
+        const Geo g = make_geo(d);
+        for_shot_groups(g, forward_group(g, v[7]), [&](const Geo &gg) { std::printf("%d ", gg.S); return 0; });
+        std::printf("\n");
+    }
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("nsteps", [0, 1, 2, 3, 4, 24, 1000])
+def test_calls_of_a_step_or_two_keep_their_batch_whole(tmp_path, nsteps):
+    """A group gains from its second step on only: loops stepped one call a step (or captured
+    in chunks of one) must not pay a round of launches for each group."""
+    if not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")):
+        pytest.skip("no hipcc")
+    src, exe = tmp_path / "steps.hip", tmp_path / "steps"
+    src.write_text(STEPS_SOURCE)
+    subprocess.run([build._hipcc(), "--offload-host-only", "-std=c++17", "-I", build.INCLUDE, "-I", build.CSRC, str(src),
+                    "-o", str(exe)], check=True, capture_output=True, timeout=120)
+    cases = [(96, 96, 96, 32, 20, 20, 20), (64, 64, 64, 24, 20, 20, 20), (57, 169, 47, 20, 12, 12, 12)]
+    for c, groups in zip(cases, _groups(str(exe), *[(*c, nsteps) for c in cases])):
+        assert sum(groups) == c[3]
+        assert (len(groups) == 1) == (nsteps < 3), (c, groups)
