@@ -33,9 +33,14 @@ __global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_stress(Geo g, Med m, ShotPtrs sh
 // ---------------------------------------------------------------------------
 // velocity sweep
 // ---------------------------------------------------------------------------
+// 8 waves to a SIMD: at 82 to 86 SGPRs, which the compiler takes by itself, 7 fit (16 more
+// belong to the trap handler), at 78 or fewer 8, and none is spilled; a launch of 3585 to 4096
+// blocks of 128 then takes one round of them, not two.  Forward step: 52x124x78 17.8 -> 16.8 us,
+// 64x132x64 18.1 -> 17.0, 128x27x55 x 6 28.0 -> 27.1, 128^3 50.6 -> 50.0, in row tiles (64, 4)
+// 64x132x64 18.9 -> 17.7.  The XCD-aware row tiles gain nothing and would spill.
 template <int BX, int BZ, int NYC, int MAP>
-__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) void k_velocity(Geo g, Med m, ShotPtrs sh, StatePtrs in,
-                                                         StatePtrs out, int it, float *gathers) {
+__global__ EFM_KERNEL_ATTRS(BX, BZ, MAP) __attribute__((amdgpu_waves_per_eu(NYC == 1 && MAP != 8 ? 8 : 1, 8))) void
+k_velocity(Geo g, Med m, ShotPtrs sh, StatePtrs in, StatePtrs out, int it, float *gathers) {
     if (g.itp) it += *g.itp;
     int x, z, s, yb;
     if (!tile_coords<BX, BZ, NYC, MAP>(g, x, z, s, yb)) return;
