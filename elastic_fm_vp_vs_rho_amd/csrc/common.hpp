@@ -226,14 +226,6 @@ struct Tile {
 // XCDs the blocks of an XCD-aware mapping are dealt over.
 __host__ __device__ constexpr int map_xcds(int map) { return map == 16 ? 8 : map; }
 
-// A forward step over many cells in short rows loses more to the guard lanes (4 of nx) than
-// to lines shared by two waves, and walks the interior cells only (Geo::dense); aligned and
-// dense walks, us per step: 105.1 and 103.1 for 10 shots of 36x138x89, 49.6 and 48.4 for 8 of
-// 40x80x80, 94.9 and 94.0 for 9 of 52x124x78; even from 66 cells a row on.  Steps that take
-// little more than their launches (one shot of 41x37x33, 48^3) keep the aligned walk, whose
-// index arithmetic is shorter: 10.8 and 11.15, 11.0 and 11.3.
-constexpr int kDenseRow = 64;
-constexpr long long kDenseCells = 1 << 20;
 // The cells a compact sweep walks in a plane: from the line of the first interior cell to
 // the last interior cell, or the interior ones.
 __host__ __device__ inline int plane_span(const Geo &g) {
@@ -250,6 +242,25 @@ inline long long sweep_tiles(const Geo &g, int bx, int bz, int ny, int map) {
     }
     const long long nbx = (g.nx + bx - 1) / bx, nbz = (g.nz + bz - 1) / bz;
     return nbx * nbz * nyc * g.S;
+}
+
+// Whether a forward step walks the interior cells only (Geo::dense) and not the cells of
+// whole lines.  Its shorter index arithmetic gives the aligned walk the launches whose blocks
+// the chip holds at once (the stress sweep: 14 of 128 lanes a CU); a few blocks more take a
+// second round, and without the four guard cells of each row they often fit.  Aligned and dense
+// walks, us per step, with the aligned walk's blocks: 64x122x64 (3658) 15.8 and 15.7,
+// 64x126x64 (3782) 16.7 and 16.0, 76x90x76 (3698) 16.5 and 16.0, 68x40x70 x 3 (3888) 18.5 and 17.5,
+// 52x124x78 (3720) 16.6 and 15.7; below, 130x60x64 (3472) 15.5 and 16.4, 61x47x53 x 3 (3096) 15.8
+// and 16.3, 45x100x100 (3264) 15.0 and 15.7, 48^3 (748) 9.7 and 10.0.  Beyond one round rows under
+// 64 cells keep the dense walk, since the guard cells are a larger share: 1.4 % shorter over
+// 40 batches (28x100x100 x 3 22.6 and 21.4, 36x138x89 x 10 109.4 and 107.8; runs differ by 0.3 %),
+// 3.3 % longer at worst (60x200x200 x 4, 257 and 266).  From 64 cells on the walks are within 1-2 %
+// of each other until memory binds them, where whole lines count (128^3 and up).
+constexpr int kDenseRow = 64;
+constexpr long long kRoundLanes = 14LL * 128 * 256;
+inline bool dense_walk(Geo g) {
+    const auto lanes = [&](int dense) { g.dense = dense; return 128 * sweep_tiles(g, 128, 1, 1, 16); };
+    return lanes(0) > kRoundLanes && (g.nx < kDenseRow || lanes(1) <= kRoundLanes);
 }
 
 // Blocks of an XCD-aware sweep: each shot's tiles are dealt over the k XCDs in

@@ -212,7 +212,7 @@ int run_forward(const Geo &g0, const EfmMedium &m, const ShotPtrs &sh, const Efm
                 hipStream_t st) {
     const int group = forward_group(g0, nsteps);
     Geo gd = g0;
-    gd.dense |= gd.nx < kDenseRow && gd.N * gd.S >= kDenseCells;
+    gd.dense |= dense_walk(g0);
     return for_shot_groups(gd, group, [&](const Geo &g) {
         bool unsaved = false;       // the borders of the step before
         for (int k = 0; k < nsteps; ++k) {
