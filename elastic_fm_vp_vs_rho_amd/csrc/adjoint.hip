@@ -675,12 +675,7 @@ int launch_adj_velocity(const Geo &g, const AdjArgs &A, int n, hipStream_t st) {
 #define X_PLAIN(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity, g, A, n)
 #define X_IMAGE(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity_image, g, A, n)
 #define X_STREAM(a, b, c, o) EFM_LAUNCH_IF(a, b, c, o, k_adj_velocity_image_stream, g, A, n)
-    // Streaming reads of the forward state pay where they keep the adjoint's own
-    // working set (15 volumes a shot, 8 of the medium, two sets of ψ slabs) in the
-    // 256 MB Infinity Cache: adjoint step at 128^3 (240 MB) 95 us with the hint, 106
-    // without; above it the hint only drops lines that the neighbouring cells still
-    // read: 256x256x128 463 with, 447 without, 200x200x100 204 and 200.
-    const bool stream = 60 * g.S * g.N + 32 * g.N + 2 * g.S * psi_bytes(g) <= 250LL * 1000 * 1000;
+    const bool stream = stream_forward_state(g);
     if (n % 2 && n != A.n0) {          // image_r2 images nothing in this step
         EFM_TILE_LIST(X_PLAIN)
     } else if (stream) {

@@ -389,6 +389,19 @@ constexpr long long kCacheBytes = 268LL * 1000 * 1000;
 inline long long field_bytes(const Geo &g) { return 36 * g.N; }
 inline long long psi_bytes(const Geo &g) { return 24LL * ((long long)g.pxc + g.pyc + g.pzc); }
 
+// Whether the imaging adjoint sweep reads the forward state with the streaming hint.  It pays
+// as long as the adjoint's own working set (9 fields, 8 sums and two sets of ψ slabs a shot, 8
+// volumes of the medium) stays largely in the Infinity Cache; beyond, the hint only drops lines
+// that the neighbouring cells still read.  Adjoint step without and with it, us, by that set:
+// 64^3 x 4 (119 MB) 56.8 and 56.2, 96^3 x 2 (193) 85.5 and 83.4, 128^3 (249) 102.7 and 93.7, 64^3 x 9
+// (257) 114.7 and 109.2, 160x150x100 (281) 118.4 and 112.2, 48^3 x 24 (290) 124.6 and 120.7,
+// 140x136x136 (304) 131.1 and 128.6, 48^3 x 28 (338) 149.3 and 148.0, 144^3 (348) 142.5 and 144.7,
+// 200x200x100 (458) 181.3 and 184.1.
+constexpr long long kStreamBytes = 320LL * 1000 * 1000;
+inline bool stream_forward_state(const Geo &g) {
+    return 68 * g.S * g.N + 32 * g.N + 2 * g.S * psi_bytes(g) <= kStreamBytes;
+}
+
 // Shots per group for a loop that touches `per_shot` bytes of each shot and
 // `shared` bytes of the medium in every step: as many groups as the cache asks for, equal
 // ones but for the last, which takes what is left.
