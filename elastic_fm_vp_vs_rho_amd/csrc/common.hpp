@@ -417,7 +417,11 @@ inline int group_shots(const Geo &g, long long per_shot, long long shared) {
 // pays the further launches: over 52 batches of 1 to 2.5 times the line, with full and with
 // uneven records, groups took 6.3 % longer than the whole batch at one step a call (10 % at
 // worst, 96^3 x 32 831.7 against 773.7 us), 1.4 % less at two (from 8 % longer to 10 %
-// less), 4.6 % less at three, 6.4 % at four, 12 % at 24.
+// less), 4.6 % less at three, 6.4 % at four, 12 % at 24.  Kept states take a second state's
+// velocities and slabs along, which these bytes leave out; whole and in groups, us per step:
+// 64^3 x 20 147.0 and 143.0, 96^3 x 8 205.0 and 189.5, 128^3 x 3 163.0 and 163.2, 36x138x89 x 16
+// 222.1 and 190.5.  Counting both states shortens some (57x169x47 x 12 144.5 -> 134.8) and lengthens
+// others (64^3 x 12 84.5 -> 90.4).
 constexpr int kGroupSteps = 3;
 inline int forward_group(const Geo &g, int nsteps) {
     return nsteps < kGroupSteps ? g.S : group_shots(g, field_bytes(g) + psi_bytes(g), 12 * g.N);

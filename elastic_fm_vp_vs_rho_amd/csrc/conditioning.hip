@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void k_gauss_pass(const float *__restrict__ in
 // caches, and written once; three passes moved 8 bytes a cell each and paid three launches
 // of about 4 us.  200x200x100 under the driver's margins: 37.4 us in
 // three passes (13.9 + 10.5 + 13), 24 here, bound by the double sums (about 17 operations
-// for each of 2.6 sums a cell; 16 rows a tile halve the surplus but leave fewer waves: 28).
+// for each of 3.1 sums a cell; 16 rows a tile halve the surplus but leave fewer waves: 28).
 constexpr int kTX = 64, kTY = 8, kTZ = 8, kR4 = 4, kGaussThreads = 576;
 __global__ __launch_bounds__(kGaussThreads) void k_gauss4(const float *__restrict__ in, float *__restrict__ out,
                                                           int nx, int ny, int nz, int ntx, int ntz, GaussTaps taps,
